@@ -1,6 +1,7 @@
 // The GLST engine behind the C ABI of include/glst_hip.h: one handle = one
 // system on one GPU with one HIP stream.  Host setup follows
 // src/glst_force.cu:178-327; the force step follows :431-1614.
+#include "harmonic_plan.hpp"
 #include "runtime.hpp"
 
 #include <hip/hip_runtime.h>
@@ -112,6 +113,12 @@ struct glst_engine {
   uint32_t ntask = 0;
   // Chebyshev matrices of the mixed structure factors (plan_chebyshev)
   DeviceBuffer cheb;
+  // far field through spherical harmonics (harmonic.hpp): tables, the cells'
+  // coefficients, which cells hold atoms outside their unit ball
+  HarmDevice harm;
+  dev::HarmPlanDev harm_plan;
+  DeviceBuffer harm_coef, harm_mom, harm_out;
+  int field_layout = -1;  // what S holds: 0 node runs, 1 node-major rows
   // fields
   DeviceBuffer S, R, partial;
   DeviceBuffer rmt_work;  // FP64 tables of the global shell-sum path
@@ -140,8 +147,8 @@ struct glst_engine {
                                   &partial,   &atoms32, &t_node0,   &t_nr,
                                   &t_koff,    &t_dir64, &t_dir32,   &kap64,
                                   &kap32,     &t_split, &near4, &atom_grp, &ag_start,
-                                  &cheb};
-    size_t s = 0;
+                                  &cheb,      &harm_coef, &harm_mom, &harm_out};
+    size_t s = harm.device_bytes();
     for (auto b : bufs) s += b->bytes();
     return s;
   }
@@ -193,16 +200,45 @@ struct glst_engine {
       ev_rmt.push_back(nullptr);
       GLST_HIP(hipEventCreateWithFlags(&ev_rmt.back(), hipEventDisableTiming));
     }
-    allocate();
+    plan_far_field();
+    try {
+      allocate();
+    } catch (const AllocError &) {
+      // no room for the expansion's work fields: the direct sums need less
+      if (!harm.ok()) throw;
+      harm.release();
+      for (DeviceBuffer *b : {&harm_coef, &harm_mom, &harm_out, &S, &R})
+        b->release();
+      allocate();
+    }
     upload_nodes();
     dev::fill_f64(fx.as<double>(), 0.0, natom, stream);
     dev::fill_f64(fy.as<double>(), 0.0, natom, stream);
     dev::fill_f64(fz.as<double>(), 0.0, natom, stream);
     dev::fill_f64(en.as<double>(), 0.0, natom, stream);
-    // the mixed structure-factor kernel never writes the padded node columns
-    dev::fill_f64(S.as<double>(), 0.0, S.bytes() / sizeof(double), stream);
+    set_field_layout();
     check_launch("init");
     GLST_HIP(hipStreamSynchronize(stream));
+  }
+
+  // The expansion of the far field, where it is worth its passes (harm_worth)
+  // and the nodes and the device can hold it.
+  size_t harm_coef_len = 0, harm_mom_len = 0;
+  void plan_far_field() {
+    if (!has_lr || Kp == 0 || !harm_worth(natom, K, mixed())) return;
+    const HarmTables t = plan_harmonic(nodes, grid.h, spherical_rule, mixed());
+    if (!t.ok) return;
+    harm_plan = harm_fit(t, mixed(), lds_limit, natom, grid.ncell);
+    if (harm_plan.nrad == 0) return;
+    try {
+      harm.upload(t, mixed());
+    } catch (const AllocError &) {
+      harm.release();
+      return;
+    }
+    harm_plan.unit = harm.unit;
+    harm_coef_len = glst::harm_coef_len(t, grid.ncell);
+    harm_mom_len = glst::harm_mom_len(t, grid.ncell);
   }
 
   void allocate() {
@@ -230,8 +266,16 @@ struct glst_engine {
     if (Kp > 0) {
       if (has_lr) {
         const size_t field = static_cast<size_t>(grid.ncell) * Kp;
-        S.resize(field * (mixed() ? sizeof(float2) : sizeof(double2)));
-        R.resize(field * (mixed() ? sizeof(float2) : sizeof(double2)));
+        const size_t rows = static_cast<size_t>(dev::harm_row(grid.ncell)) * Kp;
+        const size_t slots = harm.ok() ? rows : field;
+        S.resize(slots * (mixed() ? sizeof(float2) : sizeof(double2)));
+        R.resize(slots * (mixed() ? sizeof(float2) : sizeof(double2)));
+        if (harm.ok()) {
+          const size_t real = mixed() ? sizeof(float) : sizeof(double);
+          harm_coef.resize(harm_coef_len * real);
+          harm_mom.resize(harm_mom_len * real);
+          harm_out.resize(static_cast<size_t>(grid.ncell) * 4);
+        }
         const uint32_t ntile = (natom + 255) / 256;
         // enough workgroups to fill the chip several times over
         set_splits(ntile > 0 ? (lr_blocks + ntile - 1) / ntile : 1);
@@ -337,10 +381,47 @@ struct glst_engine {
     sf_done = rmt_done = false;
   }
 
+  // Far field through spherical harmonics: for handles that planned it,
+  // unless the options ask for the direct sums or for the global tables.
+  bool harmonic() const {
+    return harm.ok() && sf_cheb && lr_atom_groups && rmt_shape != 2;
+  }
+  // Clears S when its layout changes: the kernels never write the slots of
+  // the padded nodes.
+  void set_field_layout() {
+    const int want = harmonic() ? 1 : 0;
+    if (field_layout == want) return;
+    dev::fill_f64(S.as<double>(), 0.0, S.bytes() / sizeof(double), stream);
+    field_layout = want;
+    sf_done = rmt_done = false;
+  }
+
   void calc_sf() {
     if (!has_lr || Kp == 0) return;  // src/glst_force.cu:667-670
     if (!assigned) throw StateError("calc_sf called before assign_atoms");
+    set_field_layout();
     Scope sc(timer, "sf", stream);
+    if (harmonic()) {
+      auto run = [&](auto t) {
+        using T = decltype(t);
+        dev::harm_moments<T>(harm_plan, harm.dev<T>(), lr_atoms(),
+                             cell_start.as<uint32_t>(), grid,
+                             harm_mom.as<T>(), harm_coef.as<T>(), harm_out.as<uint32_t>(),
+                             stream);
+        dev::harm_sf<T>(harm_plan, harm.dev<T>(), lr_atoms(),
+                        cell_start.as<uint32_t>(), k64.as<double4>(), grid,
+                        harm_coef.as<T>(), harm_out.as<uint32_t>(), S.as<T>(),
+                        stream);
+      };
+      if (mixed())
+        run(0.0f);
+      else
+        run(0.0);
+      check_launch("sf");
+      sf_done = true;
+      rmt_done = false;
+      return;
+    }
     dev::sf(mixed(), lr_atoms(), cell_start.as<uint32_t>(),
             cell_sorted.as<uint32_t>(), k64.as<double4>(), task_args(),
             sf_groups, Kp, grid, S.as<void>(), stream, cheb_table());
@@ -351,28 +432,31 @@ struct glst_engine {
 
   void sum_rmt_sf() {
     if (!has_lr || Kp == 0) return;
-    if (!sf_done) throw StateError("sum_rmt_sf called before calc_sf");
+    if (!sf_done || field_layout != (harmonic() ? 1 : 0))
+      throw StateError("sum_rmt_sf called before calc_sf");
     Scope sc(timer, "rmt", stream);
+    const bool nm = harmonic();
     if (rmt_mfma_path()) {
       dev::rmt_mfma(S.as<void>(), k64.as<double4>(), group.as<uint32_t>(),
                     r_in.as<uint32_t>(), r_out.as<uint32_t>(), Kp, grid,
-                    lds_limit, R.as<void>(), stream);
+                    lds_limit, R.as<void>(), stream, 0, 0xffffffffu, nm);
     } else if (rmt_wave_path()) {
       dev::rmt_wave(S.as<void>(), k64.as<double4>(), group.as<uint32_t>(),
                     r_in.as<uint32_t>(), r_out.as<uint32_t>(), Kp, grid,
-                    R.as<void>(), stream);
+                    R.as<void>(), stream, 0, 0xffffffffu, nm);
     } else if (rmt_shape == 2 ||
         !dev::rmt_lds(mixed(), rmt_shape == 1 ? 1 : dev::kRmtMaxNodes,
                       S.as<void>(),
                       k64.as<double4>(), group.as<uint32_t>(),
                       r_in.as<uint32_t>(), r_out.as<uint32_t>(), Kp, grid,
-                      lds_limit, R.as<void>(), stream)) {
+                      lds_limit, R.as<void>(), stream, 0, 0xffffffffu,
+                      nm)) {
       // tables too large for LDS: FP64 work field, allocated on first use
       rmt_work.resize(static_cast<size_t>(grid.ncell) * Kp * sizeof(double2));
       dev::rmt_global(mixed(), S.as<void>(), rmt_work.as<double2>(),
                       k64.as<double4>(), group.as<uint32_t>(),
                       r_in.as<uint32_t>(), r_out.as<uint32_t>(), Kp, grid,
-                      R.as<void>(), stream);
+                      R.as<void>(), stream, nm);
     }
     check_launch("rmt");
     rmt_done = true;
@@ -380,7 +464,8 @@ struct glst_engine {
 
   void calc_lr_ef() {
     if (!has_lr || Kp == 0 || natom == 0) return;
-    if (!rmt_done) throw StateError("calc_lr_ef called before sum_rmt_sf");
+    if (!rmt_done || field_layout != (harmonic() ? 1 : 0))
+      throw StateError("calc_lr_ef called before sum_rmt_sf");
     lr_partials();
     reduce(false);
   }
@@ -390,7 +475,8 @@ struct glst_engine {
   void reduce(bool with_near) {
     Scope sc(timer, "lr_reduce", stream);
     const bool lr = has_lr && Kp > 0;
-    dev::lr_reduce(partial.as<double4>(), lr ? nsplit : 0, natom,
+    dev::lr_reduce(partial.as<double4>(), lr ? (harmonic() ? 1u : nsplit) : 0,
+                   natom,
                    with_near ? near4.as<double4>() : nullptr, fx.as<double>(),
                    fy.as<double>(), fz.as<double>(), en.as<double>(), stream);
     check_launch("lr_reduce");
@@ -405,6 +491,24 @@ struct glst_engine {
 
   void lr_partials() {
     Scope sc(timer, "lr", stream);
+    if (harmonic()) {
+      auto run = [&](auto t) {
+        using T = decltype(t);
+        dev::harm_lr<T>(harm_plan, harm.dev<T>(), grid, R.as<T>(),
+                        harm_coef.as<T>(), harm_mom.as<T>(), stream);
+        dev::harm_eval<T>(harm_plan, harm.dev<T>(), lr_atoms(),
+                          cell_start.as<uint32_t>(), k64.as<double4>(), K,
+                          grid, harm_mom.as<T>(), R.as<T>(),
+                          harm_out.as<uint32_t>(), partial.as<double4>(),
+                          stream);
+      };
+      if (mixed())
+        run(0.0f);
+      else
+        run(0.0);
+      check_launch("lr");
+      return;
+    }
     const dev::LrTaskArgs ta = task_args();
     dev::lr(mixed(), lr_atoms(), cell_sorted.as<uint32_t>(), ta, lr_groups,
             R.as<void>(), Kp, natom, nsplit, partial.as<double4>(), stream,
@@ -437,7 +541,8 @@ struct glst_engine {
   uint32_t pipe_tmax = 0;
   std::vector<uint32_t> tile_end, rmt_need;
   bool pipelined() const {
-    return pipeline && mixed() && has_lr && Kp > 0 && !sf_groups.empty() &&
+    return pipeline && !harmonic() && mixed() && has_lr && Kp > 0 &&
+           !sf_groups.empty() &&
            ev_sf.size() == sf_groups.size() &&
            lr_groups.size() == sf_groups.size() && !rmt_global_path();
   }
@@ -588,7 +693,8 @@ struct glst_engine {
         rmt_shape == 3 ||
         (rmt_shape == 4 && grid.nx * grid.ny * 2 >= dev::kRmtMfmaMaxXY *
                                                         dev::kRmtMfmaMaxXY);
-    return want && mixed() && dev::rmt_mfma_nodes(grid, lds_limit) > 0;
+    return want && mixed() &&
+           dev::rmt_mfma_nodes(grid, lds_limit, harmonic()) > 0;
   }
   // shell sums as window sums of small grids (CT = float, every dimension
   // up to 8)
@@ -622,7 +728,9 @@ struct glst_engine {
     const double *in[4] = {rx, ry, rz, qc};
     if (!graph_exec || !std::equal(in, in + 4, graph_in)) {
       drop_graph();
-      // nothing may allocate inside the capture
+      // nothing may allocate inside the capture, and a change of layout
+      // belongs before it
+      if (has_lr && Kp > 0) set_field_layout();
       if (has_lr && Kp > 0 && rmt_global_path())
         rmt_work.resize(static_cast<size_t>(grid.ncell) * Kp * sizeof(double2));
       const bool timing = timer.enabled;
@@ -774,12 +882,15 @@ struct glst_engine {
                             hipMemcpyDeviceToHost, stream));
   }
 
-  // Device field (R: c*Kp + k; S: node runs, sf_slot) to host arrays of
+  // Device field (node-major rows; else R: c*Kp + k, S: node runs, sf_slot)
+  // to host arrays of
   // ncell x K in reference node order.  FP32 fields hold `fstride` floats
   // per element, the first two being (re, im).
   void field_to_host(const DeviceBuffer &buf, bool single, uint32_t fstride,
                      bool tiled, double *re, double *im) {
-    const size_t n = static_cast<size_t>(grid.ncell) * Kp;
+    const uint32_t ncp = dev::harm_row(grid.ncell);
+    const bool nm = harmonic();
+    const size_t n = static_cast<size_t>(nm ? ncp : grid.ncell) * Kp;
     std::vector<double> tmp(2 * n);
     if (single) {
       std::vector<float> f(fstride * n);
@@ -798,11 +909,20 @@ struct glst_engine {
     for (uint32_t c = 0; c < grid.ncell; ++c)
       for (uint32_t k = 0; k < K; ++k) {
         const uint32_t node = dev_of_ref[k];
+        const size_t d = static_cast<size_t>(c) * K + k;
+        if (nm) {
+          const size_t a = single ? dev::harm_slot<float>(node, c, 0, ncp)
+                                  : dev::harm_slot<double>(node, c, 0, ncp);
+          const size_t b = single ? dev::harm_slot<float>(node, c, 1, ncp)
+                                  : dev::harm_slot<double>(node, c, 1, ncp);
+          if (re) re[d] = tmp[a];
+          if (im) im[d] = tmp[b];
+          continue;
+        }
         const size_t s =
             !tiled ? static_cast<size_t>(c) * Kp + node
             : single ? dev::sf_slot<true>(node, c, grid.ncell)
                      : dev::sf_slot<false>(node, c, grid.ncell);
-        const size_t d = static_cast<size_t>(c) * K + k;
         if (re) re[d] = tmp[2 * s];
         if (im) im[d] = tmp[2 * s + 1];
       }
@@ -1078,12 +1198,13 @@ glst_status_t glst_get_sf(glst_handle_t h, double *re, double *im) {
   NEED_HANDLE(h);
   return guarded(h, [&] {
     if (!h->has_lr || h->K == 0) return;
-    if (!h->sf_done) throw StateError("glst_get_sf: no structure factors");
+    if (!h->sf_done || h->field_layout != (h->harmonic() ? 1 : 0))
+      throw StateError("glst_get_sf: no structure factors");
     const size_t n = static_cast<size_t>(h->grid.ncell) * h->K;
     std::vector<double> r(n), i(n);
     h->field_to_host(h->S, h->mixed(), 2, true, r.data(), i.data());
     const auto &g = h->grid;
-    if (h->mixed()) {
+    if (h->mixed() || h->harmonic()) {
       // the field holds cell-local sums; apply exp(-i k.c)
       for (uint32_t c = 0; c < g.ncell; ++c) {
         const uint32_t x = c / (g.ny * g.nz), y = (c / g.nz) % g.ny,
@@ -1122,13 +1243,16 @@ glst_status_t glst_get_rmt(glst_handle_t h, double *re, double *im) {
   NEED_HANDLE(h);
   return guarded(h, [&] {
     if (!h->has_lr || h->K == 0) return;
-    if (!h->rmt_done) throw StateError("glst_get_rmt: no remote sums");
+    if (!h->rmt_done || h->field_layout != (h->harmonic() ? 1 : 0))
+      throw StateError("glst_get_rmt: no remote sums");
     const size_t n = static_cast<size_t>(h->grid.ncell) * h->K;
     std::vector<double> r(n), i(n);
     h->field_to_host(h->R, h->mixed(), 2, false, r.data(), i.data());
-    if (h->mixed()) {
-      // the stored (kappa |V|, arg V / 2 pi) back to V = exp(+i k.c) R_c(k),
-      // then undo the exp(+i k.c) factor in FP64
+    const bool polar = !h->harmonic();
+    if (h->mixed() || !polar) {
+      // the stored (kappa |V|, arg V / 2 pi) back to V = exp(+i k.c) R_c(k)
+      // (node-major fields hold V itself), then undo the exp(+i k.c) factor
+      // in FP64
       const auto &g = h->grid;
       const double two_pi = 2.0 * M_PI;
       std::vector<double> inv_kappa(h->K);
@@ -1147,7 +1271,8 @@ glst_status_t glst_get_rmt(glst_handle_t h, double *re, double *im) {
           const double cs = std::cos(th), sn = std::sin(th);
           const size_t o = static_cast<size_t>(c) * h->K + k;
           const double mag = r[o] * inv_kappa[k], arg = two_pi * i[o];
-          const double a = mag * std::cos(arg), b = mag * std::sin(arg);
+          const double a = polar ? mag * std::cos(arg) : r[o];
+          const double b = polar ? mag * std::sin(arg) : i[o];
           r[o] = a * cs + b * sn;
           i[o] = b * cs - a * sn;
         }

@@ -1,0 +1,1454 @@
+// Kernels of the far field through spherical harmonics (harmonic.hpp), for
+// gfx950.  Four kernels: moments of a cell's atoms -> coefficients of every
+// radial node (harm_moments), coefficients -> S at the nodes (harm_sf),
+// remote sums -> coefficients (harm_lr), coefficients -> fields at the atoms
+// (harm_eval).  The dense products of the first three are
+// v_mfma_f32_16x16x4f32 or v_mfma_f64_16x16x4f64.
+//
+// Times below are of the 288,000-charge box at tol 1e-4 (3,375 cells of 85
+// atoms, 27,453 nodes, 53 radial nodes, N = 26 mixed and 37 FP64), mixed and
+// FP64.  The direct sums that these passes replace took 724 and 9,160 us (S)
+// and 1,873 and 10,153 us (back-projection); S and R are 0.74 and 1.48 GB
+// each, 0.15 and 0.29 ms at the 5.1 TB/s of a large copy.
+//
+// Operand layouts for lane l (c = l % 16, g = l / 16): A[c][g], B[g][c];
+// accumulator register r holds D[4g + r][c] in FP32 and D[g + 4r][c] in FP64
+// (both checked on the GPU).  Where an accumulator is the B operand of a
+// following product, register r is step r of it: its rows are numbered so
+// that step r covers the indices 4r .. 4r + 3 (harm_perm).
+#include "harmonic.hpp"
+
+#include <algorithm>
+
+namespace glst {
+namespace dev {
+namespace {
+
+typedef float harm_f4 __attribute__((ext_vector_type(4)));
+typedef double harm_d4 __attribute__((ext_vector_type(4)));
+
+template <typename T>
+struct Harm;
+template <>
+struct Harm<float> {
+  using v4 = harm_f4;
+  static __device__ __forceinline__ v4 mfma(float a, float b, v4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  }
+  // row of the accumulator in register r of lane group g
+  static __device__ __forceinline__ uint32_t row(uint32_t g, uint32_t r) {
+    return 4 * g + r;
+  }
+  // the index that row R of a chained product stands for
+  static __device__ __forceinline__ uint32_t perm(uint32_t R) {
+    return 4 * (R & 3u) + (R >> 2);
+  }
+};
+template <>
+struct Harm<double> {
+  using v4 = harm_d4;
+  static __device__ __forceinline__ v4 mfma(double a, double b, v4 c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ uint32_t row(uint32_t g, uint32_t r) {
+    return g + 4 * r;
+  }
+  static __device__ __forceinline__ uint32_t perm(uint32_t R) { return R; }
+};
+
+__device__ __forceinline__ float harm_fma(float a, float b, float c) {
+  return fmaf(a, b, c);
+}
+__device__ __forceinline__ double harm_fma(double a, double b, double c) {
+  return fma(a, b, c);
+}
+
+// An atom around its cell's centre, in units of 1 / scale: position, square,
+// argument of the radial polynomials x = 2 t^2 - 1, charge, and whether it
+// lies outside the ball.  The squares are formed in FP64 (an FP32 one would
+// move the atom, for all directions alike), by the same operations in every
+// kernel, so that all agree on which atoms lie outside.
+template <typename T>
+struct HarmAtom {
+  T x, y, z, s, t, q;
+  bool out;
+};
+// An atom's offset from its cell's centre and its charge in FP64.
+struct HarmOffset {
+  double x, y, z, q;
+};
+template <typename T>
+struct HarmRecord;
+template <>
+struct HarmRecord<float> {
+  using type = float4;
+};
+template <>
+struct HarmRecord<double> {
+  using type = double4;
+};
+
+struct HarmCentre {
+  double x, y, z;
+};
+__device__ __forceinline__ HarmOffset harm_offset(const float4 *atoms,
+                                                  uint32_t i, HarmCentre) {
+  const float4 a = atoms[i];
+  return {a.x, a.y, a.z, a.w};
+}
+__device__ __forceinline__ HarmOffset harm_offset(const double4 *atoms,
+                                                  uint32_t i, HarmCentre c) {
+  const double4 a = atoms[i];
+  return {a.x - c.x, a.y - c.y, a.z - c.z, a.w};
+}
+template <typename T>
+__device__ __forceinline__ HarmAtom<T> harm_atom(
+    const HarmDev<T> &H, const typename HarmRecord<T>::type *atoms, uint32_t i,
+    HarmCentre c) {
+#pragma clang fp contract(off)
+  const HarmOffset d = harm_offset(atoms, i, c);
+  const double x = d.x * H.scale, y = d.y * H.scale, z = d.z * H.scale;
+  const double s = x * x + y * y + z * z;
+  HarmAtom<T> o = {};
+  o.q = static_cast<T>(d.q);
+  o.out = s > H.smax;
+  if (!o.out) {
+    o.x = static_cast<T>(x);
+    o.y = static_cast<T>(y);
+    o.z = static_cast<T>(z);
+    o.s = static_cast<T>(s);
+    o.t = static_cast<T>(s * H.xk - 1.0);
+  }
+  return o;
+}
+__device__ __forceinline__ HarmCentre harm_centre(uint32_t cell, uint32_t ny,
+                                                  uint32_t nz, double h) {
+  HarmCentre c;
+  c.x = (static_cast<double>(cell / (ny * nz)) + 0.5) * h;
+  c.y = (static_cast<double>((cell / nz) % ny) + 0.5) * h;
+  c.z = (static_cast<double>(cell % nz) + 0.5) * h;
+  return c;
+}
+
+// Workgroup barrier for data in LDS: waits for the LDS operations only, so that
+// loads issued ahead and stores stay in flight (__syncthreads drains them).
+__device__ __forceinline__ void harm_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+// p[byte offset], the base uniform over the wave
+template <typename T>
+__device__ __forceinline__ T harm_at_byte(const T *p, uint32_t off) {
+  return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(p) + off);
+}
+
+
+// ---------------------------------------------------------------------------
+// moments of the atoms -> coefficients of the radial nodes
+
+// Radial values of one degree l at one atom: rows p of `tab` (pitch AS) get
+// scale R_{l,p} at x, for p < 4 PK.  J: the recurrence constants of the degree
+// (staged in LDS, two scalars per p).
+template <typename T>
+__device__ __forceinline__ void harm_radial(const T *J, T x, T scale,
+                                            uint32_t PK, T *tab, uint32_t AS) {
+  T v1 = scale, v2 = T(0);
+  tab[0] = scale;
+#pragma unroll
+  for (uint32_t u = 1; u < 4; ++u) {
+    const T v = harm_fma(x + J[2 * u], v1, -J[2 * u + 1] * v2);
+    tab[u * AS] = v;
+    v2 = v1;
+    v1 = v;
+  }
+  for (uint32_t k = 1; k < PK; ++k) {
+    J += 8;
+    tab += 4 * AS;
+    T c[8];
+#pragma unroll
+    for (uint32_t u = 0; u < 8; ++u) c[u] = J[u];
+#pragma unroll
+    for (uint32_t u = 0; u < 4; ++u) {
+      const T v = harm_fma(x + c[2 * u], v1, -c[2 * u + 1] * v2);
+      tab[u * AS] = v;
+      v2 = v1;
+      v1 = v;
+    }
+  }
+}
+// Stages `n` scalars of a constant table.
+template <typename T>
+__device__ __forceinline__ void harm_stage(T *dst, const T *src, uint32_t n) {
+  for (uint32_t e = threadIdx.x; e < n; e += blockDim.x) dst[e] = src[e];
+}
+
+// degrees per round of the radial tables
+template <typename T>
+constexpr uint32_t harm_lb() {
+  return sizeof(T) == 4 ? 4 : 2;
+}
+constexpr int kHarmBlock = 512;  // threads of the transform kernels
+
+template <int V>
+struct HarmInt {
+  static constexpr int value = V;
+};
+// f(HarmInt<n>) for the uniform n in 1 .. MAX: the inner loops have constant
+// lengths (conditional steps would copy the accumulators at every branch)
+template <int MAX, class F>
+void harm_host_switch(uint32_t n, F f) {
+  if constexpr (MAX <= 1) {
+    f(HarmInt<1>{});
+  } else {
+    if (n >= static_cast<uint32_t>(MAX))
+      f(HarmInt<MAX>{});
+    else
+      harm_host_switch<MAX - 1>(n, f);
+  }
+}
+template <int MAX, class F>
+__device__ __forceinline__ void harm_switch(uint32_t n, F f) {
+  if constexpr (MAX <= 1) {
+    f(HarmInt<1>{});
+  } else {
+    if (n >= static_cast<uint32_t>(MAX))
+      f(HarmInt<MAX>{});
+    else
+      harm_switch<MAX - 1>(n, f);
+  }
+}
+
+// One workgroup per cell, wave t on the azimuthal orders 8 t .. 8 t + 7.  A
+// wave walks the degrees l of its tile: lane (c, g) carries the solid harmonic
+// of column c (order, cosine or sine) at the atoms 4k + g through the
+// recurrence in l, and
+//   Q[p][column] = sum_atoms (q R_{l,p}) Y        (steps of four atoms)
+// is one product per degree.  The radial values of LB degrees at a time are
+// tabulated in LDS by all waves; the recurrence constants of a round are
+// loaded during the one before and go through LDS too (a load inside the loop
+// over the degrees would wait for the stores before it).  Cells of more than
+// 4 KS atoms take several passes that add up in `mom`.  336 and 1,637 us
+// (422 and 1,560 with the constants loaded per degree), bound by the latency
+// of the LDS reads between the products: 59 % of the wave cycles wait.  FP32
+// takes 64 atoms a pass (more registers leave fewer waves: 388 us at 128),
+// FP64 up to 128 (1,880 us at 64).
+template <typename T, int KS>
+__device__ __forceinline__ void harm_moments_body(
+    const HarmDev<T> &H, const typename HarmRecord<T>::type *atoms,
+    const uint32_t *start, uint32_t ny, uint32_t nz, double h, uint32_t cell,
+    uint32_t turn, T *mom, uint32_t *outside, char *smem) {
+  using M = Harm<T>;
+  using v4 = typename M::v4;
+  constexpr uint32_t CH = 4 * KS, AS = CH + 4, LB = harm_lb<T>();
+  const uint32_t tid = threadIdx.x, nth = blockDim.x, nwave = nth >> 6;
+  const uint32_t lane = tid & 63u;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // the tiles' lengths differ: the first one is another wave (another SIMD)
+  // from workgroup to workgroup
+  const uint32_t t = (wave + turn) % nwave;
+  const uint32_t c16 = lane & 15u, g = lane >> 4;
+  const uint32_t N = H.N;
+  const uint32_t prow = 4 * harm_psteps(0, N);
+  T *xs = reinterpret_cast<T *>(smem);
+  T *ys = xs + CH, *zs = ys + CH;  // zs: (z, s) pairs
+  T *ts = zs + 2 * CH, *qs = ts + CH;
+  // radial tables [LB][prow][AS]; first the powers [16 nt][AS]
+  T *zt = qs + CH;
+  const uint32_t trow = LB * prow > 16 * nwave ? LB * prow : 16 * nwave;
+  T *rec = zt + trow * AS;             // [LB][8 nt]
+  T *jac = rec + LB * 8 * nwave;       // [crow[N]][2]
+  const uint32_t jrows = H.jrows;
+  uint32_t *flag = reinterpret_cast<uint32_t *>(jac + 2 * jrows);
+  if (tid == 0) *flag = 0u;
+  harm_stage(jac, H.jac, 2 * jrows);
+  const uint32_t a0 = start[cell], na = start[cell + 1] - a0;
+  const HarmCentre cc = harm_centre(cell, ny, nz, h);
+  T *out = mom + static_cast<size_t>(cell) * H.rows * 16;
+  const uint32_t pr = M::perm(c16);  // radial index of this lane's A row
+  const uint32_t row0 = (pr < prow ? pr : prow - 1) * AS + g;
+  const uint32_t row1 = (16 + pr < prow ? 16 + pr : prow - 1) * AS + g;
+  const uint32_t mu = 8 * t + (c16 >> 1);
+  for (uint32_t p0 = 0; p0 == 0 || p0 < na; p0 += CH) {
+    const uint32_t cnt = na - p0 < CH ? na - p0 : CH;
+    harm_barrier();
+    for (uint32_t e = tid; e < CH; e += nth) {
+      HarmAtom<T> a = {};
+      if (e < cnt) {
+        a = harm_atom(H, atoms, a0 + p0 + e, cc);
+        if (a.out) {
+          *flag = 1u;
+          a.q = T(0);
+        }
+      }
+      xs[e] = a.x;
+      ys[e] = a.y;
+      zs[2 * e] = a.z;
+      zs[2 * e + 1] = a.s;
+      ts[e] = a.t;
+      qs[e] = a.q;
+    }
+    harm_barrier();
+    // groups of four steps of four atoms (the staged atoms past cnt are zero)
+    const uint32_t ng = cnt ? (cnt + 31) / 32 * 2 : 2u;
+    // (x + i y)^mu of every atom, mu < 8 nt, for the start values
+    for (uint32_t e = tid; e < 16 * ng; e += nth) {
+      const T X = xs[e], Y = ys[e];
+      T re = T(1), im = T(0);
+      for (uint32_t m = 0; m < 8 * nwave; ++m) {
+        zt[(2 * m) * AS + e] = re;
+        zt[(2 * m + 1) * AS + e] = im;
+        const T nr = re * X - im * Y;
+        im = re * Y + im * X;
+        re = nr;
+      }
+    }
+    harm_barrier();
+    harm_switch<KS / 8>((ng + 1) / 2, [&](auto half) {
+      constexpr int NK = 8 * decltype(half)::value;  // steps of four atoms
+      T Y1[NK], Y2[NK];
+#pragma unroll
+      for (int k = 0; k < NK; ++k) {
+        Y1[k] = zt[(2 * mu + (c16 & 1u)) * AS + 4 * k + g];
+        Y2[k] = T(0);
+      }
+      harm_barrier();
+      // recurrence constants: thread e holds scalar e of a round's
+      // [LB][8 nt] (whole rounds are allocated)
+      const uint32_t rl = tid / (8 * nwave), rm = tid - rl * 8 * nwave;
+      const T *rc = H.rec + (static_cast<size_t>(rl) * 64 + rm) * 2;
+      T rnext = rl < LB ? rc[0] : T(0);
+      T *o = out + (H.qoff[t] + H.crow[8 * t]) * 16 + lane;
+      // one degree: PT row tiles of radial polynomials
+      // A: Y of the degree before; B: of the one before that, then of this
+      auto degree = [&](auto tiles, uint32_t l, T(&A)[NK], T(&B)[NK]) {
+        constexpr int PT = decltype(tiles)::value;
+        const uint32_t PK = harm_psteps(l, N);
+        const T *zl = zt + (l % LB) * prow * AS;
+        const T rb = rec[(l % LB) * 8 * nwave + mu];
+        const T ra = l > mu ? T(1) : T(0), one = T(1) - ra;
+        // (partial sums: the rounding of a sum grows with its length)
+        constexpr int NA = sizeof(T) == 4 ? 4 / PT : 1;
+        v4 a0s[NA], a1s[NA];
+#pragma unroll
+        for (int i = 0; i < NA; ++i)
+          a0s[i] = a1s[i] = v4{T(0), T(0), T(0), T(0)};
+#pragma unroll
+        for (int k = 0; k < NK; ++k) {
+          const T z = zs[2 * (4 * k + g)], s = zs[2 * (4 * k + g) + 1];
+          const T y = harm_fma(harm_fma(ra, z, one), A[k], -(rb * s) * B[k]);
+          B[k] = y;
+          a0s[k % NA] = M::mfma(zl[row0 + 4 * k], y, a0s[k % NA]);
+          if (PT > 1) a1s[k % NA] = M::mfma(zl[row1 + 4 * k], y, a1s[k % NA]);
+        }
+#pragma unroll
+        for (int w = NA / 2; w > 0; w /= 2)
+#pragma unroll
+          for (int i = 0; i < w; ++i) {
+            a0s[i] += a0s[i + w];
+            if (PT > 1) a1s[i] += a1s[i + w];
+          }
+        v4 acc0 = a0s[0], acc1 = a1s[0];
+        // orders above the degree are zero; register r holds the rows
+        // p = 4 r + g
+#pragma unroll
+        for (uint32_t r = 0; r < 4; ++r) {
+          acc0[r] = mu > l ? T(0) : acc0[r];
+          if (PT > 1) acc1[r] = mu > l ? T(0) : acc1[r];
+        }
+        if (p0 == 0) {
+#pragma unroll
+          for (uint32_t r = 0; r < 4 * PT; ++r)
+            if (r < PK) o[r * 64] = r < 4 ? acc0[r & 3u] : acc1[r & 3u];
+        } else {
+          for (uint32_t r = 0; r < PK; ++r) {
+            const v4 a = r < 4 ? acc0 : acc1;
+            o[r * 64] += (r & 3u) == 0   ? a[0]
+                         : (r & 3u) == 1 ? a[1]
+                         : (r & 3u) == 2 ? a[2]
+                                         : a[3];
+          }
+        }
+        o += PK * 64;
+      };
+      for (uint32_t l0 = 0; l0 < N; l0 += LB) {
+        const uint32_t nl = N - l0 < LB ? N - l0 : LB;
+        const uint32_t nch = (16 * ng + 63) / 64;
+        if (rl < LB) {
+          rec[tid] = rnext;
+          rc += LB * 64 * 2;
+          rnext = rc[0];
+        }
+        for (uint32_t e = wave; e < nl * nch; e += nwave) {
+          const uint32_t ch = e / nl, l = l0 + (e - ch * nl);
+          const uint32_t a = ch * 64 + lane;
+          if (a < 16 * ng)
+            harm_radial(jac + 2 * H.crow[l],
+                        ts[a], qs[a], harm_psteps(l, N), zt + (l - l0) * prow * AS + a, AS);
+        }
+        harm_barrier();
+        for (uint32_t l = l0 < 8 * t ? 8 * t : l0; l < l0 + nl; l += 2) {
+          if (harm_psteps(l, N) > 4)
+            degree(HarmInt<2>{}, l, Y1, Y2);
+          else
+            degree(HarmInt<1>{}, l, Y1, Y2);
+          if (l + 1 < N) {
+            if (harm_psteps(l + 1, N) > 4)
+              degree(HarmInt<2>{}, l + 1, Y2, Y1);
+            else
+              degree(HarmInt<1>{}, l + 1, Y2, Y1);
+          }
+        }
+        harm_barrier();
+      }
+    });
+  }
+  if (tid == 0) outside[cell] = *flag;
+}
+
+template <typename T, int KS>
+__global__ __launch_bounds__(512) void harm_moments_kernel(
+    HarmDev<T> H, const typename HarmRecord<T>::type *__restrict__ atoms,
+    const uint32_t *__restrict__ start, uint32_t ny, uint32_t nz, double h,
+    T *__restrict__ mom, uint32_t *__restrict__ outside) {
+  extern __shared__ char harm_smem[];
+  const uint32_t nb = gridDim.x, b = blockIdx.x;
+  const uint32_t q = nb >> 3, r = nb & 7u, x = b & 7u;
+  const uint32_t cell = x * q + (x < r ? x : r) + (b >> 3);
+  harm_moments_body<T, KS>(H, atoms, start, ny, nz, h, cell,
+                           (b >> 3) + (b >> 8), mom, outside,
+                           harm_smem);
+}
+
+// ---------------------------------------------------------------------------
+// moments <-> coefficients of the radial nodes
+
+// most steps over the radial polynomials of a degree
+template <typename T>
+constexpr int harm_max_psteps() {
+  return static_cast<int>(
+      (((sizeof(T) == 4 ? kHarmMaxN32 : kHarmMaxN) - 1) / 2 + 4) / 4);
+}
+
+// One wave: degree l and order tile t of the eight cells of a tile.  Forward:
+// B_i = sum_p gam_l[i][p] Q[p] for the radial nodes with more than l degrees,
+// the moments in registers for all eight cells; a lane ends with the eight
+// cells' values of one (node, column), adjacent in the coefficients.  73 and
+// 369 us forward, 108 and 286 us backward: memory traffic of the coefficients
+// (0.25 and 1.0 GB).
+template <typename T>
+__device__ __forceinline__ void harm_forward_wave(const HarmDev<T> &H,
+                                                  uint32_t ncell, uint32_t tile,
+                                                  uint32_t l, uint32_t t,
+                                                  const T *mom, T *coef) {
+  using M = Harm<T>;
+  using v4 = typename M::v4;
+  constexpr int MAXPK = harm_max_psteps<T>();
+  const uint32_t lane = threadIdx.x & 63u, c16 = lane & 15u, g = lane >> 4;
+  const uint4 lr = H.lrow[l];
+  const size_t cs = static_cast<size_t>(H.rows) * 16;
+  const T *Q = mom + static_cast<size_t>(H.qoff[t] + H.crow[l]) * 16 + lane;
+  T *out = coef + static_cast<size_t>(tile) * H.stride * 8;
+  harm_switch<MAXPK>(harm_psteps(l, H.N), [&](auto steps) {
+    constexpr int PK = decltype(steps)::value;
+    T q[8][PK];
+#pragma unroll
+    for (uint32_t c = 0; c < 8; ++c) {
+      const uint32_t cell = tile * 8 + c < ncell ? tile * 8 + c : ncell - 1;
+      const T *p = Q + cell * cs;
+#pragma unroll
+      for (int r = 0; r < PK; ++r) q[c][r] = p[r * 64];
+    }
+    const T *G = H.gam + static_cast<size_t>(lr.x) * 64 + lane;
+    T gm[PK];
+#pragma unroll
+    for (int r = 0; r < PK; ++r) gm[r] = G[r * 64];
+    for (uint32_t i0 = 0; i0 < lr.z; i0 += 16) {
+      T gx[PK];
+#pragma unroll
+      for (int r = 0; r < PK; ++r) gx[r] = gm[r];
+      G += PK * 64;  // (the table has room for one more load)
+#pragma unroll
+      for (int r = 0; r < PK; ++r) gm[r] = G[r * 64];
+      HarmRad ri[4];
+#pragma unroll
+      for (uint32_t r = 0; r < 4; ++r) {
+        const uint32_t i = i0 + M::row(g, r);
+        ri[r] = H.rad[i < H.nrad ? i : H.nrad - 1];
+      }
+      v4 d[8];
+#pragma unroll
+      for (uint32_t c = 0; c < 8; ++c) d[c] = v4{T(0), T(0), T(0), T(0)};
+#pragma unroll
+      for (int r = 0; r < PK; ++r)
+#pragma unroll
+        for (uint32_t c = 0; c < 8; ++c) d[c] = M::mfma(gx[r], q[c][r], d[c]);
+#pragma unroll
+      for (uint32_t r = 0; r < 4; ++r)
+        if (i0 + M::row(g, r) < lr.z) {
+          v4 *o = reinterpret_cast<v4 *>(
+              out + (ri[r].off + harm_block(t, l, ri[r].N) * 16 + c16) * 8);
+          o[0] = v4{d[0][r], d[1][r], d[2][r], d[3][r]};
+          o[1] = v4{d[4][r], d[5][r], d[6][r], d[7][r]};
+        }
+    }
+  });
+}
+
+// Backward: U[p] = sum_i gam_l[i][p] C_i, per (l, order) the pairs (cosine,
+// sine) of the rows p side by side.
+template <typename T>
+__device__ __forceinline__ void harm_backward_wave(const HarmDev<T> &H,
+                                                   uint32_t ncell,
+                                                   uint32_t tile, uint32_t l,
+                                                   uint32_t t, const T *coef,
+                                                   T *mom) {
+  using M = Harm<T>;
+  using v4 = typename M::v4;
+  const uint32_t lane = threadIdx.x & 63u, c16 = lane & 15u, g = lane >> 4;
+  const uint32_t PK = harm_psteps(l, H.N);
+  const uint4 lr = H.lrow[l];
+  const uint32_t mu = 8 * t + (c16 >> 1);
+  const T *G = H.gamt + static_cast<size_t>(lr.y) * 64 + lane;
+  const T *in = coef + static_cast<size_t>(tile) * H.stride * 8 + c16 * 8;
+  T *o = mom + 8 * (H.urow[l] + mu * PK) + 2 * g + (c16 & 1u);
+  harm_switch<2>(PK > 4 ? 2u : 1u, [&](auto tiles) {
+    constexpr int PT = decltype(tiles)::value;
+    v4 d[PT][8];
+#pragma unroll
+    for (int p = 0; p < PT; ++p)
+#pragma unroll
+      for (uint32_t c = 0; c < 8; ++c) d[p][c] = v4{T(0), T(0), T(0), T(0)};
+    // four radial nodes a step, two steps in flight; nodes past the last
+    // have zero factors and repeat it
+    for (uint32_t i0 = 0; i0 < lr.z; i0 += 8) {
+      v4 b[2][2];
+      T ga[2][PT];
+#pragma unroll
+      for (uint32_t u = 0; u < 2; ++u) {
+        const uint32_t i = i0 + 4 * u + g;
+        const HarmRad ri = H.rad[i < lr.z ? i : lr.z - 1];
+        const v4 *p = reinterpret_cast<const v4 *>(
+            in + (ri.off + harm_block(t, l, ri.N) * 16) * 8);
+        b[u][0] = p[0];
+        b[u][1] = p[1];
+#pragma unroll
+        for (int p2 = 0; p2 < PT; ++p2) {
+          const T x = G[(u * PT + p2) * 64];
+          ga[u][p2] = i0 + 4 * u < lr.z ? x : T(0);
+        }
+      }
+      G += 2 * PT * 64;
+#pragma unroll
+      for (uint32_t u = 0; u < 2; ++u)
+#pragma unroll
+        for (int p = 0; p < PT; ++p)
+#pragma unroll
+          for (uint32_t c = 0; c < 8; ++c)
+            d[p][c] = M::mfma(ga[u][p], b[u][c >> 2][c & 3u], d[p][c]);
+    }
+#pragma unroll
+    for (uint32_t c = 0; c < 8; ++c) {
+      if (tile * 8 + c >= ncell) break;
+      T *p = o + static_cast<size_t>(tile * 8 + c) * H.ustride;
+#pragma unroll
+      for (uint32_t r = 0; r < 4 * PT; ++r)
+        if (r < PK && mu <= l) p[r * 8] = d[r >> 2][c][r & 3u];
+    }
+  });
+}
+
+// Wave w of a launch: tile w / (pairs) and the (l, t) pair w % pairs of the
+// plan.
+template <typename T, bool BACK>
+__global__ __launch_bounds__(256) void harm_radial_kernel(
+    HarmDev<T> H, uint32_t ncell, uint32_t nwave, const T *__restrict__ in,
+    T *__restrict__ out) {
+  const uint32_t nb = gridDim.x, b = blockIdx.x;
+  const uint32_t q = nb >> 3, r = nb & 7u, x = b & 7u;
+  const uint32_t w =
+      (x * q + (x < r ? x : r) + (b >> 3)) * 4 +
+      __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (w >= nwave) return;
+  const uint32_t tile = w / H.npair;
+  const uint2 lt = H.pair[w - tile * H.npair];
+  if (BACK)
+    harm_backward_wave(H, ncell, tile, lt.x, lt.y, in, out);
+  else
+    harm_forward_wave(H, ncell, tile, lt.x, lt.y, in, out);
+}
+
+// ---------------------------------------------------------------------------
+// coefficients -> structure factors (414 and 1,197 us; the wave's share of the
+// tables' loads and index arithmetic, about as many scalar as vector
+// instructions, against 0.15 and 0.29 ms of stores)
+
+// Which (unit, cell tile) a workgroup serves.  With many tiles every XCD
+// (workgroups b with b % 8 == x) owns a contiguous range of them and takes
+// it unit by unit: neighbouring tiles, which share lines of S, run there at
+// the same time, and every XCD has all the units.
+__device__ __forceinline__ bool harm_place(uint32_t b, uint32_t ntile,
+                                           uint32_t nunit, uint32_t &unit,
+                                           uint32_t &tile) {
+  if (ntile < 64) {
+    unit = b / ntile;
+    tile = b - unit * ntile;
+    return unit < nunit;
+  }
+  const uint32_t x = b & 7u, i = b >> 3, q = ntile >> 3, r = ntile & 7u;
+  const uint32_t n = q + (x < r ? 1u : 0u);
+  unit = i / n;
+  tile = x * q + (x < r ? x : r) + (i - unit * n);
+  return unit < nunit;
+}
+uint32_t harm_grid(uint32_t ntile, uint32_t nunit) {
+  if (ntile < 64) return ntile * nunit;
+  return 8 * nunit * ((ntile + 7) / 8);
+}
+
+// Modes of one set (even or odd azimuthal orders), padded to whole steps of
+// four: mode 2 m + cs is the cosine (cs 0) or sine of order 2 m + set.
+__device__ __forceinline__ uint32_t harm_mode_steps(uint32_t N) {
+  return ((N + 1) / 2 + 1) / 2;
+}
+
+// One unit: eight cells, one radial node, a tile of 16 rings.  Even and odd
+// orders take turns: (1) Legendre: per order, the rings' Fourier coefficients
+// of Re (even degrees) and Im (odd degrees) into LDS; columns are (cosine or
+// sine, cell); a wave's next order is loaded while it works on one.  (2)
+// Fourier: per ring (wave and wave + 8 in FP32), the sums E over the even and
+// O over the odd orders at NPT tiles of azimuths, in registers; the values at
+// phi and phi + pi are E + O and E - O.  Columns are (cell, Re or Im) in FP32;
+// in FP64 Re and Im take turns and the columns are (ring of a pair, cell).
+template <typename T, int NPT>
+__device__ __forceinline__ void harm_sf_body(
+    const HarmDev<T> &H, const typename HarmRecord<T>::type *atoms,
+    const uint32_t *start, const double4 *k64, uint32_t ny, uint32_t nz,
+    double h, uint32_t ncell, const HarmRad &rad, const HarmGroup &gr,
+    uint32_t rt, uint32_t tile, const T *coef, const uint32_t *outside, T *S,
+    char *smem) {
+  using M = Harm<T>;
+  using v4 = typename M::v4;
+  constexpr bool F = sizeof(T) == 4;
+  constexpr uint32_t NW = kHarmBlock / 64;
+  constexpr int NR = F ? 2 : 1;  // rows of (2) per wave
+  constexpr int NP = F ? 2 : 1;  // parities per pass of (1)
+  const uint32_t tid = threadIdx.x;
+  const uint32_t lane = tid & 63u;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t c16 = lane & 15u, g = lane >> 4;
+  const uint32_t N = rad.N, KS = harm_mode_steps(N), MS = 4 * KS;
+  const uint32_t RS = MS * 16 + 8;
+  const uint32_t nrow = F ? 16u : 8u;
+  T *Gm = reinterpret_cast<T *>(smem);
+  T *tr = Gm + nrow * RS;
+  const uint32_t cell0 = tile * kHarmCells;
+  const uint32_t ncp = harm_row(ncell);
+  // columns of (1): the cosines of the eight cells, then the sines
+  const uint32_t c8 = c16 & 7u, cs = c16 >> 3;
+  const T *cf = coef + (static_cast<size_t>(tile) * H.stride + rad.off) * 8 + c16;
+  const T *leg = H.leg + (static_cast<size_t>(gr.leg) + rt * gr.leg_n) * 64 + lane;
+  for (uint32_t pass = 0; pass < (F ? 1u : 2u); ++pass) {
+    v4 E[NR][NPT];
+#pragma unroll
+    for (uint32_t set = 0; set < 2; ++set) {
+      // the Fourier matrix of the set, as far as this node's degrees go
+      for (uint32_t e = wave; e < NPT * KS; e += NW) {
+        const uint32_t pt = e / KS, ks = e - pt * KS;
+        tr[e * 64 + lane] =
+            H.trig[(static_cast<size_t>(gr.trig) +
+                    (2 * pt + set) * gr.trig_k + ks) * 64 + lane];
+      }
+      // (1) degrees l0, l0 + 2, ... of a parity: the first 16 in flight
+      T la[NP][4], lb[NP][4];
+      auto degrees = [&](uint32_t mu, uint32_t par, uint32_t &l0) {
+        l0 = mu + ((mu ^ par) & 1u);
+        return l0 < N ? (N - l0 + 1) / 2 : 0u;
+      };
+      auto fetch = [&](uint32_t mu) {
+#pragma unroll
+        for (uint32_t pp = 0; pp < NP; ++pp) {
+          const uint32_t par = F ? pp : pass;
+          uint32_t l0;
+          const uint32_t n = degrees(mu, par, l0);
+          const T *A = leg + H.mup[gr.mup + 2 * mu + par].x * 64;
+          const T *B = cf + (n ? harm_block(mu >> 3, l0, N) * 16 +
+                                     2 * (mu & 7u) : 0u) * 8;
+#pragma unroll
+          for (uint32_t u = 0; u < 4; ++u) {
+            const uint32_t j = 4 * u + g;
+            la[pp][u] = A[u * 64];  // (the table ends with four more steps)
+            const T b = B[(j < n ? j : 0u) * 256];
+            lb[pp][u] = j < n ? b : T(0);
+          }
+        }
+      };
+      if (2 * wave + set < N) fetch(2 * wave + set);
+      for (uint32_t m = wave; m < 2 * KS; m += NW) {
+        const uint32_t mu = 2 * m + set, mode = 2 * m + cs;
+        v4 acc[NP];
+#pragma unroll
+        for (uint32_t pp = 0; pp < NP; ++pp)
+          acc[pp] = v4{T(0), T(0), T(0), T(0)};
+        if (mu < N) {
+          T xa[NP][4], xb[NP][4];
+#pragma unroll
+          for (uint32_t pp = 0; pp < NP; ++pp)
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) {
+              xa[pp][u] = la[pp][u];
+              xb[pp][u] = lb[pp][u];
+            }
+          if (mu + 2 * NW < N) fetch(mu + 2 * NW);
+#pragma unroll
+          for (uint32_t u = 0; u < 4; ++u)
+#pragma unroll
+            for (uint32_t pp = 0; pp < NP; ++pp)
+              acc[pp] = M::mfma(xa[pp][u], xb[pp][u], acc[pp]);
+#pragma unroll
+          for (uint32_t pp = 0; pp < NP; ++pp) {
+            const uint32_t par = F ? pp : pass;
+            uint32_t l0;
+            const uint32_t n = degrees(mu, par, l0);
+            if (n > 16) {
+              const T *A = leg + H.mup[gr.mup + 2 * mu + par].x * 64;
+              const T *B =
+                  cf + (harm_block(mu >> 3, l0, N) * 16 + 2 * (mu & 7u)) * 8;
+              for (uint32_t k = 16; k < n; k += 4) {
+                const uint32_t j = k + g;
+                const T b = B[(j < n ? j : 0u) * 256];
+                acc[pp] = M::mfma(A[k * 16], j < n ? b : T(0), acc[pp]);
+              }
+            }
+          }
+        }
+#pragma unroll
+        for (uint32_t pp = 0; pp < NP; ++pp)
+#pragma unroll
+          for (uint32_t r = 0; r < 4; ++r) {
+            const uint32_t ring = M::row(g, r);
+            if (F)
+              Gm[ring * RS + mode * 16 + c8 * 2 + pp] = acc[pp][r];
+            else
+              Gm[(ring >> 1) * RS + mode * 16 + (ring & 1u) * 8 + c8] =
+                  acc[pp][r];
+          }
+      }
+      harm_barrier();
+      // (2)
+      v4 X[NR][NPT];
+#pragma unroll
+      for (int u = 0; u < NR; ++u)
+#pragma unroll
+        for (int pt = 0; pt < NPT; ++pt) X[u][pt] = v4{T(0), T(0), T(0), T(0)};
+      const T *At = tr + lane, *Bt = Gm + wave * RS + lane;
+#pragma unroll 2
+      for (uint32_t ks = 0; ks < KS; ++ks) {
+        T a[NPT], b[NR];
+#pragma unroll
+        for (int pt = 0; pt < NPT; ++pt) a[pt] = At[(pt * KS + ks) * 64];
+#pragma unroll
+        for (int u = 0; u < NR; ++u) b[u] = Bt[u * NW * RS + ks * 64];
+#pragma unroll
+        for (int u = 0; u < NR; ++u)
+#pragma unroll
+          for (int pt = 0; pt < NPT; ++pt)
+            X[u][pt] = M::mfma(a[pt], b[u], X[u][pt]);
+      }
+      harm_barrier();
+      if (set == 0) {
+#pragma unroll
+        for (int u = 0; u < NR; ++u)
+#pragma unroll
+          for (int pt = 0; pt < NPT; ++pt) E[u][pt] = X[u][pt];
+      } else {
+        // bytes of an azimuth: a ring's offsets fit 32 bits
+        const uint32_t az =
+            gr.nr * static_cast<uint32_t>(2 * ncp * sizeof(T));
+#pragma unroll
+        for (int u = 0; u < NR; ++u) {
+          const uint32_t row = wave + u * NW;
+          const uint32_t ring0 = 16 * rt + (F ? row : 2 * row);
+          if (ring0 >= gr.nring) continue;
+          const uint32_t dir0 =
+              gr.equator ? (ring0 ? gr.h + 2 * gr.h * (ring0 - 1) : 0u)
+                         : 2 * gr.h * ring0;
+          char *base = reinterpret_cast<char *>(
+              S + harm_slot<T>(gr.node0 + dir0 * gr.nr + rad.idx, cell0,
+                               F ? 0u : pass, ncp));
+          bool eq = gr.equator && ring0 == 0, on = true;
+          uint32_t off = c16 * 4;
+          if (!F) {  // lanes 8 .. 15 of a row: the next ring
+            const bool next = c16 >> 3;
+            off = (c16 & 7u) * 8 + (next ? (eq ? gr.h : 2 * gr.h) * az : 0u);
+            on = !next || ring0 + 1 < gr.nring;
+            eq = eq && !next;
+          }
+#pragma unroll
+          for (int pt = 0; pt < NPT; ++pt)
+#pragma unroll
+            for (uint32_t r = 0; r < 4; ++r) {
+              const uint32_t phi = 16 * pt + M::row(g, r);
+              if (phi < gr.h && on) {
+                const uint32_t oa = off + phi * az;
+                *reinterpret_cast<T *>(base + oa) = E[u][pt][r] + X[u][pt][r];
+                if (!eq)
+                  *reinterpret_cast<T *>(base + oa + gr.h * az) =
+                      E[u][pt][r] - X[u][pt][r];
+              }
+            }
+        }
+      }
+    }
+  }
+  uint32_t any = 0;
+  for (uint32_t c = 0; c < kHarmCells; ++c)
+    if (cell0 + c < ncell) any |= outside[cell0 + c];
+  if (!any) return;
+  // atoms outside the unit ball: their terms one by one
+  __syncthreads();
+  const uint32_t nd = gr.nring * 2 * gr.h - (gr.equator ? gr.h : 0u);
+  const uint32_t d0 = rt ? 32 * gr.h * rt - (gr.equator ? gr.h : 0u) : 0u;
+  const uint32_t d1 =
+      32 * gr.h * (rt + 1) - (gr.equator ? gr.h : 0u) < nd
+          ? 32 * gr.h * (rt + 1) - (gr.equator ? gr.h : 0u)
+          : nd;
+  for (uint32_t e = tid; e < (d1 - d0) * kHarmCells; e += kHarmBlock) {
+    const uint32_t cell = cell0 + (e & (kHarmCells - 1));
+    if (cell >= ncell || !outside[cell]) continue;
+    const uint32_t node = gr.node0 + (d0 + e / kHarmCells) * gr.nr + rad.idx;
+    const double4 k = k64[node];
+    const HarmCentre cc = harm_centre(cell, ny, nz, h);
+    double re = 0.0, im = 0.0;
+    for (uint32_t j = start[cell]; j < start[cell + 1]; ++j) {
+      if (harm_atom(H, atoms, j, cc).out) {
+        const HarmOffset d = harm_offset(atoms, j, cc);
+        const double ph = k.x * d.x + k.y * d.y + k.z * d.z;
+        re += d.q * cos(ph);
+        im -= d.q * sin(ph);
+      }
+    }
+    T *sr = S + harm_slot<T>(node, cell, 0, ncp);
+    T *si = S + harm_slot<T>(node, cell, 1, ncp);
+    *sr += static_cast<T>(re);
+    *si += static_cast<T>(im);
+  }
+}
+
+template <typename T, int NPT>
+__global__ __launch_bounds__(kHarmBlock) void harm_sf_kernel(
+    HarmDev<T> H, const uint2 *__restrict__ units, uint32_t nunit,
+    const typename HarmRecord<T>::type *__restrict__ atoms,
+    const uint32_t *__restrict__ start, const double4 *__restrict__ k64,
+    uint32_t ny, uint32_t nz, double h, uint32_t ncell,
+    const T *__restrict__ coef, const uint32_t *__restrict__ outside,
+    T *__restrict__ S) {
+  extern __shared__ char harm_smem[];
+  uint32_t unit, tile;
+  if (!harm_place(blockIdx.x, (ncell + kHarmCells - 1) / kHarmCells, nunit,
+                  unit, tile))
+    return;
+  const uint2 u = units[unit];
+  const HarmRad rad = H.rad[u.x];
+  const HarmGroup gr = H.grp[rad.group];
+  // tiles of 16 azimuths over half a ring
+  harm_switch<NPT>((gr.h + 15) / 16, [&](auto npt) {
+    harm_sf_body<T, decltype(npt)::value>(H, atoms, start, k64, ny, nz, h,
+                                          ncell, rad, gr, u.y, tile, coef,
+                                          outside, S, harm_smem);
+  });
+}
+
+// ---------------------------------------------------------------------------
+// remote sums -> coefficients (436 and 1,310 us; reads R once, 0.15 and 0.29 ms,
+// and is held by the wait for it and by the same overhead as harm_sf)
+
+// One unit: eight cells, one radial node, all rings; the transpose of
+// harm_sf_body.  Every wave first loads its rings' values, all loads in
+// flight at once (RW rows of 2 HK values per lane; FP64 rows are pairs of
+// rings, and Re and Im take turns).  Even and odd orders take turns, so that
+// all the rings' Fourier sums of one set fit in LDS: (1) per ring, the sums
+// over the azimuths of V(phi) +- V(phi + pi) against the cosines and sines;
+// (2) per order and parity, the sums over the rings against the Legendre
+// functions, stored as the cells' coefficients.
+template <typename T, int RW, int HK, int MT>
+__device__ __forceinline__ void harm_lr_body(
+    const HarmDev<T> &H, uint32_t ncell, const HarmRad &rad,
+    const HarmGroup &gr, uint32_t tile, const T *R, T *coef, char *smem) {
+  using M = Harm<T>;
+  using v4 = typename M::v4;
+  constexpr bool F = sizeof(T) == 4;
+  constexpr uint32_t NW = kHarmBlock / 64;
+  constexpr int NP = F ? 2 : 1;  // parities per pass of (2)
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t c16 = lane & 15u, g = lane >> 4;
+  const uint32_t N = rad.N, KS = harm_mode_steps(N), MS = 4 * KS;
+  const uint32_t RS = MS * 16 + 8;
+  const uint32_t hk = gr.trigt_k;
+  const uint32_t nrow = F ? 4 * gr.legt_k : 2 * gr.legt_k;  // padded rings
+  T *Gm = reinterpret_cast<T *>(smem);
+  T *tr = Gm + nrow * RS;
+  const uint32_t cell0 = tile * kHarmCells;
+  const uint32_t ncp = harm_row(ncell);
+  // columns of (2): the cosines of the eight cells, then the sines
+  const uint32_t c8 = c16 & 7u, cs = c16 >> 3;
+  T *cf = coef + (static_cast<size_t>(tile) * H.stride + rad.off) * 8 + c16;
+  const T *legt = H.legt + static_cast<size_t>(gr.legt) * 64 + lane;
+  // bytes of an azimuth: a row's offsets stay below 4 h of them (32 bits)
+  const uint32_t az = gr.nr * static_cast<uint32_t>(2 * ncp * sizeof(T));
+  for (uint32_t pass = 0; pass < (F ? 1u : 2u); ++pass) {
+    // A row past the rings and an azimuth past the half ring repeat the last
+    // one (their factors are zero); the equator has no second half.
+    T va[RW][HK], vb[RW][HK];
+#pragma unroll
+    for (int w = 0; w < RW; ++w) {
+      const uint32_t ring0 = F ? wave + w * NW : 2 * (wave + w * NW);
+      const uint32_t r0 = ring0 < gr.nring ? ring0 : gr.nring - 1;
+      const uint32_t dir0 =
+          gr.equator ? (r0 ? gr.h + 2 * gr.h * (r0 - 1) : 0u) : 2 * gr.h * r0;
+      const T *base = R + harm_slot<T>(gr.node0 + dir0 * gr.nr + rad.idx, cell0,
+                                       F ? 0u : pass, ncp);
+      const bool eq = gr.equator && r0 == 0;
+      uint32_t off = c16 * 4, second = eq ? 0u : gr.h * az;
+      if (!F) {  // lanes 8 .. 15 of a row: the next ring
+        const bool next = (c16 >> 3) && r0 + 1 < gr.nring;
+        off = (c16 & 7u) * 8 + (next ? (eq ? gr.h : 2 * gr.h) * az : 0u);
+        if (next) second = gr.h * az;
+      }
+      const uint32_t end = off + (gr.h - 1) * az;
+      off += g * az;
+#pragma unroll
+      for (int ks = 0; ks < HK; ++ks) {
+        const uint32_t o = off + 4 * ks * az;
+        const uint32_t oc = o < end ? o : end;
+        va[w][ks] = harm_at_byte(base, oc);
+        vb[w][ks] = harm_at_byte(base, oc + second);
+      }
+    }
+    if (pass == 0) {
+      for (uint32_t e = wave; e < 2 * MT * HK; e += NW) {
+        const uint32_t sm = e / HK, ks = e - sm * HK;
+        const uint32_t set = sm / MT, mt = sm - set * MT;
+        const T x = H.trigt[(static_cast<size_t>(gr.trigt) +
+                             (set * gr.trigt_m + mt) * hk +
+                             (ks < hk ? ks : 0u)) * 64 + lane];
+        tr[e * 64 + lane] = ks < hk ? x : T(0);
+      }
+      harm_barrier();
+    }
+    for (uint32_t set = 0; set < 2; ++set) {
+      T la[NP][4];
+      auto fetch = [&](uint32_t mu) {
+#pragma unroll
+        for (uint32_t pp = 0; pp < NP; ++pp) {
+          const T *A = legt + H.mup[gr.mup + 2 * mu + (F ? pp : pass)].y * 64;
+#pragma unroll
+          for (uint32_t u = 0; u < 4; ++u) la[pp][u] = A[u * 64];
+        }
+      };
+      if (2 * wave + set < N) fetch(2 * wave + set);
+      // (1)
+#pragma unroll
+      for (int w = 0; w < RW; ++w) {
+        const uint32_t row = wave + w * NW;
+        const uint32_t ring = F ? row : 2 * row + (c16 >> 3);
+        const T half2 = gr.equator && ring == 0 ? T(0) : set ? T(-1) : T(1);
+        // (partial sums: the rounding of a sum grows with its length)
+        constexpr int NA = F && MT == 1 ? 2 : 1;
+        v4 acc[MT * NA];
+#pragma unroll
+        for (int m = 0; m < MT * NA; ++m)
+          acc[m] = v4{T(0), T(0), T(0), T(0)};
+        const T *At = tr + set * MT * HK * 64 + lane;
+#pragma unroll
+        for (int ks = 0; ks < HK; ++ks) {
+          const T v = harm_fma(half2, vb[w][ks], va[w][ks]);
+#pragma unroll
+          for (int m = 0; m < MT; ++m)
+            acc[m + ks % NA] =
+                M::mfma(At[(m * HK + ks) * 64], v, acc[m + ks % NA]);
+        }
+        if (NA > 1) acc[0] += acc[NA - 1];
+        if (row < nrow) {
+#pragma unroll
+          for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (uint32_t r = 0; r < 4; ++r) {
+              const uint32_t mode = 16 * m + M::row(g, r);
+              if (mode < MS) Gm[row * RS + mode * 16 + c16] = acc[m][r];
+            }
+        }
+      }
+      harm_barrier();
+      // (2)
+      for (uint32_t m = wave; 2 * m + set < N; m += NW) {
+        const uint32_t mu = 2 * m + set;
+        const uint32_t mode = 2 * m + cs;
+        T xa[NP][4];
+#pragma unroll
+        for (uint32_t pp = 0; pp < NP; ++pp)
+#pragma unroll
+          for (uint32_t u = 0; u < 4; ++u) xa[pp][u] = la[pp][u];
+        if (mu + 2 * NW < N) fetch(mu + 2 * NW);
+        auto ring_sum = [&](uint32_t ks, uint32_t par) {
+          const uint32_t ring = 4 * ks + g;
+          return F ? Gm[ring * RS + mode * 16 + c8 * 2 + par]
+                   : Gm[(ring >> 1) * RS + mode * 16 + (ring & 1u) * 8 + c8];
+        };
+        v4 acc[NP];
+#pragma unroll
+        for (uint32_t pp = 0; pp < NP; ++pp)
+          acc[pp] = v4{T(0), T(0), T(0), T(0)};
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u)
+#pragma unroll
+          for (uint32_t pp = 0; pp < NP; ++pp)
+            acc[pp] = M::mfma(xa[pp][u], ring_sum(u, F ? pp : pass), acc[pp]);
+#pragma unroll
+        for (uint32_t pp = 0; pp < NP; ++pp) {
+          const uint32_t par = F ? pp : pass;
+          const uint32_t l0 = mu + ((mu ^ par) & 1u);
+          if (l0 >= N) continue;
+          const uint32_t n = (N - l0 + 1) / 2;
+          const T *A = legt + H.mup[gr.mup + 2 * mu + par].y * 64;
+          T *o = cf + (harm_block(mu >> 3, l0, N) * 16 + 2 * (mu & 7u)) * 8;
+          // rings past the first 16, degrees past the first 16 of a parity
+          for (uint32_t k = 4; k < gr.legt_k; ++k)
+            acc[pp] = M::mfma(A[k * 64], ring_sum(k, par), acc[pp]);
+#pragma unroll
+          for (uint32_t r = 0; r < 4; ++r) {
+            const uint32_t i = M::row(g, r);
+            if (i < n) o[i * 256] = acc[pp][r];
+          }
+          for (uint32_t i0 = 16; i0 < n; i0 += 16) {
+            A += gr.legt_k * 64;
+            v4 more = {T(0), T(0), T(0), T(0)};
+            for (uint32_t k = 0; k < gr.legt_k; ++k)
+              more = M::mfma(A[k * 64], ring_sum(k, par), more);
+#pragma unroll
+            for (uint32_t r = 0; r < 4; ++r) {
+              const uint32_t i = i0 + M::row(g, r);
+              if (i < n) o[i * 256] = more[r];
+            }
+          }
+        }
+      }
+      harm_barrier();
+    }
+  }
+}
+
+// Waves per SIMD that the registers of the rows' values leave room for.
+template <typename T>
+constexpr int harm_lr_waves(int hk) {
+  return sizeof(T) == 4 ? (hk <= 8 ? 5 : hk <= 12 ? 3 : 2) : (hk <= 8 ? 3 : 2);
+}
+template <typename T, int RW, int HK>
+__global__ __launch_bounds__(kHarmBlock, harm_lr_waves<T>(HK)) void harm_lr_kernel(
+    HarmDev<T> H, uint32_t ncell, const T *__restrict__ R,
+    T *__restrict__ coef) {
+  extern __shared__ char harm_smem[];
+  uint32_t unit, tile;
+  if (!harm_place(blockIdx.x, (ncell + kHarmCells - 1) / kHarmCells, H.nrad,
+                  unit, tile))
+    return;
+  const HarmRad rad = H.rad[unit];
+  const HarmGroup gr = H.grp[rad.group];
+  // tiles of 16 orders of a set; steps of four azimuths over half a ring
+  constexpr int MM = sizeof(T) == 4 ? 3 : 4;
+  harm_switch<MM>((harm_mode_steps(rad.N) + 3) / 4, [&](auto mt) {
+    constexpr int MT = decltype(mt)::value;
+    if (gr.trigt_k <= HK - 3)
+      harm_lr_body<T, RW, HK - 3, MT>(H, ncell, rad, gr, tile, R, coef,
+                                      harm_smem);
+    else
+      harm_lr_body<T, RW, HK, MT>(H, ncell, rad, gr, tile, R, coef, harm_smem);
+  });
+}
+
+// ---------------------------------------------------------------------------
+// coefficients -> energies and forces
+
+// Fields of an atom outside the unit ball: the direct sum over the nodes.
+template <typename T>
+__device__ void harm_outside_eval(const HarmOffset &a, uint32_t cell, const double4 *k64,
+                                  uint32_t K, const T *R, uint32_t ncp,
+                                  double *red, double4 *out) {
+  double e = 0.0, fx = 0.0, fy = 0.0, fz = 0.0;
+  for (uint32_t n = threadIdx.x; n < K; n += blockDim.x) {
+    const double4 k = k64[n];
+    const double ph = k.x * a.x + k.y * a.y + k.z * a.z;
+    const double vr = R[harm_slot<T>(n, cell, 0, ncp)];
+    const double vi = R[harm_slot<T>(n, cell, 1, ncp)];
+    const double c = cos(ph), s = sin(ph);
+    const double b = c * vi + s * vr;
+    e += c * vr - s * vi;
+    fx += k.x * b;
+    fy += k.y * b;
+    fz += k.z * b;
+  }
+  double v[4] = {fx, fy, fz, e};
+  for (int d = 0; d < 4; ++d) {
+    harm_barrier();
+    red[threadIdx.x] = v[d];
+    harm_barrier();
+    for (uint32_t o = 256; o > 0; o >>= 1) {
+      if (threadIdx.x < o && threadIdx.x + o < blockDim.x)
+        red[threadIdx.x] += red[threadIdx.x + o];
+      harm_barrier();
+    }
+    v[d] = red[0];
+  }
+  harm_barrier();
+  if (threadIdx.x == 0) {
+    *out = make_double4(a.q * v[0], a.q * v[1], a.q * v[2], a.q * v[3]);
+  }
+}
+
+// Uniform loads of constant data.
+template <typename T>
+using HarmConst = const __attribute__((address_space(4))) T;
+template <typename T>
+__device__ __forceinline__ HarmConst<T> *harm_const(const T *p) {
+  return reinterpret_cast<HarmConst<T> *>(reinterpret_cast<uintptr_t>(p));
+}
+
+// One workgroup per cell and 64 of its atoms at a time, a lane per atom.  Wave
+// w takes the azimuthal orders w, 2W - 1 - w, 2W + w, ... (W waves: their
+// lengths N - mu add up to nearly the same everywhere), at most MO of them,
+// and walks the degrees l: the radial values R_{l,p} and their derivatives in
+// registers, then per order the sums F = sum_p R U, F' = sum_p R' U over the
+// contracted coefficients and the recurrences of the Legendre part M_l and of
+// its derivative in s.  The coefficients are the same for all lanes and come as
+// scalar operands; one vector load per 128-byte line at the start brings them
+// into the L2 cache, where the scalar loads find them.  The terms of a degree,
+// then the waves, meet in FP64.
+template <typename T, int W, int MO, int PM>
+__device__ __forceinline__ void harm_eval_body(
+    const HarmDev<T> &H, const typename HarmRecord<T>::type *atoms, uint32_t a0,
+    uint32_t na, const HarmCentre &cc, const T *U, double4 *out, double *red) {
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t N = H.N;
+  HarmAtom<T> a = {};
+  if (lane < na) a = harm_atom(H, atoms, a0 + lane, cc);
+  uint32_t mu[MO];
+  // (x + i y)^mu and ^(mu - 1); M and dM/ds of the last two degrees
+  T xc[MO], xs[MO], yc[MO], ys[MO], P1[MO], P2[MO], D1[MO], D2[MO];
+  {
+    T re = T(1), im = T(0), r1 = T(0), i1 = T(0);
+    uint32_t m = 0;
+#pragma unroll
+    for (int i = 0; i < MO; ++i) {
+      mu[i] = i * W + (i & 1 ? W - 1 - wave : wave);
+      for (; m < mu[i] && m < N; ++m) {
+        r1 = re;
+        i1 = im;
+        re = r1 * a.x - i1 * a.y;
+        im = r1 * a.y + i1 * a.x;
+      }
+      xc[i] = re;
+      xs[i] = im;
+      yc[i] = r1 * static_cast<T>(mu[i]);
+      ys[i] = i1 * static_cast<T>(mu[i]);
+      P1[i] = P2[i] = D1[i] = D2[i] = T(0);
+    }
+  }
+  double E = 0.0, A1 = 0.0, A2 = 0.0, Gz = 0.0, Hx = 0.0, Hy = 0.0;
+  HarmConst<uint32_t> *urow = harm_const(H.urow);
+  for (uint32_t l = wave; l < N; ++l) {
+    HarmConst<T> *J = harm_const(H.jac + 2 * H.crow[l]);
+    HarmConst<T> *rec = harm_const(H.rec + 128 * l);
+    const T *Ul = U + 8 * urow[l];
+    T e = T(0), f1 = T(0), f2 = T(0), gz = T(0), hx = T(0), hy = T(0);
+    const uint32_t PKl = harm_psteps(l, N);
+    harm_switch<PM>(PKl, [&](auto steps) {
+      constexpr int PK = decltype(steps)::value;
+      T R[4 * PK], Q[4 * PK];  // R_{l,p}, dR_{l,p}/dx
+      R[0] = T(1);
+      Q[0] = T(0);
+      R[1] = a.t + J[2];
+      Q[1] = T(1);
+#pragma unroll
+      for (int p = 2; p < 4 * PK; ++p) {
+        const T v = a.t + J[2 * p], c2 = J[2 * p + 1];
+        R[p] = harm_fma(v, R[p - 1], -c2 * R[p - 2]);
+        Q[p] = harm_fma(v, Q[p - 1], harm_fma(-c2, Q[p - 2], R[p - 1]));
+      }
+#pragma unroll
+      for (int i = 0; i < MO; ++i)
+        if (mu[i] <= l) {  // uniform
+          HarmConst<T> *u = harm_const(Ul + 8 * mu[i] * PK);
+          const T b = rec[2 * mu[i]], ez = rec[2 * mu[i] + 1];
+          T Fc = u[0], Fs = u[1], Gc = T(0), Gs = T(0);
+#pragma unroll
+          for (int p = 1; p < 4 * PK; ++p) {
+            Fc = harm_fma(R[p], u[2 * p], Fc);
+            Fs = harm_fma(R[p], u[2 * p + 1], Fs);
+            Gc = harm_fma(Q[p], u[2 * p], Gc);
+            Gs = harm_fma(Q[p], u[2 * p + 1], Gs);
+          }
+          const T one = mu[i] == l ? T(1) : T(0);
+          const T m = harm_fma(-(b * a.s), P2[i],
+                               harm_fma(a.z, P1[i], one));
+          const T d = harm_fma(-b, harm_fma(a.s, D2[i], P2[i]), a.z * D1[i]);
+          const T F = harm_fma(Fc, xc[i], Fs * xs[i]);
+          const T G = harm_fma(Gc, xc[i], Gs * xs[i]);
+          const T hc = harm_fma(Fc, yc[i], Fs * ys[i]);
+          const T hs = harm_fma(Fs, yc[i], -Fc * ys[i]);
+          gz = harm_fma(ez * P1[i], F, gz);
+          e = harm_fma(m, F, e);
+          f1 = harm_fma(m, G, f1);
+          f2 = harm_fma(d, F, f2);
+          hx = harm_fma(m, hc, hx);
+          hy = harm_fma(m, hs, hy);
+          P2[i] = P1[i];
+          P1[i] = m;
+          D2[i] = D1[i];
+          D1[i] = d;
+        }
+    });
+    E += static_cast<double>(e);
+    A1 += static_cast<double>(f1);
+    A2 += static_cast<double>(f2);
+    Gz += static_cast<double>(gz);
+    Hx += static_cast<double>(hx);
+    Hy += static_cast<double>(hy);
+  }
+  // s = x^2 + y^2 + z^2; the derivative of M in z is the full one
+  A1 *= H.xk;
+  double v[4] = {2.0 * (A1 + A2) * static_cast<double>(a.x) + Hx,
+                 2.0 * (A1 + A2) * static_cast<double>(a.y) + Hy,
+                 2.0 * A1 * static_cast<double>(a.z) + Gz, E};
+  // [wave][component][lane]
+#pragma unroll
+  for (int d = 0; d < 4; ++d) red[(4 * wave + d) * 64 + lane] = v[d];
+  harm_barrier();
+  if (threadIdx.x < 64 && lane < na) {
+#pragma unroll
+    for (int w = 1; w < W; ++w)
+#pragma unroll
+      for (int d = 0; d < 4; ++d) v[d] += red[(4 * w + d) * 64 + lane];
+    const double q = a.q, f = -q * H.scale;
+    out[a0 + lane] = make_double4(f * v[0], f * v[1], f * v[2], q * v[3]);
+  }
+  harm_barrier();
+}
+
+// Workgroup w: set w % nset of 64 atoms of cell w / nset, then every nset-th.
+// 400 and 1,545 us (products on the matrix cores over LDS tables of the radial
+// values: 835 and 2,764; without the first touch of the lines 497 and 2,947),
+// bound by vector instructions: 22 per (degree, order) beyond the sums, and
+// each wave forms the radial values anew.
+template <typename T, int W, int MO, int PM>
+__global__ __launch_bounds__(64 * W) void harm_eval_kernel(
+    HarmDev<T> H, const typename HarmRecord<T>::type *__restrict__ atoms,
+    const uint32_t *__restrict__ start, const double4 *__restrict__ k64,
+    uint32_t K, uint32_t ny, uint32_t nz, double h, uint32_t ncell,
+    uint32_t nset, const T *__restrict__ mom, const T *__restrict__ R,
+    const uint32_t *__restrict__ outside, double4 *__restrict__ out) {
+  __shared__ double red[W * 256];
+  const uint32_t nb = gridDim.x, b = blockIdx.x;
+  const uint32_t q = nb >> 3, r = nb & 7u, x = b & 7u;
+  const uint32_t w = x * q + (x < r ? x : r) + (b >> 3);
+  const uint32_t cell = w / nset, set = w - cell * nset;
+  const uint32_t a0 = start[cell], na = start[cell + 1] - a0;
+  const HarmCentre cc = harm_centre(cell, ny, nz, h);
+  const T *U = mom + static_cast<size_t>(cell) * H.ustride;
+  T touch[2] = {T(0), T(0)};
+  constexpr uint32_t line = 128 / sizeof(T);
+#pragma unroll
+  for (uint32_t i = 0; i < 2; ++i) {
+    const uint32_t e = (threadIdx.x + i * 64 * W) * line;
+    if (e < H.ustride) touch[i] = U[e];
+  }
+  for (uint32_t p0 = 64 * set; p0 < na; p0 += 64 * nset) {
+    const uint32_t cnt = na - p0 < 64 ? na - p0 : 64u;
+    harm_eval_body<T, W, MO, PM>(H, atoms, a0 + p0, cnt, cc, U, out, red);
+    if (outside[cell])  // uniform; the same wave stores again
+      for (uint32_t i = a0 + p0; i < a0 + p0 + cnt; ++i)
+        if (harm_atom(H, atoms, i, cc).out)
+          harm_outside_eval<T>(harm_offset(atoms, i, cc), cell, k64, K, R,
+                               harm_row(ncell), red, out + i);
+  }
+  asm volatile("" ::"v"(touch[0]), "v"(touch[1]));
+}
+
+}  // namespace
+
+// ---------------------------------------------------------------------------
+// launchers
+
+void prepare_harmonic(size_t lds_limit) {
+  const int n = static_cast<int>(lds_limit);
+  auto allow = [&](auto *k) {
+    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(k),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, n);
+  };
+  allow(harm_moments_kernel<float, 16>);
+  allow(harm_moments_kernel<double, 16>);
+  allow(harm_moments_kernel<double, 24>);
+  allow(harm_moments_kernel<double, 32>);
+  allow(harm_sf_kernel<float, 2>);
+  allow(harm_sf_kernel<float, 3>);
+  allow(harm_sf_kernel<float, 4>);
+  allow(harm_sf_kernel<double, 2>);
+  allow(harm_sf_kernel<double, 3>);
+  allow(harm_sf_kernel<double, 4>);
+  allow(harm_lr_kernel<float, 2, 8>);
+  allow(harm_lr_kernel<float, 3, 12>);
+  allow(harm_lr_kernel<float, 4, 16>);
+  allow(harm_lr_kernel<double, 1, 8>);
+  allow(harm_lr_kernel<double, 2, 12>);
+  allow(harm_lr_kernel<double, 2, 16>);
+}
+
+template <typename T>
+size_t harm_lds_moments(uint32_t N, uint32_t ksteps) {
+  const size_t prow = 4 * harm_psteps(0, N), nt = (N + 7) / 8;
+  const size_t ch = 4 * ksteps;
+  uint32_t jrows = 0;
+  for (uint32_t l = 0; l < N; ++l) jrows += 4 * harm_psteps(l, N);
+  return (6 * ch + std::max<size_t>(harm_lb<T>() * prow, 16 * nt) * (ch + 4) +
+          harm_lb<T>() * 8 * nt + 2 * jrows) * sizeof(T) + 8;
+}
+template <typename T>
+size_t harm_lds_sf(uint32_t N, uint32_t h) {
+  const size_t KS = ((N + 1) / 2 + 1) / 2;
+  return ((sizeof(T) == 4 ? 16 : 8) * (4 * KS * 16 + 8) +
+          ((h + 15) / 16) * KS * 64) *
+         sizeof(T);
+}
+template <typename T>
+size_t harm_lds_lr(uint32_t N, uint32_t h, uint32_t nring) {
+  const size_t KS = ((N + 1) / 2 + 1) / 2, MS = 4 * KS;
+  const size_t lk = std::max<size_t>(4, (nring + 3) / 4);
+  const size_t hk = (h + 3) / 4, top = hk <= 8 ? 8 : hk <= 12 ? 12 : 16;
+  return ((sizeof(T) == 4 ? 4 : 2) * lk * (MS * 16 + 8) +
+          2 * ((MS + 15) / 16) * top * 64) *
+         sizeof(T);
+}
+template size_t harm_lds_moments<float>(uint32_t, uint32_t);
+template size_t harm_lds_moments<double>(uint32_t, uint32_t);
+template size_t harm_lds_sf<float>(uint32_t, uint32_t);
+template size_t harm_lds_sf<double>(uint32_t, uint32_t);
+template size_t harm_lds_lr<float>(uint32_t, uint32_t, uint32_t);
+template size_t harm_lds_lr<double>(uint32_t, uint32_t, uint32_t);
+
+template <typename T>
+void harm_moments(const HarmPlanDev &P, const HarmDev<T> &H, const void *atoms,
+                  const uint32_t *start, const GridShape &g, T *mom, T *coef,
+                  uint32_t *outside, hipStream_t s) {
+  auto *at = static_cast<const typename HarmRecord<T>::type *>(atoms);
+  const uint32_t block = 64 * ((H.N + 7) / 8);
+  auto go = [&](auto *kernel) {
+    kernel<<<g.ncell, block, P.lds_moments, s>>>(H, at, start, g.ny, g.nz, g.h,
+                                                 mom, outside);
+  };
+  if constexpr (sizeof(T) == 4) {
+    go(harm_moments_kernel<T, 16>);
+  } else {
+    if (P.ksteps <= 16)
+      go(harm_moments_kernel<T, 16>);
+    else if (P.ksteps <= 24)
+      go(harm_moments_kernel<T, 24>);
+    else
+      go(harm_moments_kernel<T, 32>);
+  }
+  const uint32_t nw = (g.ncell + kHarmCells - 1) / kHarmCells * H.npair;
+  harm_radial_kernel<T, false>
+      <<<(nw + 3) / 4, 256, 0, s>>>(H, g.ncell, nw, mom, coef);
+}
+
+template <typename T>
+void harm_sf(const HarmPlanDev &P, const HarmDev<T> &H, const void *atoms,
+             const uint32_t *start, const double4 *k64, const GridShape &g,
+             const T *coef, const uint32_t *outside, T *S, hipStream_t s) {
+  const uint32_t nt = (g.ncell + kHarmCells - 1) / kHarmCells;
+  auto go = [&](auto *kernel) {
+    kernel<<<harm_grid(nt, P.nunit), kHarmBlock, P.lds_sf, s>>>(
+        H, P.unit, P.nunit,
+        static_cast<const typename HarmRecord<T>::type *>(atoms), start, k64,
+        g.ny, g.nz, g.h, g.ncell, coef, outside, S);
+  };
+  if (P.hsteps <= 8)
+    go(harm_sf_kernel<T, 2>);
+  else if (P.hsteps <= 12)
+    go(harm_sf_kernel<T, 3>);
+  else
+    go(harm_sf_kernel<T, 4>);
+}
+
+template <typename T>
+void harm_lr(const HarmPlanDev &P, const HarmDev<T> &H, const GridShape &g,
+             const T *R, T *coef, T *mom, hipStream_t s) {
+  const uint32_t nt = (g.ncell + kHarmCells - 1) / kHarmCells;
+  auto go = [&](auto *kernel) {
+    kernel<<<harm_grid(nt, H.nrad), kHarmBlock, P.lds_lr, s>>>(H, g.ncell, R,
+                                                               coef);
+  };
+  // rows per wave and steps of four azimuths over half a ring
+  constexpr bool F = sizeof(T) == 4;
+  if (P.hsteps <= 8)
+    go(harm_lr_kernel<T, F ? 2 : 1, 8>);
+  else if (P.hsteps <= 12)
+    go(harm_lr_kernel<T, F ? 3 : 2, 12>);
+  else
+    go(harm_lr_kernel<T, F ? 4 : 2, 16>);
+  const uint32_t nw = nt * H.npair;
+  harm_radial_kernel<T, true>
+      <<<(nw + 3) / 4, 256, 0, s>>>(H, g.ncell, nw, coef, mom);
+}
+
+template <typename T>
+void harm_eval(const HarmPlanDev &P, const HarmDev<T> &H, const void *atoms,
+               const uint32_t *start, const double4 *k64, uint32_t K,
+               const GridShape &g, const T *mom, const T *R,
+               const uint32_t *outside, double4 *out, hipStream_t s) {
+  const uint32_t ps = harm_psteps(0, H.N);
+  auto go = [&](auto waves, auto orders, auto steps) {
+    constexpr int W = decltype(waves)::value, MO = decltype(orders)::value;
+    harm_eval_kernel<T, W, MO, decltype(steps)::value>
+        <<<g.ncell * P.nset, 64 * W, 0, s>>>(
+            H, static_cast<const typename HarmRecord<T>::type *>(atoms), start,
+            k64, K, g.ny, g.nz, g.h, g.ncell, P.nset, mom, R, outside, out);
+  };
+  // W MO >= N (N <= 8 ps).  FP32: four waves of twice the orders form the
+  // radial values half as often (400 against 439 us at 3,375 cells), eight
+  // fill the device on small grids (69 against 102 us at 64 cells)
+  if (sizeof(T) == 4 && g.ncell * P.nset >= 512) {
+    harm_host_switch<5>(ps, [&](auto k) {
+      constexpr int PM = decltype(k)::value;
+      if (H.N <= 8 * PM - 4)
+        go(HarmInt<4>{}, HarmInt<2 * PM - 1>{}, k);
+      else
+        go(HarmInt<4>{}, HarmInt<2 * PM>{}, k);
+    });
+  } else {
+    harm_host_switch<sizeof(T) == 4 ? 5 : 7>(
+        ps, [&](auto k) { go(HarmInt<8>{}, k, k); });
+  }
+}
+
+#define GLST_HARM(T)                                                          \
+  template void harm_moments<T>(const HarmPlanDev &, const HarmDev<T> &,      \
+                                const void *, const uint32_t *,               \
+                                const GridShape &, T *, T *, uint32_t *,      \
+                                hipStream_t);                                 \
+  template void harm_sf<T>(const HarmPlanDev &, const HarmDev<T> &,           \
+                           const void *, const uint32_t *, const double4 *,   \
+                           const GridShape &, const T *, const uint32_t *,    \
+                           T *, hipStream_t);                                 \
+  template void harm_lr<T>(const HarmPlanDev &, const HarmDev<T> &,           \
+                           const GridShape &, const T *, T *, T *,            \
+                           hipStream_t);                                      \
+  template void harm_eval<T>(const HarmPlanDev &, const HarmDev<T> &,         \
+                             const void *, const uint32_t *, const double4 *, \
+                             uint32_t, const GridShape &, const T *,          \
+                             const T *, const uint32_t *, double4 *,          \
+                             hipStream_t);
+GLST_HARM(float)
+GLST_HARM(double)
+#undef GLST_HARM
+
+}  // namespace dev
+}  // namespace glst

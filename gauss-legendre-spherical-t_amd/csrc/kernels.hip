@@ -22,6 +22,7 @@
 //    covered floor(256/n) times by interleaved neighbour phases.
 //  * Every kernel body is a __device__ function shared by the single-system
 //    kernel and its batched twin, which looks its system up in a run table.
+#include "harmonic.hpp"
 #include "kernels.hpp"
 #include "sincos64.hpp"
 
@@ -540,10 +541,37 @@ __device__ inline float kappa_rev(const double4 &k) {
   return static_cast<float>(sqrt(k.x * k.x + k.y * k.y + k.z * k.z) * kInv2Pi);
 }
 
-// R_c(k) = W_k (cube_out - cube_in); the mixed path multiplies by
-// exp(+i k.c) = a b c (the cell's three FP64 axis factors) and stores FP32,
-// the FP64 path stores R_c(k).
-template <bool MIXED, class G>
+// V of one (node, cell) of a node-major field.
+template <bool MIXED>
+__device__ inline void store_rmt_nm(void *R, uint32_t node, uint32_t cell,
+                                    uint32_t ncp, double re, double im) {
+  if constexpr (MIXED) {
+    static_cast<float2 *>(R)[static_cast<size_t>(node) * ncp + cell] =
+        make_float2(static_cast<float>(re), static_cast<float>(im));
+  } else {
+    double *r = static_cast<double *>(R);
+    r[harm_slot<double>(node, cell, 0, ncp)] = re;
+    r[harm_slot<double>(node, cell, 1, ncp)] = im;
+  }
+}
+template <bool MIXED>
+__device__ __forceinline__ double2 load_sf_nm(const void *S, uint32_t node,
+                                              uint32_t cell, uint32_t ncp) {
+  if constexpr (MIXED) {
+    const float2 f =
+        static_cast<const float2 *>(S)[static_cast<size_t>(node) * ncp + cell];
+    return make_double2(f.x, f.y);
+  } else {
+    const double *r = static_cast<const double *>(S);
+    return make_double2(r[harm_slot<double>(node, cell, 0, ncp)],
+                        r[harm_slot<double>(node, cell, 1, ncp)]);
+  }
+}
+
+// R_c(k) = W_k (cube_out - cube_in); the mixed path and node-major fields
+// multiply by exp(+i k.c) = a b c (the cell's three FP64 axis factors), the
+// cell-major FP64 path stores R_c(k).
+template <bool MIXED, bool NM, class G>
 __device__ inline void shell_store(const G &P, uint32_t x, uint32_t y,
                                    uint32_t z, uint32_t node, const double4 &k,
                                    uint32_t rin, uint32_t rout, uint32_t nx,
@@ -553,12 +581,16 @@ __device__ inline void shell_store(const G &P, uint32_t x, uint32_t y,
   const double2 o = cube_sum(P, x, y, z, rout, nx, ny, nz);
   const double2 in = cube_sum(P, x, y, z, rin, nx, ny, nz);
   const double re = (o.x - in.x) * k.w, im = (o.y - in.y) * k.w;
-  const size_t off = static_cast<size_t>((x * ny + y) * nz + z) * Kp + node;
-  if (MIXED) {
+  const uint32_t cell = (x * ny + y) * nz + z;
+  const size_t off = static_cast<size_t>(cell) * Kp + node;
+  if (MIXED || NM) {
     const double pr = a.x * b.x - a.y * b.y, pi = a.x * b.y + a.y * b.x;
     const double cr = pr * c.x - pi * c.y, ci = pr * c.y + pi * c.x;
-    store_rmt_mixed(R, off, re * cr - im * ci, re * ci + im * cr,
-                    kappa_rev(k));
+    const double vr = re * cr - im * ci, vi = re * ci + im * cr;
+    if (NM)
+      store_rmt_nm<MIXED>(R, node, cell, harm_row(nx * ny * nz), vr, vi);
+    else
+      store_rmt_mixed(R, off, vr, vi, kappa_rev(k));
   } else {
     static_cast<double2 *>(R)[off] = make_double2(re, im);
   }
@@ -746,7 +778,7 @@ __device__ inline void rmt_border(double2 *P, const RmtGeom &g) {
 // consecutive (node, z), every thread walking y; the mixed path applies
 // w exp(+i k.c) with the node weight folded into the thread's x and z
 // factors.
-template <uint32_t BS, bool MIXED, bool ZDONE, class F>
+template <uint32_t BS, bool MIXED, bool ZDONE, bool NM, class F>
 __device__ __forceinline__ void rmt_compute(
     double2 *P, const double2 *phase, const RmtGeom &g,
     const double4 *__restrict__ k64, const uint32_t *__restrict__ group,
@@ -817,13 +849,13 @@ __device__ __forceinline__ void rmt_compute(
     const uint32_t rin = r_in[gr], rout = r_out[gr];
     const double4 kn = k64[node];
     const double w = kn.w;
-    const float kr = MIXED ? kappa_rev(kn) : 0.f;
+    const float kr = MIXED && !NM ? kappa_rev(kn) : 0.f;
     const double2 *Pt = P + t * ts;
     const CubeXZ co = cube_xz(x, z, rout, nx, nz, plane);
     const CubeXZ ci = cube_xz(x, z, rin, nx, nz, plane);
     const double2 *ph = phase + t * nax;
     double qr = 0.0, qi = 0.0;
-    if (MIXED) {  // w exp(+i k_x c_x) exp(+i k_z c_z)
+    if (MIXED || NM) {  // w exp(+i k_x c_x) exp(+i k_z c_z)
       const double2 a = ph[x], c = ph[nx + ny + z];
       qr = (a.x * c.x - a.y * c.y) * w;
       qi = (a.x * c.y + a.y * c.x) * w;
@@ -846,11 +878,16 @@ __device__ __forceinline__ void rmt_compute(
       omi += (y >= rin) ? zp : 0u;
       const double2 o = cube_sum(ko), in = cube_sum(ki);
       const double dr = o.x - in.x, di = o.y - in.y;
-      const size_t off = static_cast<size_t>((x * ny + y) * nz + z) * Kp + node;
-      if (MIXED) {
+      const uint32_t cell = (x * ny + y) * nz + z;
+      const size_t off = static_cast<size_t>(cell) * Kp + node;
+      if (MIXED || NM) {
         const double2 b = ph[nx + y];
         const double er = qr * b.x - qi * b.y, ei = qr * b.y + qi * b.x;
-        store_rmt_mixed(R, off, dr * er - di * ei, dr * ei + di * er, kr);
+        const double vr = dr * er - di * ei, vi = dr * ei + di * er;
+        if (NM)
+          store_rmt_nm<MIXED>(R, node, cell, harm_row(g.ncell), vr, vi);
+        else
+          store_rmt_mixed(R, off, vr, vi, kr);
       } else {
         static_cast<double2 *>(R)[off] = make_double2(dr * w, di * w);
       }
@@ -895,7 +932,7 @@ __device__ __forceinline__ double2 rmt_slot(const void *__restrict__ Sv,
   }
 }
 
-template <bool MIXED, uint32_t LEN>
+template <bool NM, bool MIXED, uint32_t LEN>
 __device__ __forceinline__ void rmt_line_fetch(const void *__restrict__ Sv,
                                                const RmtGeom &g,
                                                uint32_t node0, uint32_t l,
@@ -903,10 +940,21 @@ __device__ __forceinline__ void rmt_line_fetch(const void *__restrict__ Sv,
   constexpr uint32_t L = LEN, G = sf_run<MIXED>();
   const uint32_t t = l & (g.T - 1), q = l >> g.lgT;
   const size_t base = sf_slot<MIXED>(node0 + t, q * g.nz, g.ncell);
+  const uint32_t ncp = harm_row(g.ncell);
 #pragma unroll
   for (uint32_t z = 0; z < L; ++z) {
     const uint32_t zz = z < g.nz ? z : g.nz - 1;  // clamped: in the line
-    if constexpr (MIXED) {
+    if constexpr (NM) {
+      const uint32_t c = q * g.nz + zz;
+      if constexpr (MIXED) {
+        ln.v[z] = static_cast<const float2 *>(
+            Sv)[static_cast<size_t>(node0 + t) * ncp + c];
+      } else {
+        const double2 v = load_sf_nm<false>(Sv, node0 + t, c, ncp);
+        ln.re[z] = v.x;
+        ln.im[z] = v.y;
+      }
+    } else if constexpr (MIXED) {
       ln.v[z] = static_cast<const float2 *>(Sv)[base + G * zz];
     } else {
       const double2 v = static_cast<const double2 *>(Sv)[base + G * zz];
@@ -916,7 +964,7 @@ __device__ __forceinline__ void rmt_line_fetch(const void *__restrict__ Sv,
   }
 }
 
-template <bool MIXED, uint32_t LEN>
+template <bool NM, bool MIXED, uint32_t LEN>
 __device__ __forceinline__ void rmt_line_put(double2 *P,
                                              const double2 *phase,
                                              const RmtGeom &g,
@@ -928,7 +976,8 @@ __device__ __forceinline__ void rmt_line_put(double2 *P,
   const uint32_t x = fast_div(q, g.ny, g.rny), y = q - x * g.ny;
   double2 *p = P + t * g.ts + (x + 1) * g.plane + (y + 1) * g.zp + 1;
   const size_t base = sf_slot<MIXED>(node0 + t, q * g.nz, g.ncell);
-  if constexpr (MIXED) {
+  if constexpr (MIXED || NM) {
+    const uint32_t ncp = harm_row(g.ncell);
     const double2 *ph = phase + t * g.nax;
     const double2 a = ph[x], b = ph[g.nx + y];
     const double pr = a.x * b.x - a.y * b.y, pi = a.x * b.y + a.y * b.x;
@@ -944,9 +993,18 @@ __device__ __forceinline__ void rmt_line_put(double2 *P,
     };
 #pragma unroll
     for (uint32_t z = 0; z < L; ++z)
-      if (z < g.nz) step(z, make_double2(ln.v[z].x, ln.v[z].y));
-    for (uint32_t z = L; z < g.nz; ++z)
-      step(z, rmt_slot<true>(Sv, base + G * z));
+      if (z < g.nz) {
+        if constexpr (MIXED)
+          step(z, make_double2(ln.v[z].x, ln.v[z].y));
+        else
+          step(z, make_double2(ln.re[z], ln.im[z]));
+      }
+    for (uint32_t z = L; z < g.nz; ++z) {
+      if constexpr (NM)
+        step(z, load_sf_nm<MIXED>(Sv, node0 + t, q * g.nz + z, ncp));
+      else
+        step(z, rmt_slot<true>(Sv, base + G * z));
+    }
   } else {
     // past the line's end the fetch repeated its last slot, so the clamped
     // store rewrites that slot's value (a loop bounded by nz instead would
@@ -979,11 +1037,11 @@ __device__ __forceinline__ void rmt_lds_body(
   const uint32_t nline = T * nx * ny;
   for (uint32_t l = threadIdx.x; l < nline; l += kRmtBlock) {
     RmtLineB<MIXED> ln;
-    rmt_line_fetch(Sv, g, node0, l, ln);
-    rmt_line_put(P, phase, g, Sv, node0, l, ln);
+    rmt_line_fetch<false>(Sv, g, node0, l, ln);
+    rmt_line_put<false>(P, phase, g, Sv, node0, l, ln);
   }
   __syncthreads();
-  rmt_compute<kRmtBlock, MIXED, true>(P, phase, g, k64, group, r_in, r_out,
+  rmt_compute<kRmtBlock, MIXED, true, false>(P, phase, g, k64, group, r_in, r_out,
                                       Kp, node0, R, [] {});
 }
 
@@ -995,7 +1053,7 @@ __device__ __forceinline__ void rmt_lds_body(
 // a workgroup gathers one tile's shells, the next tile's z-lines are already
 // on their way into registers and its phase factors are written to the
 // second of two phase buffers.
-template <bool MIXED>
+template <bool MIXED, bool NM>
 __global__ __launch_bounds__(kRmtPBlock, GLST_RMT_MIN_WAVES) void rmt_lds_kernel(
     const void *__restrict__ Sv, const double4 *__restrict__ k64,
     const uint32_t *__restrict__ group, const uint32_t *__restrict__ r_in,
@@ -1019,7 +1077,7 @@ __global__ __launch_bounds__(kRmtPBlock, GLST_RMT_MIN_WAVES) void rmt_lds_kernel
     end = ntile;
     step = nwg;
   }
-  const uint32_t nph = MIXED ? T * g.nax : 0u;
+  const uint32_t nph = MIXED || NM ? T * g.nax : 0u;
   const uint32_t nline = T * nx * ny;
   double2 *phase0 = P + T * g.ts;
   rmt_border<kRmtPBlock>(P, g);
@@ -1028,29 +1086,29 @@ __global__ __launch_bounds__(kRmtPBlock, GLST_RMT_MIN_WAVES) void rmt_lds_kernel
     const uint32_t node0 = (tile0 + tile) * T;
     for (uint32_t e = tid; e < nph; e += kRmtPBlock)
       phase0[e] = rmt_phase(k64, g, node0, h, e);
-    if (tid < nline) rmt_line_fetch(Sv, g, node0, tid, ln);
+    if (tid < nline) rmt_line_fetch<NM>(Sv, g, node0, tid, ln);
   }
   __syncthreads();  // the first tile's phase factors
   uint32_t buf = 0;
   while (tile < end) {  // uniform over the workgroup
     const uint32_t node0 = (tile0 + tile) * T;
     const double2 *phase = phase0 + buf * nph;
-    if (tid < nline) rmt_line_put(P, phase, g, Sv, node0, tid, ln);
+    if (tid < nline) rmt_line_put<NM>(P, phase, g, Sv, node0, tid, ln);
     for (uint32_t l = tid + kRmtPBlock; l < nline; l += kRmtPBlock) {
       RmtLineP<MIXED> more;
-      rmt_line_fetch(Sv, g, node0, l, more);
-      rmt_line_put(P, phase, g, Sv, node0, l, more);
+      rmt_line_fetch<NM>(Sv, g, node0, l, more);
+      rmt_line_put<NM>(P, phase, g, Sv, node0, l, more);
     }
     __syncthreads();
     const uint32_t next = tile + step;
-    rmt_compute<kRmtPBlock, MIXED, true>(
+    rmt_compute<kRmtPBlock, MIXED, true, NM>(
         P, phase, g, k64, group, r_in, r_out, Kp, node0, R, [&] {
           if (next < end) {
             const uint32_t n1 = (tile0 + next) * T;
             double2 *ph1 = phase0 + (buf ^ 1u) * nph;
             for (uint32_t e = tid; e < nph; e += kRmtPBlock)
               ph1[e] = rmt_phase(k64, g, n1, h, e);
-            if (tid < nline) rmt_line_fetch(Sv, g, n1, tid, ln);
+            if (tid < nline) rmt_line_fetch<NM>(Sv, g, n1, tid, ln);
           }
         });
     __syncthreads();  // the tables are free, the next phases written
@@ -1101,13 +1159,16 @@ __device__ __forceinline__ void rmt_mfma_load(const float2 *__restrict__ p,
 
 // One tile of the matrix-core shell sums: nodes n0 .. n0+NPW-1 (see
 // rmt_mfma_kernel).
-template <uint32_t NPW>
+template <uint32_t NPW, bool NM>
 __device__ __forceinline__ void rmt_mfma_tile(
     const float2 *__restrict__ S, const double4 *__restrict__ k64,
     const uint32_t *__restrict__ group, const uint32_t *__restrict__ r_in,
     const uint32_t *__restrict__ r_out, uint32_t Kp, uint32_t n0,
-    uint32_t nx, uint32_t ny, uint32_t nz, double h, float2 *__restrict__ R,
+    uint32_t gx, uint32_t ny, uint32_t gz, double h, float2 *__restrict__ R,
     float2 *__restrict__ rmt_mfma_lds) {
+  // node-major fields: the x and z axes change places, so that the columns
+  // of a slice are consecutive cells of a row
+  const uint32_t nx = NM ? gz : gx, nz = NM ? gx : gz;
   const uint32_t tid = threadIdx.x;
   const uint32_t nax = nx + ny + nz, zp = rmt_zpitch(nz);
   const uint32_t nline = nx * ny, ts = nline * zp, ncell = nline * nz;
@@ -1120,11 +1181,11 @@ __device__ __forceinline__ void rmt_mfma_tile(
     const double4 k = k64[n0 + t];
     double2 r;
     if (a < nx)
-      axis_phase(&r, k.x, h, a);
+      axis_phase(&r, NM ? k.z : k.x, h, a);
     else if (a < nx + ny)
       axis_phase(&r, k.y, h, a - nx);
     else
-      axis_phase(&r, k.z, h, a - nx - ny);
+      axis_phase(&r, NM ? k.x : k.z, h, a - nx - ny);
     ph[e] = make_float2(static_cast<float>(r.x), static_cast<float>(r.y));
   }
   __syncthreads();
@@ -1139,9 +1200,42 @@ __device__ __forceinline__ void rmt_mfma_tile(
     }
   }
   __syncthreads();
-  // (1a) Y = S conj(exp(i k.c)): sixteen lanes per line, consecutive lanes
-  // on consecutive z, so a wave reads consecutive cells
-  {
+  const uint32_t ncp = harm_row(ncell);
+  if constexpr (NM) {
+    // (1a) Y = S conj(exp(i k.c)): sixteen lanes per row of x cells, so a
+    // wave reads consecutive cells; 8 loads per thread in flight at once
+    constexpr uint32_t kB = 8 / NPW, kLs = kRmtMfmaBlock / 16;
+    const float rny = 1.0f / static_cast<float>(ny);
+    const uint32_t xl = tid & 15u, nrow = ny * nz;
+    const uint32_t xc = xl < nx ? xl : nx - 1;
+    for (uint32_t lb = tid >> 4; lb < nrow; lb += kB * kLs) {
+      float2 v[kB][NPW];
+#pragma unroll
+      for (uint32_t u = 0; u < kB; ++u) {
+        const uint32_t l = lb + u * kLs < nrow ? lb + u * kLs : lb;
+#pragma unroll
+        for (uint32_t t = 0; t < NPW; ++t)
+          v[u][t] = S[static_cast<size_t>(n0 + t) * ncp + l * nx + xc];
+      }
+#pragma unroll
+      for (uint32_t u = 0; u < kB; ++u) {
+        const uint32_t l = lb + u * kLs;
+        if (l < nrow && xl < nx) {
+          const uint32_t z = fast_div(l, ny, rny), y = l - z * ny;
+#pragma unroll
+          for (uint32_t t = 0; t < NPW; ++t) {
+            const float2 e = cmulf(stage[t * nline + xl * ny + y],
+                                   ph[t * nax + nx + ny + z]);
+            tab[t * ts + (xl * ny + y) * zp + z + 1] =
+                make_float2(v[u][t].x * e.x + v[u][t].y * e.y,
+                            v[u][t].y * e.x - v[u][t].x * e.y);
+          }
+        }
+      }
+    }
+  } else {
+    // (1a) Y = S conj(exp(i k.c)): sixteen lanes per line, consecutive lanes
+    // on consecutive z, so a wave reads consecutive cells
     // batches of 8 lines per thread, all 8 loads in flight at once
     constexpr uint32_t kB = 8, kLs = kRmtMfmaBlock / 16;
     const uint32_t zl = tid & 15u;
@@ -1208,7 +1302,7 @@ __device__ __forceinline__ void rmt_mfma_tile(
     rout[t] = r_out[gr];
     const double4 kn = k64[n0 + t];
     wk[t] = static_cast<float>(kn.w);
-    kr[t] = kappa_rev(kn);
+    kr[t] = NM ? 0.f : kappa_rev(kn);
 #pragma unroll
     for (uint32_t m = 0; m < 4; ++m) {
       const int dx = static_cast<int>(c) - static_cast<int>(4 * m + g4);
@@ -1283,9 +1377,29 @@ __device__ __forceinline__ void rmt_mfma_tile(
         const float dr = wor[v] - wir[v], di = woi[v] - wii[v];
         const float2 e = cmulf(e0, pt[nx + yo]);
         const float vr = dr * e.x - di * e.y, vi = dr * e.y + di * e.x;
-        const float mag = __builtin_amdgcn_sqrtf(fmaf(vr, vr, vi * vi));
-        val[t][v] = make_float2(kr[t] * mag, arg_rev(vr, vi));
+        if constexpr (NM) {
+          val[t][v] = make_float2(vr, vi);
+        } else {
+          const float mag = __builtin_amdgcn_sqrtf(fmaf(vr, vr, vi * vi));
+          val[t][v] = make_float2(kr[t] * mag, arg_rev(vr, vi));
+        }
       }
+    }
+    if constexpr (NM) {
+      // sixteen lanes store consecutive cells of a row
+      if (c < nx) {
+#pragma unroll
+        for (uint32_t v = 0; v < 4; ++v) {
+          const uint32_t yo = 4 * g4 + v;
+          if (yo < ny) {
+#pragma unroll
+            for (uint32_t t = 0; t < NPW; ++t)
+              R[static_cast<size_t>(n0 + t) * ncp + (z * ny + yo) * nx + c] =
+                  val[t][v];
+          }
+        }
+      }
+      continue;
     }
     // each cell's NPW consecutive nodes with one store
     if (c < nx) {
@@ -1323,7 +1437,7 @@ __device__ __forceinline__ void rmt_mfma_tile(
 // rounds, ran 0.68 ms alone at 288k atoms against 0.72 ms, but the tuned
 // step, where S(k) and the back-projection share the CUs, took 4.77 ms
 // against 4.72.)
-template <uint32_t NPW>
+template <uint32_t NPW, bool NM>
 __global__ __launch_bounds__(kRmtMfmaBlock) void rmt_mfma_kernel(
     const float2 *__restrict__ S, const double4 *__restrict__ k64,
     const uint32_t *__restrict__ group, const uint32_t *__restrict__ r_in,
@@ -1339,7 +1453,7 @@ __global__ __launch_bounds__(kRmtMfmaBlock) void rmt_mfma_kernel(
     const uint32_t x = blockIdx.x & 7u, q = ntile >> 3, r = ntile & 7u;
     tile = x * q + (x < r ? x : r) + (blockIdx.x >> 3);
   }
-  rmt_mfma_tile<NPW>(S, k64, group, r_in, r_out, Kp, (tile0 + tile) * NPW, nx,
+  rmt_mfma_tile<NPW, NM>(S, k64, group, r_in, r_out, Kp, (tile0 + tile) * NPW, nx,
                      ny, nz, h, R, rmt_mfma_lds);
 }
 
@@ -1405,6 +1519,7 @@ __device__ __forceinline__ void rmt_prefix8(float2 (&v)[8]) {
 // run (four adjacent slots of a cell) and each R store (cell-major, the
 // nodes of a cell adjacent) is one contiguous segment, and the window
 // tables, [cell][M] in LDS, are read and written without bank conflicts.
+template <bool NM>
 __device__ __forceinline__ void rmt_wave_tile(
     const float2 *__restrict__ S, const double4 *__restrict__ k64,
     const uint32_t *__restrict__ group, const uint32_t *__restrict__ r_in,
@@ -1471,8 +1586,11 @@ __device__ __forceinline__ void rmt_wave_tile(
     const uint32_t nf =
         n0 + (s + j < kRmtWaveNodes ? s + j : kRmtWaveNodes - 1);
 #pragma unroll
-    for (uint32_t z = 0; z < 8; ++z)
-      sv[z] = S[sf_slot<true>(nf, qf * nz + (z < nz ? z : nz - 1), ncell)];
+    for (uint32_t z = 0; z < 8; ++z) {
+      const uint32_t c = qf * nz + (z < nz ? z : nz - 1);
+      sv[z] = S[NM ? static_cast<size_t>(nf) * harm_row(ncell) + c
+                   : sf_slot<true>(nf, c, ncell)];
+    }
   };
   fetch(0);
   __syncthreads();  // the axis factors and node parameters
@@ -1563,9 +1681,15 @@ __device__ __forceinline__ void rmt_wave_tile(
           const float dr = co[y].x - ci[y].x, di = co[y].y - ci[y].y;
           const float2 e = cmulf(e0, pt[nx + y]);
           const float vr = dr * e.x - di * e.y, vi2 = dr * e.y + di * e.x;
-          const float mag = __builtin_amdgcn_sqrtf(fmaf(vr, vr, vi2 * vi2));
-          R[static_cast<size_t>((x * ny + y) * nz + z) * Kp + nd] =
-              make_float2(kr * mag, arg_rev(vr, vi2));
+          const uint32_t c = (x * ny + y) * nz + z;
+          if constexpr (NM) {
+            R[static_cast<size_t>(nd) * harm_row(ncell) + c] =
+                make_float2(vr, vi2);
+          } else {
+            const float mag = __builtin_amdgcn_sqrtf(fmaf(vr, vr, vi2 * vi2));
+            R[static_cast<size_t>(c) * Kp + nd] =
+                make_float2(kr * mag, arg_rev(vr, vi2));
+          }
         }
     }
     rmt_lds_barrier();  // the windows are free for the next nodes
@@ -1583,6 +1707,7 @@ __device__ __forceinline__ void rmt_wave_tile(
 #ifndef GLST_RMT_WAVE_MIN_WG
 #define GLST_RMT_WAVE_MIN_WG 1
 #endif
+template <bool NM>
 __global__ __launch_bounds__(kRmtWaveBlock, GLST_RMT_WAVE_MIN_WG) void rmt_wave_kernel(
     const float2 *__restrict__ S, const double4 *__restrict__ k64,
     const uint32_t *__restrict__ group, const uint32_t *__restrict__ r_in,
@@ -1594,7 +1719,7 @@ __global__ __launch_bounds__(kRmtWaveBlock, GLST_RMT_WAVE_MIN_WG) void rmt_wave_
     const uint32_t x = blockIdx.x & 7u, q = ntile >> 3, r = ntile & 7u;
     tile = x * q + (x < r ? x : r) + (blockIdx.x >> 3);
   }
-  rmt_wave_tile(S, k64, group, r_in, r_out, Kp,
+  rmt_wave_tile<NM>(S, k64, group, r_in, r_out, Kp,
                 (tile0 + tile) * kRmtWaveNodes, nx, ny, nz, h, R);
 }
 
@@ -1604,7 +1729,7 @@ __global__ __launch_bounds__(kRmtWaveBlock, GLST_RMT_WAVE_MIN_WG) void rmt_wave_
 // the mixed path applies exp(-i k.c) to the cell-local sums and takes the
 // running sum along z (the FP64 slots hold z-running sums already).  One
 // thread per (node, z-column).
-template <bool MIXED>
+template <bool MIXED, bool NM>
 __global__ void rmt_global_load_kernel(const void *__restrict__ Sv,
                                        const double4 *__restrict__ k64,
                                        double2 *__restrict__ G, uint32_t Kp,
@@ -1614,7 +1739,7 @@ __global__ void rmt_global_load_kernel(const void *__restrict__ Sv,
   const uint32_t col = col0 + blockIdx.y;
   if (node >= Kp || col >= nx * ny) return;
   const uint32_t ncell = nx * ny * nz;
-  if (!MIXED) {
+  if (!MIXED && !NM) {
     for (uint32_t z = 0; z < nz; ++z) {
       const uint32_t cell = col * nz + z;
       G[static_cast<size_t>(cell) * Kp + node] =
@@ -1634,7 +1759,9 @@ __global__ void rmt_global_load_kernel(const void *__restrict__ Sv,
     double2 c;
     axis_phase(&c, k.z, h, z);
     const double er = pr * c.x - pi * c.y, ei = pr * c.y + pi * c.x;
-    const float2 v = static_cast<const float2 *>(Sv)[sf_slot<true>(node, cell, ncell)];
+    const double2 v =
+        NM ? load_sf_nm<MIXED>(Sv, node, cell, harm_row(ncell))
+           : rmt_slot<true>(Sv, sf_slot<true>(node, cell, ncell));
     run.x += v.x * er + v.y * ei;
     run.y += v.y * er - v.x * ei;
     G[static_cast<size_t>(cell) * Kp + node] = run;
@@ -1659,7 +1786,7 @@ __global__ void prefix_axis_kernel(double2 *__restrict__ S, uint32_t Kp,
   }
 }
 
-template <bool MIXED>
+template <bool MIXED, bool NM>
 __global__ void rmt_gather_kernel(const double2 *__restrict__ P,
                                   const double4 *__restrict__ k64,
                                   const uint32_t *__restrict__ group,
@@ -1675,13 +1802,13 @@ __global__ void rmt_gather_kernel(const double2 *__restrict__ P,
   const double4 k = k64[node];
   const uint32_t x = cell / (ny * nz), y = (cell / nz) % ny, z = cell % nz;
   double2 a = make_double2(1.0, 0.0), b = a, c = a;
-  if (MIXED) {
+  if (MIXED || NM) {
     axis_phase(&a, k.x, h, x);
     axis_phase(&b, k.y, h, y);
     axis_phase(&c, k.z, h, z);
   }
   GlobalGrid grid{P, Kp, node};
-  shell_store<MIXED>(grid, x, y, z, node, k, r_in[g], r_out[g], nx, ny, nz,
+  shell_store<MIXED, NM>(grid, x, y, z, node, k, r_in[g], r_out[g], nx, ny, nz,
                      a, b, c, Kp, R);
 }
 
@@ -3059,7 +3186,7 @@ __global__ __launch_bounds__(kRmtWaveBlock, GLST_RMT_WAVE_MIN_WG) void rmt_wave_
   const uint32_t blk = xcd_remap(blockIdx.x, gridDim.x);
   const Seg g = seg[run_of(seg, nseg, blk)];
   const SysDev &d = sys[g.sys];
-  rmt_wave_tile(S + d.field0, k64 + d.node0, group + d.node0,
+  rmt_wave_tile<false>(S + d.field0, k64 + d.node0, group + d.node0,
                 r_in + d.group0, r_out + d.group0, d.Kp,
                 (blk - g.blk0) * kRmtWaveNodes, d.nx, d.ny, d.nz, d.h,
                 R + d.field0);
@@ -3407,15 +3534,15 @@ void prepare_kernels(size_t lds_limit) {
   }
   (void)hipGetLastError();
   const int lds = static_cast<int>(lds_limit);
-  const void *fns[] = {reinterpret_cast<const void *>(&rmt_lds_kernel<true>),
-                       reinterpret_cast<const void *>(&rmt_lds_kernel<false>),
-                       reinterpret_cast<const void *>(&rmt_lds_batch_kernel<true>),
-                       reinterpret_cast<const void *>(&rmt_lds_batch_kernel<false>),
-                       reinterpret_cast<const void *>(&step_fused_kernel<2>),
-                       reinterpret_cast<const void *>(&step_fused_kernel<3>),
-                       reinterpret_cast<const void *>(&rmt_mfma_kernel<1>),
-                       reinterpret_cast<const void *>(&rmt_mfma_kernel<2>),
-                       reinterpret_cast<const void *>(&rmt_mfma_kernel<4>)};
+  auto fn = [](auto *k) { return reinterpret_cast<const void *>(k); };
+  const void *fns[] = {
+      fn(rmt_lds_kernel<true, false>), fn(rmt_lds_kernel<false, false>),
+      fn(rmt_lds_kernel<true, true>),  fn(rmt_lds_kernel<false, true>),
+      fn(rmt_lds_batch_kernel<true>),  fn(rmt_lds_batch_kernel<false>),
+      fn(step_fused_kernel<2>),        fn(step_fused_kernel<3>),
+      fn(rmt_mfma_kernel<1, false>),   fn(rmt_mfma_kernel<2, false>),
+      fn(rmt_mfma_kernel<4, false>),   fn(rmt_mfma_kernel<1, true>),
+      fn(rmt_mfma_kernel<2, true>),    fn(rmt_mfma_kernel<4, true>)};
   for (const void *f : fns) {
     const hipError_t e = hipFuncSetAttribute(
         f, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
@@ -3423,6 +3550,8 @@ void prepare_kernels(size_t lds_limit) {
       (void)hipGetLastError();
     }
   }
+  prepare_harmonic(lds_limit);
+  (void)hipGetLastError();
 }
 
 void fill_u32(uint32_t *p, uint32_t value, size_t n, hipStream_t s) {
@@ -3525,7 +3654,7 @@ bool rmt_lds(bool mixed, uint32_t tmax, const void *S, const double4 *k64,
              const uint32_t *group, const uint32_t *r_in,
              const uint32_t *r_out, uint32_t Kp, const GridShape &g,
              size_t lds_limit, void *R, hipStream_t s, uint32_t tile0,
-             uint32_t tile1) {
+             uint32_t tile1, bool nm) {
   const uint32_t T = rmt_nodes_per_group(g.nx, g.ny, g.nz, lds_limit, tmax);
   if (T == 0) return false;
   const uint32_t all = Kp / T;  // Kp is a multiple of 256
@@ -3540,15 +3669,15 @@ bool rmt_lds(bool mixed, uint32_t tmax, const void *S, const double4 *k64,
   per_cu = per_cu < 1 ? 1 : (per_cu > wave_cap ? wave_cap : per_cu);
   const uint32_t nwg = static_cast<uint32_t>(
       std::min<size_t>(ntile, static_cast<size_t>(g_cu_count) * per_cu));
-  if (mixed) {
-    rmt_lds_kernel<true><<<nwg, kRmtPBlock, lds, s>>>(
-        S, k64, group, r_in, r_out, Kp, T, tile0, ntile, g.nx, g.ny, g.nz,
-        g.h, R);
-  } else {
-    rmt_lds_kernel<false><<<nwg, kRmtPBlock, lds, s>>>(
-        S, k64, group, r_in, r_out, Kp, T, tile0, ntile, g.nx, g.ny, g.nz,
-        g.h, R);
-  }
+  auto go = [&](auto *kernel) {
+    kernel<<<nwg, kRmtPBlock, lds, s>>>(S, k64, group, r_in, r_out, Kp, T,
+                                        tile0, ntile, g.nx, g.ny, g.nz, g.h,
+                                        R);
+  };
+  if (mixed)
+    go(nm ? rmt_lds_kernel<true, true> : rmt_lds_kernel<true, false>);
+  else
+    go(nm ? rmt_lds_kernel<false, true> : rmt_lds_kernel<false, false>);
   return true;
 }
 
@@ -3557,51 +3686,54 @@ bool rmt_lds(bool mixed, uint32_t tmax, const void *S, const double4 *k64,
 #ifndef GLST_RMT_MFMA_NPW
 #define GLST_RMT_MFMA_NPW 2
 #endif
-uint32_t rmt_mfma_nodes(const GridShape &g, size_t lds_limit) {
+uint32_t rmt_mfma_nodes(const GridShape &g, size_t lds_limit, bool nm) {
   if (g.nx > kRmtMfmaMaxXY || g.ny > kRmtMfmaMaxXY || g.ncell == 0) return 0;
+  if (nm && g.nz > kRmtMfmaMaxXY) return 0;
+  const uint32_t a = nm ? g.nz : g.nx, c = nm ? g.nx : g.nz;
   for (uint32_t npw = GLST_RMT_MFMA_NPW; npw >= 1; npw >>= 1)
-    if (rmt_mfma_lds_bytes(g.nx, g.ny, g.nz, npw) <= lds_limit) return npw;
+    if (rmt_mfma_lds_bytes(a, g.ny, c, npw) <= lds_limit) return npw;
   return 0;
 }
 
 bool rmt_mfma(const void *S, const double4 *k64, const uint32_t *group,
               const uint32_t *r_in, const uint32_t *r_out, uint32_t Kp,
               const GridShape &g, size_t lds_limit, void *R, hipStream_t s,
-              uint32_t tile0, uint32_t tile1) {
-  const uint32_t npw = rmt_mfma_nodes(g, lds_limit);
+              uint32_t tile0, uint32_t tile1, bool nm) {
+  const uint32_t npw = rmt_mfma_nodes(g, lds_limit, nm);
   if (npw == 0) return false;
   const uint32_t all = Kp / npw;  // Kp is a multiple of 256
   if (tile1 > all) tile1 = all;
   if (tile0 >= tile1) return true;
   const uint32_t ntile = tile1 - tile0;
-  const size_t lds = rmt_mfma_lds_bytes(g.nx, g.ny, g.nz, npw);
+  const size_t lds = nm ? rmt_mfma_lds_bytes(g.nz, g.ny, g.nx, npw)
+                        : rmt_mfma_lds_bytes(g.nx, g.ny, g.nz, npw);
   const float2 *Sf = static_cast<const float2 *>(S);
   float2 *Rf = static_cast<float2 *>(R);
+  auto go = [&](auto *kernel) {
+    kernel<<<ntile, kRmtMfmaBlock, lds, s>>>(Sf, k64, group, r_in, r_out, Kp,
+                                             tile0, ntile, g.nx, g.ny, g.nz,
+                                             g.h, Rf);
+  };
   if (npw == 4)
-    rmt_mfma_kernel<4><<<ntile, kRmtMfmaBlock, lds, s>>>(
-        Sf, k64, group, r_in, r_out, Kp, tile0, ntile, g.nx, g.ny, g.nz, g.h,
-        Rf);
+    go(nm ? rmt_mfma_kernel<4, true> : rmt_mfma_kernel<4, false>);
   else if (npw == 2)
-    rmt_mfma_kernel<2><<<ntile, kRmtMfmaBlock, lds, s>>>(
-        Sf, k64, group, r_in, r_out, Kp, tile0, ntile, g.nx, g.ny, g.nz, g.h,
-        Rf);
+    go(nm ? rmt_mfma_kernel<2, true> : rmt_mfma_kernel<2, false>);
   else
-    rmt_mfma_kernel<1><<<ntile, kRmtMfmaBlock, lds, s>>>(
-        Sf, k64, group, r_in, r_out, Kp, tile0, ntile, g.nx, g.ny, g.nz, g.h,
-        Rf);
+    go(nm ? rmt_mfma_kernel<1, true> : rmt_mfma_kernel<1, false>);
   return true;
 }
 
 bool rmt_wave(const void *S, const double4 *k64, const uint32_t *group,
               const uint32_t *r_in, const uint32_t *r_out, uint32_t Kp,
               const GridShape &g, void *R, hipStream_t s, uint32_t tile0,
-              uint32_t tile1) {
+              uint32_t tile1, bool nm) {
   if (!rmt_wave_fits(g)) return false;
   const uint32_t all = Kp / kRmtWaveNodes;  // Kp is a multiple of 256
   if (tile1 > all) tile1 = all;
   if (tile0 >= tile1) return true;
   const uint32_t ntile = tile1 - tile0;
-  rmt_wave_kernel<<<ntile, kRmtWaveBlock, 0, s>>>(
+  auto *kernel = nm ? rmt_wave_kernel<true> : rmt_wave_kernel<false>;
+  kernel<<<ntile, kRmtWaveBlock, 0, s>>>(
       static_cast<const float2 *>(S), k64, group, r_in, r_out, Kp, tile0,
       ntile, g.nx, g.ny, g.nz, g.h, static_cast<float2 *>(R));
   return true;
@@ -3610,18 +3742,18 @@ bool rmt_wave(const void *S, const double4 *k64, const uint32_t *group,
 void rmt_global(bool mixed, const void *S, double2 *G, const double4 *k64,
                 const uint32_t *group, const uint32_t *r_in,
                 const uint32_t *r_out, uint32_t Kp, const GridShape &g,
-                void *R, hipStream_t s) {
+                void *R, hipStream_t s, bool nm) {
   const uint32_t bx = blocks_for(Kp, 256);
   constexpr uint32_t kMaxY = 65535;  // grid.y limit
   const uint32_t ncol = g.nx * g.ny;
   for (uint32_t c0 = 0; c0 < ncol; c0 += kMaxY) {
     const uint32_t cnt = (ncol - c0 < kMaxY) ? ncol - c0 : kMaxY;
-    if (mixed)
-      rmt_global_load_kernel<true><<<dim3(bx, cnt), 256, 0, s>>>(
-          S, k64, G, Kp, c0, g.nx, g.ny, g.nz, g.h);
-    else
-      rmt_global_load_kernel<false><<<dim3(bx, cnt), 256, 0, s>>>(
-          S, k64, G, Kp, c0, g.nx, g.ny, g.nz, g.h);
+    auto *load = mixed ? (nm ? rmt_global_load_kernel<true, true>
+                             : rmt_global_load_kernel<true, false>)
+                       : (nm ? rmt_global_load_kernel<false, true>
+                             : rmt_global_load_kernel<false, false>);
+    load<<<dim3(bx, cnt), 256, 0, s>>>(S, k64, G, Kp, c0, g.nx, g.ny, g.nz,
+                                       g.h);
   }
   auto prefix = [&](uint32_t nlines, uint32_t n, uint32_t stride,
                     uint32_t inner) {
@@ -3635,12 +3767,12 @@ void rmt_global(bool mixed, const void *S, double2 *G, const double4 *k64,
   prefix(g.ny * g.nz, g.nx, g.ny * g.nz, g.ny * g.nz);  // x lines
   for (uint32_t c0 = 0; c0 < g.ncell; c0 += kMaxY) {
     const uint32_t cnt = (g.ncell - c0 < kMaxY) ? g.ncell - c0 : kMaxY;
-    if (mixed)
-      rmt_gather_kernel<true><<<dim3(bx, cnt), 256, 0, s>>>(
-          G, k64, group, r_in, r_out, Kp, c0, g.nx, g.ny, g.nz, g.h, R);
-    else
-      rmt_gather_kernel<false><<<dim3(bx, cnt), 256, 0, s>>>(
-          G, k64, group, r_in, r_out, Kp, c0, g.nx, g.ny, g.nz, g.h, R);
+    auto *gather = mixed ? (nm ? rmt_gather_kernel<true, true>
+                               : rmt_gather_kernel<true, false>)
+                         : (nm ? rmt_gather_kernel<false, true>
+                               : rmt_gather_kernel<false, false>);
+    gather<<<dim3(bx, cnt), 256, 0, s>>>(G, k64, group, r_in, r_out, Kp, c0,
+                                         g.nx, g.ny, g.nz, g.h, R);
   }
 }
 

@@ -87,6 +87,19 @@ __host__ __device__ inline size_t sf_slot(uint32_t node, uint32_t cell,
   return (static_cast<size_t>(node / G) * ncell + cell) * G + node % G;
 }
 
+// Node-major fields (the harmonic far field, harmonic.hpp): a row of harm_row
+// cells per node (whole 128-byte lines); mixed: (re, im) pairs, FP64: the row
+// of real parts, then the row of imaginary parts.
+__host__ __device__ inline uint32_t harm_row(uint32_t ncell) {
+  return (ncell + 15u) / 16u * 16u;
+}
+// Offset of (node, cell, part 0 re / 1 im) in a node-major field of T.
+template <typename T>
+__host__ __device__ inline size_t harm_slot(size_t node, uint32_t cell,
+                                            uint32_t part, uint32_t ncp) {
+  return sizeof(T) == 4 ? (node * ncp + cell) * 2 + part
+                        : (node * 2 + part) * ncp + cell;
+}
 // Mixed structure factors: one wave per (cell, 64 directions of a group), the
 // NR radial nodes of a direction unrolled for NR <= kSfMaxUnrolled (larger
 // counts run a generic kernel); each lane stores its direction's NR slots.
@@ -141,6 +154,9 @@ inline void sf(bool mixed, const void *atoms, const uint32_t *start,
 }
 
 // ---- remote (shell) sums (sum_rmt_sf) --------------------------------------
+// nm: S and R are node-major fields (harm_slot), S the cell-local sums and
+// R = V = W exp(+i k.c) (shell sums) in Cartesian form, for either type.
+// Otherwise S is in node runs and R cell-major (mixed: polar form).
 // LDS layout of the shell-sum workgroups.  A workgroup holds the summed-
 // volume tables of T nodes (T = 1 or a power of two), T tables of
 // rmt_table_stride elements (double2) plus two buffers of T * (nx+ny+nz)
@@ -195,7 +211,7 @@ bool rmt_lds(bool mixed, uint32_t tmax, const void *S, const double4 *k64,
              const uint32_t *group, const uint32_t *r_in,
              const uint32_t *r_out, uint32_t Kp, const GridShape &g,
              size_t lds_limit, void *R, hipStream_t s, uint32_t tile0 = 0,
-             uint32_t tile1 = 0xffffffffu);
+             uint32_t tile1 = 0xffffffffu, bool nm = false);
 // Shell sums on the matrix cores (CT = float, nx and ny up to 16):
 // workgroups of kRmtMfmaBlock threads take tiles of NPW consecutive nodes
 // and hold NPW z-running-sum tables of nx * ny * rmt_zpitch(nz) float2, the
@@ -208,14 +224,17 @@ inline size_t rmt_mfma_lds_bytes(uint32_t nx, uint32_t ny, uint32_t nz,
   return npw * (nline * (rmt_zpitch(nz) + 1) + nx + ny + nz) * 8;
 }
 // Nodes per workgroup tile of the matrix-core shell sums on this grid (0:
-// the grid is too wide for them, or one node's table does not fit).
-uint32_t rmt_mfma_nodes(const GridShape &g, size_t lds_limit);
+// the grid is too wide for them, or one node's table does not fit).  On
+// node-major fields the slices are (z, y) planes, so that a slice's cells are
+// consecutive in the rows, and nz is limited as well.
+uint32_t rmt_mfma_nodes(const GridShape &g, size_t lds_limit, bool nm = false);
 // Tiles [tile0, tile1) of rmt_mfma_nodes() nodes (tile1 clamped to
 // Kp / nodes).  False: the grid is not supported (nothing launched).
 bool rmt_mfma(const void *S, const double4 *k64, const uint32_t *group,
               const uint32_t *r_in, const uint32_t *r_out, uint32_t Kp,
               const GridShape &g, size_t lds_limit, void *R, hipStream_t s,
-              uint32_t tile0 = 0, uint32_t tile1 = 0xffffffffu);
+              uint32_t tile0 = 0, uint32_t tile1 = 0xffffffffu,
+              bool nm = false);
 // Shell sums of small grids (CT = float, every dimension up to
 // kRmtWaveMaxDim): workgroups of kRmtWaveBlock threads take tiles of
 // kRmtWaveNodes consecutive nodes, up to 16 at a time, and sum them as
@@ -233,14 +252,14 @@ inline bool rmt_wave_fits(const GridShape &g) {
 bool rmt_wave(const void *S, const double4 *k64, const uint32_t *group,
               const uint32_t *r_in, const uint32_t *r_out, uint32_t Kp,
               const GridShape &g, void *R, hipStream_t s, uint32_t tile0 = 0,
-              uint32_t tile1 = 0xffffffffu);
+              uint32_t tile1 = 0xffffffffu, bool nm = false);
 // Global-memory tables: G (ncell*Kp double2, scratch) receives S in FP64
 // cell-major order, is prefix-summed in place, and the shells are gathered
 // from it.  S is left unchanged.
 void rmt_global(bool mixed, const void *S, double2 *G, const double4 *k64,
                 const uint32_t *group, const uint32_t *r_in,
                 const uint32_t *r_out, uint32_t Kp, const GridShape &g,
-                void *R, hipStream_t s);
+                void *R, hipStream_t s, bool nm = false);
 
 // ---- long-range back-projection (calc_lr_ef) -------------------------------
 // Task table of the direction-major node order: task t covers nodes

@@ -175,7 +175,15 @@ glst_status_t glst_get_sf(glst_handle_t h, double *re, double *im);
  * keeps them on the device in polar form; they are converted back here. */
 glst_status_t glst_get_rmt(glst_handle_t h, double *re, double *im);
 
-/* Tuning options of a handle:
+/* The far field (either CT) runs through an expansion of each cell in
+ * spherical harmonics on systems of at least 2e8 (CT = float) or 3e8
+ * (CT = double) (atom, node) pairs with the product rule, where the kernels
+ * hold its degrees (phases to about 20 and 28 radians) and "sf_cheb" and
+ * "lr_atom_groups" are 1 and "rmt_shape" is not 2; otherwise through direct
+ * sums over atoms and nodes.  The two agree to the rounding of CT.  With it,
+ * "lr_blocks" and "pipeline" have no effect.
+ *
+ * Tuning options of a handle:
  *   "overlap_near" (default 1): calc_ener_force runs the near field on a
  *   second stream of the handle, started with the structure factors (1) or
  *   after them, overlapping the shell sums and the back-projection (2); 0
