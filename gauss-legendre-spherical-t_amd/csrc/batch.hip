@@ -20,6 +20,7 @@ std::shared_ptr<const ShapeSetup> make_shape_setup(int ct, const double box[3],
                                                    double rcut, double tol) {
   auto p = std::make_shared<ShapeSetup>();
   p->su = setup_system(ct, box[0], box[1], box[2], rcut, tol);
+  p->ct = ct;
   if (p->su.has_lr && p->su.K > 0) {
     p->nl = layout_nodes(p->su.nodes, p->su.K, p->su.Kp);
     if (ct == GLST_CT_FLOAT) {
@@ -36,11 +37,12 @@ std::shared_ptr<const ShapeSetup> make_shape_setup(int ct, const double box[3],
 }
 
 std::shared_ptr<const BatchSystem> make_batch_system(
-    uint32_t natom, std::shared_ptr<const ShapeSetup> shape) {
+    uint32_t natom, std::shared_ptr<const ShapeSetup> shape, bool direct) {
   if (natom == 0) throw ArgError("a system without atoms");
   auto b = std::make_shared<BatchSystem>();
   b->natom = natom;
   b->shape = std::move(shape);
+  b->direct = direct;
   return b;
 }
 
@@ -56,10 +58,14 @@ size_t BatchLayout::device_bytes() const {
   b += table_bytes + t_split.size() * 4;
   b += field * (mixed() ? 8 : 16) * 2;  // S and R
   b += partial * sizeof(double4);
-  b += sys.size() * sizeof(dev::SysDev);
+  b += (sys.size() + sys_harm.size()) * sizeof(dev::SysDev);
+  b += std::min<size_t>(harm.size(), kHarmSlots) *
+           (harm_coef + harm_mom + harm_out) +
+       harm_bytes;
   size_t nseg = bin.seg.size() + hist_p.seg.size() + scatter.seg.size() +
                 sr.seg.size() + reduce.seg.size() + rmt.seg.size() +
                 rmt_small.seg.size() + rmt_rest.seg.size() +
+                rmt_small_direct.seg.size() + rmt_rest_direct.seg.size() +
                 sf_f64.seg.size() + lr_f64.seg.size();
   for (auto &kv : sf_nr) nseg += kv.second.seg.size();
   for (auto &kv : lr_nr) nseg += kv.second.seg.size();
@@ -181,7 +187,14 @@ void ShapeTables::upload(hipStream_t s) {
   GLST_HIP(hipStreamSynchronize(s));
 }
 
+const HarmDevice &ShapeTables::harm_device(const ShapeSetup &shape) {
+  HarmDevice &d = harm[&shape];
+  if (!d.ok()) d.upload(shape.harm(), shape.ct == GLST_CT_FLOAT);
+  return d;
+}
+
 void ShapeTables::clear() {
+  harm.clear();
   for (auto *v : {&group, &r_in, &r_out, &t_node0, &t_nr, &t_koff, &t_coff})
     v->clear();
   cheb.clear();
@@ -208,6 +221,7 @@ size_t ShapeTables::device_bytes() const {
                                 &d_nr, &d_koff, &d_dir64, &d_dir32, &d_kap64,
                                 &d_kap32, &d_coff, &d_cheb})
     b += d->bytes();
+  for (const auto &kv : harm) b += kv.second.device_bytes();
   return b;
 }
 
@@ -238,7 +252,7 @@ BatchLayout pack_batch(int ct,
   std::vector<SplitPlan> splits(nsys);
   std::vector<uint32_t> task_first(nsys, 0);
   uint32_t split_base = 0;
-  std::map<const ShapeSetup *, bool> seen;
+  std::map<const ShapeSetup *, bool> seen, expanded;
   for (uint32_t s = 0; s < nsys; ++s) {
     const SystemSetup &u = cs[s]->su();
     const uint32_t na = cs[s]->natom;
@@ -272,6 +286,24 @@ BatchLayout pack_batch(int ct,
     d.partial0 = B.partial;
     d.ag0 = static_cast<uint32_t>(B.nag);
     d.agtile = 0;
+    // expanded far field: the rule of a handle (harm_worth)
+    HarmSystem hs{s, 0, {}};
+    if (cheb && lr && !cs[s]->direct &&
+        harm_worth(na, u.K, ct == GLST_CT_FLOAT)) {
+      const HarmTables &t = cs[s]->shape->harm();
+      if (t.ok)
+        hs.plan = harm_fit(t, ct == GLST_CT_FLOAT, lds_limit, na, d.ncell);
+      if (hs.plan.nrad) {
+        const size_t real = ct == GLST_CT_FLOAT ? 4 : 8;
+        B.harm_coef = std::max(B.harm_coef, harm_coef_len(t, d.ncell) * real);
+        B.harm_mom = std::max(B.harm_mom, harm_mom_len(t, d.ncell) * real);
+        B.harm_out = std::max<size_t>(B.harm_out, size_t{4} * d.ncell);
+        if (!expanded[cs[s]->shape.get()]) B.harm_bytes += t.bytes(real);
+        expanded[cs[s]->shape.get()] = true;
+        B.harm.push_back(hs);
+      }
+    }
+    const bool harm = hs.plan.nrad > 0;
     B.natom += na;
     B.ncell += u.grid.ncell;
     B.hist += static_cast<uint64_t>(d.nchunk) * u.grid.ncell;
@@ -303,7 +335,9 @@ BatchLayout pack_batch(int ct,
       // the end of its task range
       for (uint32_t q = 0; q <= P.nsplit; ++q)
         B.t_split.push_back(off.task0 + P.split[q]);
-      B.field += static_cast<uint64_t>(u.grid.ncell) * u.Kp;
+      B.field += static_cast<uint64_t>(
+                     harm ? dev::harm_row(u.grid.ncell) : u.grid.ncell) *
+                 u.Kp;
       B.partial += static_cast<uint64_t>(P.nsplit) * na;
       split_base += P.nsplit + 1;
       if (ct == GLST_CT_FLOAT) {  // back-projection over atom groups
@@ -317,6 +351,26 @@ BatchLayout pack_batch(int ct,
     B.sys.push_back(d);
   }
   if (B.t_split.empty()) B.t_split.push_back(0);
+  // the longest first, each to the slot with the least work
+  auto work = [&](const HarmSystem &h) {
+    return static_cast<double>(cs[h.sys]->natom) * cs[h.sys]->su().K;
+  };
+  std::vector<bool> harm(nsys, false);
+  std::stable_sort(B.harm.begin(), B.harm.end(),
+                   [&](const HarmSystem &x, const HarmSystem &y) {
+                     return work(x) > work(y);
+                   });
+  double load[kHarmSlots] = {};
+  for (HarmSystem &h : B.harm) {
+    harm[h.sys] = true;
+    h.slot = static_cast<uint32_t>(
+        std::min_element(load, load + kHarmSlots) - load);
+    load[h.slot] += kHarmPairs32 + work(h);
+  }
+  if (!B.harm.empty()) {
+    B.sys_harm = B.sys;
+    for (const HarmSystem &h : B.harm) B.sys_harm[h.sys].nsplit = 1;
+  }
   // units of the fused step's S(k) and back-projection phases, largest
   // radial count first
   struct FusedRun {
@@ -334,12 +388,17 @@ BatchLayout pack_batch(int ct,
     if (d.Kp == 0) continue;
     B.rmt.add(s, d.Kp / d.T);
     const dev::GridShape gs{d.nx, d.ny, d.nz, d.ncell, d.h};
-    if (wave && ct == GLST_CT_FLOAT && dev::rmt_wave_fits(gs))
+    if (wave && ct == GLST_CT_FLOAT && dev::rmt_wave_fits(gs)) {
       B.rmt_small.add(s, d.Kp / dev::kRmtWaveNodes);
-    else
+      if (!harm[s]) B.rmt_small_direct.add(s, d.Kp / dev::kRmtWaveNodes);
+    } else {
       B.rmt_rest.add(s, d.Kp / d.T);
-    B.sf_f64.add(s, d.nx * d.ny * (d.Kp / 256));
-    B.lr_f64.add(s, d.ntile * d.nsplit);
+      if (!harm[s]) B.rmt_rest_direct.add(s, d.Kp / d.T);
+    }
+    if (!harm[s]) {
+      B.sf_f64.add(s, d.nx * d.ny * (d.Kp / 256));
+      B.lr_f64.add(s, d.ntile * d.nsplit);
+    }
     const SplitPlan &P = splits[s];
     const uint32_t task0 = task_first[s];  // first task of the system
     for (size_t g = 0; g < P.sf_groups.size(); ++g) {
@@ -352,15 +411,17 @@ BatchLayout pack_batch(int ct,
       const std::vector<uint32_t> &cm = cs[s]->shape->cheb_m;
       const uint32_t m = cheb && g < cm.size() ? cm[g] : 0u;
       const uint32_t skey = m ? dev::kSfChebKey + m : key;
-      Plan &pf = B.sf_nr[skey];
-      pf.nr = skey;
-      pf.add(s, d.ncell * div_up(sg.ntask, 64),
-             task0 + sg.task0, sg.ntask);
-      Plan &pl = B.lr_nr[key];
-      pl.nr = key;
       // atom-group tiles for the unrolled radial counts (see lr_batch)
       const uint32_t tiles = key != 0 && d.agtile ? d.agtile : d.ntile;
-      pl.add(s, tiles * lg.nsplit, d.split0 + lg.split0, lg.nsplit);
+      if (!harm[s]) {
+        Plan &pf = B.sf_nr[skey];
+        pf.nr = skey;
+        pf.add(s, d.ncell * div_up(sg.ntask, 64),
+               task0 + sg.task0, sg.ntask);
+        Plan &pl = B.lr_nr[key];
+        pl.nr = key;
+        pl.add(s, tiles * lg.nsplit, d.split0 + lg.split0, lg.nsplit);
+      }
       if (ct == GLST_CT_FLOAT) {
         fsf.push_back({sg.nr, s,
                        div_up(d.ncell, dev::kFusedSfCells) *
@@ -389,6 +450,10 @@ glst_batch::~glst_batch() {
   drop_graph();
   if (fail_host) (void)hipHostFree(fail_host);
   if (side) (void)hipStreamDestroy(side);
+  for (hipStream_t h : harm_stream)
+    if (h) (void)hipStreamDestroy(h);
+  for (hipEvent_t e : ev_harm)
+    if (e) (void)hipEventDestroy(e);
   if (ev_assigned) (void)hipEventDestroy(ev_assigned);
   if (ev_near) (void)hipEventDestroy(ev_near);
   if (own_stream && stream) (void)hipStreamDestroy(stream);
@@ -463,9 +528,23 @@ void glst_batch::configure(
   S.grow(B.field * fbytes, hr);
   R.grow(B.field * fbytes, hr);
   partial.grow(B.partial * sizeof(double4), hr);
+  const size_t nslot = std::min<size_t>(B.harm.size(), kHarmSlots);
+  for (size_t i = 0; i < nslot; ++i) {
+    harm_coef[i].grow(B.harm_coef, hr);
+    harm_mom[i].grow(B.harm_mom, hr);
+    harm_out[i].grow(B.harm_out, hr);
+    if (!harm_stream[i])
+      GLST_HIP(hipStreamCreateWithFlags(&harm_stream[i],
+                                        hipStreamNonBlocking));
+    if (!ev_harm[i])
+      GLST_HIP(hipEventCreateWithFlags(&ev_harm[i], hipEventDisableTiming));
+  }
+  for (HarmSystem &h : B.harm)
+    h.plan.unit = tables->harm_device(*cs[h.sys]->shape).unit;
   // B and host_seg stay unchanged until the next configure, which first
   // waits for this batch's stream: the copies may still be in flight
   upload(d_sys, B.sys, stream, hr);
+  if (!B.harm.empty()) upload(d_sys_harm, B.sys_harm, stream, hr);
   upload(t_split, B.t_split, stream, hr);
   // all run tables in one buffer; launches hold offsets until it exists
   std::vector<dev::Seg> &all = host_seg;
@@ -491,6 +570,8 @@ void glst_batch::configure(
   stage(B.rmt, L_rmt);
   stage(B.rmt_small, L_rmt_small);
   stage(B.rmt_rest, L_rmt_rest);
+  stage(B.rmt_small_direct, L_rmt_small_direct);
+  stage(B.rmt_rest_direct, L_rmt_rest_direct);
   stage(B.fsf, L_fsf);
   stage(B.flr, L_flr);
   if (mixed()) {
@@ -508,6 +589,7 @@ void glst_batch::configure(
   if (B.field)
     dev::fill_f64(S.as<double>(), 0.0, B.field * fbytes / sizeof(double),
                   stream);
+  field_layout = -1;
   zero_ef();
   assigned = false;
   // a failed fused step left nothing behind that a new configuration uses
@@ -611,8 +693,12 @@ void glst_batch::release_arenas() {
   for (DeviceBuffer *b :
        {&d_sys, &d_seg, &atom_cell, &rank, &hist, &cell_count, &cell_start,
         &maxc, &sorted_idx, &cell_sorted, &atoms64, &atoms32, &near4, &fx, &fy,
-        &fz, &en, &t_split, &S, &R, &partial, &atom_grp, &ag_start})
+        &fz, &en, &t_split, &S, &R, &partial, &atom_grp, &ag_start,
+        &d_sys_harm})
     b->release();
+  for (uint32_t i = 0; i < kHarmSlots; ++i)
+    for (DeviceBuffer *b : {&harm_coef[i], &harm_mom[i], &harm_out[i]})
+      b->release();
 }
 
 void glst_batch::zero_ef() {
@@ -628,6 +714,58 @@ void glst_batch::near_field(hipStream_t s) {
   check_launch("near field");
 }
 
+void glst_batch::set_field_layout() {
+  if (B.harm.empty()) return;
+  const int want = fused == 0 ? 1 : 0;
+  if (field_layout >= 0 && field_layout != want)
+    dev::fill_f64(S.as<double>(), 0.0,
+                  B.field * (mixed() ? sizeof(float2) : sizeof(double2)) /
+                      sizeof(double),
+                  stream);
+  field_layout = want;
+}
+
+// The far field of one expanded system, on its slot's stream.
+template <typename T>
+void glst_batch::harm_step(const HarmSystem &h) {
+  const dev::SysDev &d = B.sys[h.sys];
+  const ShapeTables &tb = *tables;
+  const dev::HarmDev<T> &H =
+      tables->harm_device(*B.cs[h.sys]->shape).template dev<T>();
+  const hipStream_t s = harm_stream[h.slot];
+  const dev::GridShape g{d.nx, d.ny, d.nz, d.ncell, d.h};
+  const void *atoms = mixed() ? atoms32.as<void>()
+                              : static_cast<const void *>(atoms64.as<void>());
+  const uint32_t *start = cell_start.as<uint32_t>() + d.cell0;
+  const double4 *k64 = tb.d_k64.as<double4>() + d.node0;
+  const uint32_t *group = tb.d_group.as<uint32_t>() + d.node0;
+  const uint32_t *r_in = tb.d_r_in.as<uint32_t>() + d.group0;
+  const uint32_t *r_out = tb.d_r_out.as<uint32_t>() + d.group0;
+  T *Ss = S.as<T>() + 2 * d.field0, *Rs = R.as<T>() + 2 * d.field0;
+  T *coef = harm_coef[h.slot].as<T>(), *mom = harm_mom[h.slot].as<T>();
+  uint32_t *out = harm_out[h.slot].as<uint32_t>();
+  dev::harm_moments<T>(h.plan, H, atoms, start, g, mom, coef, out, s);
+  dev::harm_sf<T>(h.plan, H, atoms, start, k64, g, coef, out, Ss, s);
+  if (mixed() && rmt_wave && dev::rmt_wave_fits(g))
+    dev::rmt_wave(Ss, k64, group, r_in, r_out, d.Kp, g, Rs, s, 0, 0xffffffffu,
+                  true);
+  else if (!(mixed() && dev::rmt_mfma_nodes(g, lds_limit, true) > 0 &&
+             dev::rmt_mfma(Ss, k64, group, r_in, r_out, d.Kp, g, lds_limit, Rs,
+                           s, 0, 0xffffffffu, true)) &&
+           !dev::rmt_lds(mixed(), dev::kRmtMaxNodes, Ss, k64, group, r_in,
+                         r_out, d.Kp, g, lds_limit, Rs, s, 0, 0xffffffffu,
+                         true))
+    throw StateError("shell sums: the cell table does not fit");
+  dev::harm_lr<T>(h.plan, H, g, Rs, coef, mom, s);
+  // the atoms' indices count from the batch's first atom
+  dev::harm_eval<T>(
+      h.plan, H, atoms, start, k64, B.cs[h.sys]->su().K, g, mom, Rs, out,
+      reinterpret_cast<double4 *>(
+          reinterpret_cast<uintptr_t>(partial.as<double4>()) +
+          (d.partial0 - d.atom0) * sizeof(double4)),
+      s);
+}
+
 void glst_batch::step_async(const double *rx, const double *ry,
                             const double *rz, const double *qc) {
   if (!rx || !ry || !rz || !qc)
@@ -637,6 +775,8 @@ void glst_batch::step_async(const double *rx, const double *ry,
     assigned = true;
     return;
   }
+  set_field_layout();
+  const bool expand = fused == 0 && !B.harm.empty();
   const dev::SysDev *sys = d_sys.as<dev::SysDev>();
   // assign_atoms of every system
   dev::fill_u32(hist.as<uint32_t>(), 0u, std::max<uint64_t>(B.hist, 1),
@@ -658,8 +798,23 @@ void glst_batch::step_async(const double *rx, const double *ry,
                          ag_start.as<uint32_t>(), ag);
   check_launch("assign_atoms");
   assigned = true;
+  if (overlap_near || expand) GLST_HIP(hipEventRecord(ev_assigned, stream));
+  if (expand) {
+    bool used[kHarmSlots] = {};
+    for (const HarmSystem &h : B.harm) {
+      if (!used[h.slot])
+        GLST_HIP(hipStreamWaitEvent(harm_stream[h.slot], ev_assigned, 0));
+      used[h.slot] = true;
+      if (mixed())
+        harm_step<float>(h);
+      else
+        harm_step<double>(h);
+    }
+    for (uint32_t i = 0; i < kHarmSlots; ++i)
+      if (used[i]) GLST_HIP(hipEventRecord(ev_harm[i], harm_stream[i]));
+    check_launch("expanded far fields");
+  }
   if (overlap_near) {
-    GLST_HIP(hipEventRecord(ev_assigned, stream));
     GLST_HIP(hipStreamWaitEvent(side, ev_assigned, 0));
     near_field(side);
     GLST_HIP(hipEventRecord(ev_near, side));
@@ -681,11 +836,13 @@ void glst_batch::step_async(const double *rx, const double *ry,
   check_launch("calc_sf");
   dev::rmt_batch(mixed(), S.as<void>(), tb.d_k64.as<double4>(),
                  tb.d_group.as<uint32_t>(), tb.d_r_in.as<uint32_t>(),
-                 tb.d_r_out.as<uint32_t>(), sys, L_rmt_rest, B.lds,
+                 tb.d_r_out.as<uint32_t>(), sys,
+                 fused == 0 ? L_rmt_rest_direct : L_rmt_rest, B.lds,
                  R.as<void>(), stream);
   dev::rmt_wave_batch(S.as<void>(), tb.d_k64.as<double4>(),
                       tb.d_group.as<uint32_t>(), tb.d_r_in.as<uint32_t>(),
-                      tb.d_r_out.as<uint32_t>(), sys, L_rmt_small,
+                      tb.d_r_out.as<uint32_t>(), sys,
+                      fused == 0 ? L_rmt_small_direct : L_rmt_small,
                       R.as<void>(), stream);
   check_launch("sum_rmt_sf");
   if (fused == 3 && mixed())
@@ -699,6 +856,11 @@ void glst_batch::step_async(const double *rx, const double *ry,
     GLST_HIP(hipStreamWaitEvent(stream, ev_near, 0));
   else
     near_field(stream);
+  if (expand) {
+    for (size_t i = 0; i < std::min<size_t>(B.harm.size(), kHarmSlots); ++i)
+      GLST_HIP(hipStreamWaitEvent(stream, ev_harm[i], 0));
+    sys = d_sys_harm.as<dev::SysDev>();
+  }
   dev::lr_reduce_batch(partial.as<double4>(), sys, L_reduce,
                        near4.as<double4>(), fx.as<double>(), fy.as<double>(),
                        fz.as<double>(), en.as<double>(), stream);
@@ -728,6 +890,7 @@ void glst_batch::step(const double *rx, const double *ry, const double *rz,
     return;
   }
   drop_graph();
+  set_field_layout();
   hipGraph_t g = nullptr;
   GLST_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
   try {
@@ -850,9 +1013,11 @@ size_t glst_batch::device_bytes() const {
       &d_sys,   &d_seg,   &atom_cell, &rank,    &hist,    &cell_count,
       &cell_start, &maxc, &sorted_idx, &cell_sorted, &atoms64, &atoms32,
       &near4,   &fx,      &fy,        &fz,      &en,      &t_split,
-      &S,       &R,       &partial, &atom_grp, &ag_start};
+      &S,       &R,       &partial, &atom_grp, &ag_start, &d_sys_harm};
   size_t b = tables ? tables->device_bytes() : 0;
   for (auto p : bufs) b += p->bytes();
+  for (uint32_t i = 0; i < kHarmSlots; ++i)
+    b += harm_coef[i].bytes() + harm_mom[i].bytes() + harm_out[i].bytes();
   return b;
 }
 

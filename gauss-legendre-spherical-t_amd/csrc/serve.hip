@@ -171,6 +171,13 @@ struct glst_server {
       if (!inp[k] || !outp[k]) throw ArgError("null input or output array");
     check_system_args(ct, box[0], box[1], box[2], rcut, tol);
     SysEntry &e = lookup(natom, box, rcut);
+    if (e.bytes > share() && !e.sys->direct) {
+      // the direct sums need fewer work fields
+      ShapeTables sizing;
+      e.sys = make_batch_system(natom, e.sys->shape, true);
+      e.bytes = pack_batch(ct, {e.sys}, sizing, lds_limit).device_bytes() +
+                8 * sizeof(double) * static_cast<size_t>(natom);
+    }
     if (e.bytes > share()) {
       ++stats.rejected;
       throw AllocError("request needs " + std::to_string(e.bytes) +
