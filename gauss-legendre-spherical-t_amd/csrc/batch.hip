@@ -189,7 +189,8 @@ void ShapeTables::upload(hipStream_t s) {
 
 const HarmDevice &ShapeTables::harm_device(const ShapeSetup &shape) {
   HarmDevice &d = harm[&shape];
-  if (!d.ok()) d.upload(shape.harm(), shape.ct == GLST_CT_FLOAT);
+  if (!d.ok())
+    d.upload(shape.harm(), shape.ct == GLST_CT_FLOAT, shape.nl.k64);
   return d;
 }
 
@@ -730,14 +731,14 @@ template <typename T>
 void glst_batch::harm_step(const HarmSystem &h) {
   const dev::SysDev &d = B.sys[h.sys];
   const ShapeTables &tb = *tables;
-  const dev::HarmDev<T> &H =
-      tables->harm_device(*B.cs[h.sys]->shape).template dev<T>();
+  const HarmDevice &hd = tables->harm_device(*B.cs[h.sys]->shape);
+  const dev::HarmDev<T> &H = hd.template dev<T>();
   const hipStream_t s = harm_stream[h.slot];
   const dev::GridShape g{d.nx, d.ny, d.nz, d.ncell, d.h};
   const void *atoms = mixed() ? atoms32.as<void>()
                               : static_cast<const void *>(atoms64.as<void>());
   const uint32_t *start = cell_start.as<uint32_t>() + d.cell0;
-  const double4 *k64 = tb.d_k64.as<double4>() + d.node0;
+  const double4 *k64 = hd.k64;
   const uint32_t *group = tb.d_group.as<uint32_t>() + d.node0;
   const uint32_t *r_in = tb.d_r_in.as<uint32_t>() + d.group0;
   const uint32_t *r_out = tb.d_r_out.as<uint32_t>() + d.group0;

@@ -224,6 +224,7 @@ struct glst_engine {
   // The expansion of the far field, where it is worth its passes (harm_worth)
   // and the nodes and the device can hold it.
   size_t harm_coef_len = 0, harm_mom_len = 0;
+  std::vector<uint32_t> harm_row_of;  // row of the fields of a node
   void plan_far_field() {
     if (!has_lr || Kp == 0 || !harm_worth(natom, K, mixed())) return;
     const HarmTables t = plan_harmonic(nodes, grid.h, spherical_rule, mixed());
@@ -231,12 +232,15 @@ struct glst_engine {
     harm_plan = harm_fit(t, mixed(), lds_limit, natom, grid.ncell);
     if (harm_plan.nrad == 0) return;
     try {
-      harm.upload(t, mixed());
+      harm.upload(t, mixed(), layout_nodes(nodes, K, Kp).k64);
     } catch (const AllocError &) {
       harm.release();
       return;
     }
     harm_plan.unit = harm.unit;
+    harm_row_of.resize(t.node_of_row.size());
+    for (uint32_t r = 0; r < harm_row_of.size(); ++r)
+      harm_row_of[t.node_of_row[r]] = r;
     harm_coef_len = glst::harm_coef_len(t, grid.ncell);
     harm_mom_len = glst::harm_mom_len(t, grid.ncell);
   }
@@ -409,7 +413,7 @@ struct glst_engine {
                              harm_mom.as<T>(), harm_coef.as<T>(), harm_out.as<uint32_t>(),
                              stream);
         dev::harm_sf<T>(harm_plan, harm.dev<T>(), lr_atoms(),
-                        cell_start.as<uint32_t>(), k64.as<double4>(), grid,
+                        cell_start.as<uint32_t>(), harm.k64, grid,
                         harm_coef.as<T>(), harm_out.as<uint32_t>(), S.as<T>(),
                         stream);
       };
@@ -436,25 +440,26 @@ struct glst_engine {
       throw StateError("sum_rmt_sf called before calc_sf");
     Scope sc(timer, "rmt", stream);
     const bool nm = harmonic();
+    const double4 *kn = nm ? harm.k64 : k64.as<double4>();
     if (rmt_mfma_path()) {
-      dev::rmt_mfma(S.as<void>(), k64.as<double4>(), group.as<uint32_t>(),
+      dev::rmt_mfma(S.as<void>(), kn, group.as<uint32_t>(),
                     r_in.as<uint32_t>(), r_out.as<uint32_t>(), Kp, grid,
                     lds_limit, R.as<void>(), stream, 0, 0xffffffffu, nm);
     } else if (rmt_wave_path()) {
-      dev::rmt_wave(S.as<void>(), k64.as<double4>(), group.as<uint32_t>(),
+      dev::rmt_wave(S.as<void>(), kn, group.as<uint32_t>(),
                     r_in.as<uint32_t>(), r_out.as<uint32_t>(), Kp, grid,
                     R.as<void>(), stream, 0, 0xffffffffu, nm);
     } else if (rmt_shape == 2 ||
         !dev::rmt_lds(mixed(), rmt_shape == 1 ? 1 : dev::kRmtMaxNodes,
                       S.as<void>(),
-                      k64.as<double4>(), group.as<uint32_t>(),
+                      kn, group.as<uint32_t>(),
                       r_in.as<uint32_t>(), r_out.as<uint32_t>(), Kp, grid,
                       lds_limit, R.as<void>(), stream, 0, 0xffffffffu,
                       nm)) {
       // tables too large for LDS: FP64 work field, allocated on first use
       rmt_work.resize(static_cast<size_t>(grid.ncell) * Kp * sizeof(double2));
       dev::rmt_global(mixed(), S.as<void>(), rmt_work.as<double2>(),
-                      k64.as<double4>(), group.as<uint32_t>(),
+                      kn, group.as<uint32_t>(),
                       r_in.as<uint32_t>(), r_out.as<uint32_t>(), Kp, grid,
                       R.as<void>(), stream, nm);
     }
@@ -497,7 +502,7 @@ struct glst_engine {
         dev::harm_lr<T>(harm_plan, harm.dev<T>(), grid, R.as<T>(),
                         harm_coef.as<T>(), harm_mom.as<T>(), stream);
         dev::harm_eval<T>(harm_plan, harm.dev<T>(), lr_atoms(),
-                          cell_start.as<uint32_t>(), k64.as<double4>(), K,
+                          cell_start.as<uint32_t>(), harm.k64, K,
                           grid, harm_mom.as<T>(), R.as<T>(),
                           harm_out.as<uint32_t>(), partial.as<double4>(),
                           stream);
@@ -908,7 +913,7 @@ struct glst_engine {
     }
     for (uint32_t c = 0; c < grid.ncell; ++c)
       for (uint32_t k = 0; k < K; ++k) {
-        const uint32_t node = dev_of_ref[k];
+        const uint32_t node = nm ? harm_row_of[dev_of_ref[k]] : dev_of_ref[k];
         const size_t d = static_cast<size_t>(c) * K + k;
         if (nm) {
           const size_t a = single ? dev::harm_slot<float>(node, c, 0, ncp)

@@ -135,6 +135,21 @@ __device__ __forceinline__ HarmCentre harm_centre(uint32_t cell, uint32_t ny,
 __device__ __forceinline__ void harm_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
+// The scalar at byte `off` of the `bytes` from a base uniform over the wave, or
+// zero past them: the buffer's own range check takes the place of a compare,
+// a clamped address and a select per load.
+template <typename T>
+__device__ __forceinline__ T harm_ranged(const T *base, uint32_t bytes,
+                                         uint32_t off) {
+  const auto r = __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(base), 0,
+                                                   bytes, 0x00020000);
+  if constexpr (sizeof(T) == 4)
+    return __builtin_bit_cast(
+        T, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
+  else
+    return __builtin_bit_cast(
+        T, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
+}
 // p[byte offset], the base uniform over the wave
 template <typename T>
 __device__ __forceinline__ T harm_at_byte(const T *p, uint32_t off) {
@@ -637,6 +652,7 @@ __device__ __forceinline__ void harm_sf_body(
   const uint32_t c16 = lane & 15u, g = lane >> 4;
   const uint32_t N = rad.N, KS = harm_mode_steps(N), MS = 4 * KS;
   const uint32_t RS = MS * 16 + 8;
+  const uint32_t nd = harm_dirs(gr);
   const uint32_t nrow = F ? 16u : 8u;
   T *Gm = reinterpret_cast<T *>(smem);
   T *tr = Gm + nrow * RS;
@@ -644,7 +660,9 @@ __device__ __forceinline__ void harm_sf_body(
   const uint32_t ncp = harm_row(ncell);
   // columns of (1): the cosines of the eight cells, then the sines
   const uint32_t c8 = c16 & 7u, cs = c16 >> 3;
-  const T *cf = coef + (static_cast<size_t>(tile) * H.stride + rad.off) * 8 + c16;
+  const T *cf = coef + (static_cast<size_t>(tile) * H.stride + rad.off) * 8;
+  constexpr uint32_t kRow = 256 * sizeof(T);  // from a degree to the next but one
+  const uint32_t brow = g * kRow + c16 * sizeof(T);
   const T *leg = H.leg + (static_cast<size_t>(gr.leg) + rt * gr.leg_n) * 64 + lane;
   for (uint32_t pass = 0; pass < (F ? 1u : 2u); ++pass) {
     v4 E[NR][NPT];
@@ -674,10 +692,8 @@ __device__ __forceinline__ void harm_sf_body(
                                      2 * (mu & 7u) : 0u) * 8;
 #pragma unroll
           for (uint32_t u = 0; u < 4; ++u) {
-            const uint32_t j = 4 * u + g;
             la[pp][u] = A[u * 64];  // (the table ends with four more steps)
-            const T b = B[(j < n ? j : 0u) * 256];
-            lb[pp][u] = j < n ? b : T(0);
+            lb[pp][u] = harm_ranged(B, n * kRow, brow + 4 * u * kRow);
           }
         }
       };
@@ -712,11 +728,10 @@ __device__ __forceinline__ void harm_sf_body(
               const T *A = leg + H.mup[gr.mup + 2 * mu + par].x * 64;
               const T *B =
                   cf + (harm_block(mu >> 3, l0, N) * 16 + 2 * (mu & 7u)) * 8;
-              for (uint32_t k = 16; k < n; k += 4) {
-                const uint32_t j = k + g;
-                const T b = B[(j < n ? j : 0u) * 256];
-                acc[pp] = M::mfma(A[k * 16], j < n ? b : T(0), acc[pp]);
-              }
+              for (uint32_t k = 16; k < n; k += 4)
+                acc[pp] = M::mfma(
+                    A[k * 16], harm_ranged(B, n * kRow, brow + k * kRow),
+                    acc[pp]);
             }
           }
         }
@@ -740,8 +755,10 @@ __device__ __forceinline__ void harm_sf_body(
 #pragma unroll
         for (int pt = 0; pt < NPT; ++pt) X[u][pt] = v4{T(0), T(0), T(0), T(0)};
       const T *At = tr + lane, *Bt = Gm + wave * RS + lane;
+      // (a wave whose first row is past the rings has nothing to do)
+      const bool some = 16 * rt + (F ? wave : 2 * wave) < gr.nring;
 #pragma unroll 2
-      for (uint32_t ks = 0; ks < KS; ++ks) {
+      for (uint32_t ks = 0; some && ks < KS; ++ks) {
         T a[NPT], b[NR];
 #pragma unroll
         for (int pt = 0; pt < NPT; ++pt) a[pt] = At[(pt * KS + ks) * 64];
@@ -762,7 +779,7 @@ __device__ __forceinline__ void harm_sf_body(
       } else {
         // bytes of an azimuth: a ring's offsets fit 32 bits
         const uint32_t az =
-            gr.nr * static_cast<uint32_t>(2 * ncp * sizeof(T));
+            static_cast<uint32_t>(2 * ncp * sizeof(T));
 #pragma unroll
         for (int u = 0; u < NR; ++u) {
           const uint32_t row = wave + u * NW;
@@ -772,7 +789,7 @@ __device__ __forceinline__ void harm_sf_body(
               gr.equator ? (ring0 ? gr.h + 2 * gr.h * (ring0 - 1) : 0u)
                          : 2 * gr.h * ring0;
           char *base = reinterpret_cast<char *>(
-              S + harm_slot<T>(gr.node0 + dir0 * gr.nr + rad.idx, cell0,
+              S + harm_slot<T>(gr.node0 + rad.idx * nd + dir0, cell0,
                                F ? 0u : pass, ncp));
           bool eq = gr.equator && ring0 == 0, on = true;
           uint32_t off = c16 * 4;
@@ -805,7 +822,6 @@ __device__ __forceinline__ void harm_sf_body(
   if (!any) return;
   // atoms outside the unit ball: their terms one by one
   __syncthreads();
-  const uint32_t nd = gr.nring * 2 * gr.h - (gr.equator ? gr.h : 0u);
   const uint32_t d0 = rt ? 32 * gr.h * rt - (gr.equator ? gr.h : 0u) : 0u;
   const uint32_t d1 =
       32 * gr.h * (rt + 1) - (gr.equator ? gr.h : 0u) < nd
@@ -814,7 +830,7 @@ __device__ __forceinline__ void harm_sf_body(
   for (uint32_t e = tid; e < (d1 - d0) * kHarmCells; e += kHarmBlock) {
     const uint32_t cell = cell0 + (e & (kHarmCells - 1));
     if (cell >= ncell || !outside[cell]) continue;
-    const uint32_t node = gr.node0 + (d0 + e / kHarmCells) * gr.nr + rad.idx;
+    const uint32_t node = gr.node0 + rad.idx * nd + d0 + e / kHarmCells;
     const double4 k = k64[node];
     const HarmCentre cc = harm_centre(cell, ny, nz, h);
     double re = 0.0, im = 0.0;
@@ -894,7 +910,8 @@ __device__ __forceinline__ void harm_lr_body(
   T *cf = coef + (static_cast<size_t>(tile) * H.stride + rad.off) * 8 + c16;
   const T *legt = H.legt + static_cast<size_t>(gr.legt) * 64 + lane;
   // bytes of an azimuth: a row's offsets stay below 4 h of them (32 bits)
-  const uint32_t az = gr.nr * static_cast<uint32_t>(2 * ncp * sizeof(T));
+  const uint32_t az = static_cast<uint32_t>(2 * ncp * sizeof(T));
+  const uint32_t nd = harm_dirs(gr);
   for (uint32_t pass = 0; pass < (F ? 1u : 2u); ++pass) {
     // A row past the rings and an azimuth past the half ring repeat the last
     // one (their factors are zero); the equator has no second half.
@@ -905,7 +922,7 @@ __device__ __forceinline__ void harm_lr_body(
       const uint32_t r0 = ring0 < gr.nring ? ring0 : gr.nring - 1;
       const uint32_t dir0 =
           gr.equator ? (r0 ? gr.h + 2 * gr.h * (r0 - 1) : 0u) : 2 * gr.h * r0;
-      const T *base = R + harm_slot<T>(gr.node0 + dir0 * gr.nr + rad.idx, cell0,
+      const T *base = R + harm_slot<T>(gr.node0 + rad.idx * nd + dir0, cell0,
                                        F ? 0u : pass, ncp);
       const bool eq = gr.equator && r0 == 0;
       uint32_t off = c16 * 4, second = eq ? 0u : gr.h * az;

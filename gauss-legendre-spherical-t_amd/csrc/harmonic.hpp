@@ -21,7 +21,11 @@
 //
 // Fields of this path are node-major: S and R hold a row of `ncp` cells for
 // every node (mixed: (re, im) pairs; FP64: the row of real parts, then the
-// row of imaginary parts).  S = sum_j q_j exp(-i k.d_j) around the cell
+// row of imaginary parts).  The rows of a group run over its directions for
+// each radial node in turn (elsewhere: over the radial nodes for each
+// direction), so that a workgroup, which holds one radial node, meets adjacent
+// rows: at 1.0M charges, where they were 1.2 MB apart, S took 3,938 us and the
+// way back 2,599; the nodes' table of this path is in the same order.  S = sum_j q_j exp(-i k.d_j) around the cell
 // centre, R = V = exp(+i k.c) R_c(k).
 #pragma once
 
@@ -80,6 +84,11 @@ struct HarmGroup {
   uint32_t trig, trig_k;  // Fourier, orders -> azimuths: [tile][set][step]
   uint32_t trigt, trigt_m, trigt_k;  // azimuths -> orders: [set][tile][step]
 };
+
+// directions of a group
+__host__ __device__ inline uint32_t harm_dirs(const HarmGroup &g) {
+  return g.nring * 2 * g.h - (g.equator ? g.h : 0u);
+}
 
 // Expansion tables on the device (T: the calculation type).
 template <typename T>

@@ -86,6 +86,7 @@ struct HarmTables {
   std::vector<uint32_t> crow, urow, qoff;
   uint32_t rows = 0;
   std::vector<uint2> unit;  // (radial node, ring tile)
+  std::vector<uint32_t> node_of_row;  // node (device order) of a fields' row
   uint32_t N = 0, stride = 0;
   double scale = 0.0, smax = 0.0;
   uint32_t hsteps = 0;
@@ -97,6 +98,7 @@ struct HarmTables {
            rad.size() * sizeof(rad[0]) + grp.size() * sizeof(grp[0]) +
            (mup.size() + pair.size() + unit.size()) * sizeof(uint2) +
            lrow.size() * sizeof(uint4) + (crow.size() + urow.size()) * 4 +
+           (node_of_row.size() + 256) * sizeof(double4) +
            20 * 256;
   }
 };
@@ -142,6 +144,9 @@ inline HarmTables plan_harmonic(const NodeTable &nodes, double h,
       T.rad.push_back({N, static_cast<uint32_t>(g), i, 0u});
     }
     T.grp.push_back(G);
+    for (uint32_t i = 0; i < G.nr; ++i)
+      for (uint32_t j = 0; j < d.size(); ++j)
+        T.node_of_row.push_back(G.node0 + j * G.nr + i);
   }
   std::stable_sort(T.rad.begin(), T.rad.end(),
                    [](const dev::HarmRad &a, const dev::HarmRad &b) {
@@ -422,11 +427,13 @@ class HarmDevice {
   bool ok() const { return buf_.bytes() > 0; }
   size_t device_bytes() const { return buf_.bytes(); }
   const uint2 *unit = nullptr;  // HarmPlanDev::unit
+  const double4 *k64 = nullptr;  // the nodes in the order of the fields' rows
   template <typename T>
   const dev::HarmDev<T> &dev() const;
   void release() { buf_.release(); }
 
-  void upload(const HarmTables &t, bool single) {
+  void upload(const HarmTables &t, bool single,
+              const std::vector<double4> &nodes) {
     // one buffer, every table on a 256-byte boundary
     std::vector<char> host;
     auto raw = [&](const void *p, size_t bytes) {
@@ -447,6 +454,10 @@ class HarmDevice {
     const size_t pair = raw(t.pair.data(), t.pair.size() * sizeof(uint2));
     const size_t crow = raw(t.crow.data(), t.crow.size() * 4);
     const size_t urow = raw(t.urow.data(), t.urow.size() * 4);
+    std::vector<double4> k(nodes);
+    for (size_t r = 0; r < t.node_of_row.size(); ++r)
+      k[r] = nodes[t.node_of_row[r]];
+    const size_t kat = raw(k.data(), k.size() * sizeof(double4));
     const size_t units = raw(t.unit.data(), t.unit.size() * sizeof(uint2));
     const size_t leg = real(t.leg), legt = real(t.legt);
     const size_t trig = real(t.trig), trigt = real(t.trigt);
@@ -486,6 +497,7 @@ class HarmDevice {
       d.smax = t.smax;
       d.xk = 2.0 / t.smax;
       unit = reinterpret_cast<const uint2 *>(b + units);
+      k64 = reinterpret_cast<const double4 *>(b + kat);
     };
     if (single)
       fill(f_);
