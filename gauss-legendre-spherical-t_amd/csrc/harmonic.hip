@@ -592,9 +592,10 @@ __global__ __launch_bounds__(256) void harm_radial_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// coefficients -> structure factors (414 and 1,197 us; the wave's share of the
-// tables' loads and index arithmetic, about as many scalar as vector
-// instructions, against 0.15 and 0.29 ms of stores)
+// coefficients -> structure factors (374 and 943 us, 400 and 1,131 with the
+// azimuths up to pi summed one by one, 415 and 1,194 before that with a select
+// per coefficient; the workgroups' phases between barriers, two to three
+// workgroups per CU, against 0.15 and 0.29 ms of stores)
 
 // Which (unit, cell tile) a workgroup serves.  With many tiles every XCD
 // (workgroups b with b % 8 == x) owns a contiguous range of them and takes
@@ -619,20 +620,21 @@ uint32_t harm_grid(uint32_t ntile, uint32_t nunit) {
   return 8 * nunit * ((ntile + 7) / 8);
 }
 
-// Modes of one set (even or odd azimuthal orders), padded to whole steps of
-// four: mode 2 m + cs is the cosine (cs 0) or sine of order 2 m + set.
-__device__ __forceinline__ uint32_t harm_mode_steps(uint32_t N) {
-  return ((N + 1) / 2 + 1) / 2;
+// Steps of four over the orders of one set (even or odd azimuthal orders).
+__host__ __device__ inline uint32_t harm_order_steps(uint32_t N) {
+  return ((N + 1) / 2 + 3) / 4;
 }
 
 // One unit: eight cells, one radial node, a tile of 16 rings.  Even and odd
 // orders take turns: (1) Legendre: per order, the rings' Fourier coefficients
 // of Re (even degrees) and Im (odd degrees) into LDS; columns are (cosine or
 // sine, cell); a wave's next order is loaded while it works on one.  (2)
-// Fourier: per ring (wave and wave + 8 in FP32), the sums E over the even and
-// O over the odd orders at NPT tiles of azimuths, in registers; the values at
-// phi and phi + pi are E + O and E - O.  Columns are (cell, Re or Im) in FP32;
-// in FP64 Re and Im take turns and the columns are (ring of a pair, cell).
+// Fourier: per ring (wave and wave + 8 in FP32), the sums C over the cosines
+// and Z over the sines at NPT tiles of azimuths phi in 0 .. pi / 2, in
+// registers, which give those at pi - phi too (C - Z for even, Z - C for odd
+// orders); the values at phi and phi + pi are the even sum plus and minus the
+// odd one.  Columns are (cell, Re or Im) in FP32; in FP64 Re and Im take turns
+// and the columns are (ring of a pair, cell).
 template <typename T, int NPT>
 __device__ __forceinline__ void harm_sf_body(
     const HarmDev<T> &H, const typename HarmRecord<T>::type *atoms,
@@ -650,8 +652,9 @@ __device__ __forceinline__ void harm_sf_body(
   const uint32_t lane = tid & 63u;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t c16 = lane & 15u, g = lane >> 4;
-  const uint32_t N = rad.N, KS = harm_mode_steps(N), MS = 4 * KS;
-  const uint32_t RS = MS * 16 + 8;
+  // a ring's cosines, then its sines (other banks), in steps of four orders
+  const uint32_t N = rad.N, KC = harm_order_steps(N), MH = 4 * KC;
+  const uint32_t sines = MH * 16 + 16, RS = 2 * MH * 16 + 24;
   const uint32_t nd = harm_dirs(gr);
   const uint32_t nrow = F ? 16u : 8u;
   T *Gm = reinterpret_cast<T *>(smem);
@@ -665,15 +668,16 @@ __device__ __forceinline__ void harm_sf_body(
   const uint32_t brow = g * kRow + c16 * sizeof(T);
   const T *leg = H.leg + (static_cast<size_t>(gr.leg) + rt * gr.leg_n) * 64 + lane;
   for (uint32_t pass = 0; pass < (F ? 1u : 2u); ++pass) {
-    v4 E[NR][NPT];
+    v4 E[2][NR][NPT];
 #pragma unroll
     for (uint32_t set = 0; set < 2; ++set) {
       // the Fourier matrix of the set, as far as this node's degrees go
-      for (uint32_t e = wave; e < NPT * KS; e += NW) {
-        const uint32_t pt = e / KS, ks = e - pt * KS;
+      for (uint32_t e = wave; e < 2 * NPT * KC; e += NW) {
+        const uint32_t pc = e / KC, ks = e - pc * KC;  // pc: 2 pt + cs
+        const uint32_t from = pc < 2 * gr.trig_t ? pc : pc & 1u;
         tr[e * 64 + lane] =
             H.trig[(static_cast<size_t>(gr.trig) +
-                    (2 * pt + set) * gr.trig_k + ks) * 64 + lane];
+                    (2 * from + set) * gr.trig_k + ks) * 64 + lane];
       }
       // (1) degrees l0, l0 + 2, ... of a parity: the first 16 in flight
       T la[NP][4], lb[NP][4];
@@ -698,8 +702,9 @@ __device__ __forceinline__ void harm_sf_body(
         }
       };
       if (2 * wave + set < N) fetch(2 * wave + set);
-      for (uint32_t m = wave; m < 2 * KS; m += NW) {
-        const uint32_t mu = 2 * m + set, mode = 2 * m + cs;
+      for (uint32_t m = wave; m < MH; m += NW) {
+        const uint32_t mu = 2 * m + set;
+        const uint32_t mode = cs * sines + m * 16;
         v4 acc[NP];
 #pragma unroll
         for (uint32_t pp = 0; pp < NP; ++pp)
@@ -741,41 +746,52 @@ __device__ __forceinline__ void harm_sf_body(
           for (uint32_t r = 0; r < 4; ++r) {
             const uint32_t ring = M::row(g, r);
             if (F)
-              Gm[ring * RS + mode * 16 + c8 * 2 + pp] = acc[pp][r];
+              Gm[ring * RS + mode + c8 * 2 + pp] = acc[pp][r];
             else
-              Gm[(ring >> 1) * RS + mode * 16 + (ring & 1u) * 8 + c8] =
-                  acc[pp][r];
+              Gm[(ring >> 1) * RS + mode + (ring & 1u) * 8 + c8] = acc[pp][r];
           }
       }
       harm_barrier();
       // (2)
-      v4 X[NR][NPT];
+      v4 X[2][NR][NPT];  // cosines, sines
 #pragma unroll
-      for (int u = 0; u < NR; ++u)
-#pragma unroll
-        for (int pt = 0; pt < NPT; ++pt) X[u][pt] = v4{T(0), T(0), T(0), T(0)};
-      const T *At = tr + lane, *Bt = Gm + wave * RS + lane;
-      // (a wave whose first row is past the rings has nothing to do)
-      const bool some = 16 * rt + (F ? wave : 2 * wave) < gr.nring;
-#pragma unroll 2
-      for (uint32_t ks = 0; some && ks < KS; ++ks) {
-        T a[NPT], b[NR];
-#pragma unroll
-        for (int pt = 0; pt < NPT; ++pt) a[pt] = At[(pt * KS + ks) * 64];
-#pragma unroll
-        for (int u = 0; u < NR; ++u) b[u] = Bt[u * NW * RS + ks * 64];
+      for (int c = 0; c < 2; ++c)
 #pragma unroll
         for (int u = 0; u < NR; ++u)
 #pragma unroll
           for (int pt = 0; pt < NPT; ++pt)
-            X[u][pt] = M::mfma(a[pt], b[u], X[u][pt]);
+            X[c][u][pt] = v4{T(0), T(0), T(0), T(0)};
+      const T *At = tr + lane, *Bt = Gm + wave * RS + lane;
+      // (a wave whose first row is past the rings has nothing to do)
+      const bool some = 16 * rt + (F ? wave : 2 * wave) < gr.nring;
+#pragma unroll 2
+      for (uint32_t ks = 0; some && ks < KC; ++ks) {
+        T a[2][NPT], b[2][NR];
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+#pragma unroll
+          for (int pt = 0; pt < NPT; ++pt)
+            a[c][pt] = At[((2 * pt + c) * KC + ks) * 64];
+#pragma unroll
+          for (int u = 0; u < NR; ++u)
+            b[c][u] = Bt[u * NW * RS + c * sines + ks * 64];
+        }
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+          for (int u = 0; u < NR; ++u)
+#pragma unroll
+            for (int pt = 0; pt < NPT; ++pt)
+              X[c][u][pt] = M::mfma(a[c][pt], b[c][u], X[c][u][pt]);
       }
       harm_barrier();
       if (set == 0) {
 #pragma unroll
-        for (int u = 0; u < NR; ++u)
+        for (int c = 0; c < 2; ++c)
 #pragma unroll
-          for (int pt = 0; pt < NPT; ++pt) E[u][pt] = X[u][pt];
+          for (int u = 0; u < NR; ++u)
+#pragma unroll
+            for (int pt = 0; pt < NPT; ++pt) E[c][u][pt] = X[c][u][pt];
       } else {
         // bytes of an azimuth: a ring's offsets fit 32 bits
         const uint32_t az =
@@ -804,13 +820,16 @@ __device__ __forceinline__ void harm_sf_body(
 #pragma unroll
             for (uint32_t r = 0; r < 4; ++r) {
               const uint32_t phi = 16 * pt + M::row(g, r);
-              if (phi < gr.h && on) {
-                const uint32_t oa = off + phi * az;
-                *reinterpret_cast<T *>(base + oa) = E[u][pt][r] + X[u][pt][r];
-                if (!eq)
-                  *reinterpret_cast<T *>(base + oa + gr.h * az) =
-                      E[u][pt][r] - X[u][pt][r];
-              }
+              const T ec = E[0][u][pt][r], es = E[1][u][pt][r];
+              const T oc = X[0][u][pt][r], os = X[1][u][pt][r];
+              auto put = [&](uint32_t k, T e, T o) {
+                const uint32_t oa = off + k * az;
+                *reinterpret_cast<T *>(base + oa) = e + o;
+                if (!eq) *reinterpret_cast<T *>(base + oa + gr.h * az) = e - o;
+              };
+              if (2 * phi <= gr.h && on) put(phi, ec + es, oc + os);
+              if (phi > 0 && 2 * phi < gr.h && on)
+                put(gr.h - phi, ec - es, os - oc);
             }
         }
       }
@@ -865,8 +884,8 @@ __global__ __launch_bounds__(kHarmBlock) void harm_sf_kernel(
   const uint2 u = units[unit];
   const HarmRad rad = H.rad[u.x];
   const HarmGroup gr = H.grp[rad.group];
-  // tiles of 16 azimuths over half a ring
-  harm_switch<NPT>((gr.h + 15) / 16, [&](auto npt) {
+  // tiles of 16 azimuths up to pi / 2
+  harm_switch<NPT>(gr.trig_t, [&](auto npt) {
     harm_sf_body<T, decltype(npt)::value>(H, atoms, start, k64, ny, nz, h,
                                           ncell, rad, gr, u.y, tile, coef,
                                           outside, S, harm_smem);
@@ -874,15 +893,18 @@ __global__ __launch_bounds__(kHarmBlock) void harm_sf_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// remote sums -> coefficients (436 and 1,310 us; reads R once, 0.15 and 0.29 ms,
-// and is held by the wait for it and by the same overhead as harm_sf)
+// remote sums -> coefficients (420 and 1,162 us, 438 and 1,311 with the azimuths
+// up to pi summed one by one and every group in the registers of the largest;
+// reads R once, 0.15 and 0.29 ms, all loads of a workgroup in flight, then the
+// phases between barriers as in harm_sf)
 
 // One unit: eight cells, one radial node, all rings; the transpose of
 // harm_sf_body.  Every wave first loads its rings' values, all loads in
-// flight at once (RW rows of 2 HK values per lane; FP64 rows are pairs of
+// flight at once (RW rows of 4 HK values per lane; FP64 rows are pairs of
 // rings, and Re and Im take turns).  Even and odd orders take turns, so that
-// all the rings' Fourier sums of one set fit in LDS: (1) per ring, the sums
-// over the azimuths of V(phi) +- V(phi + pi) against the cosines and sines;
+// all the rings' Fourier sums of one set fit in LDS: (1) per ring, f =
+// V(phi) +- V(phi + pi), and f(phi) +- f(pi - phi) summed over the azimuths up
+// to pi / 2 against the cosines and, with the other sign, the sines;
 // (2) per order and parity, the sums over the rings against the Legendre
 // functions, stored as the cells' coefficients.
 template <typename T, int RW, int HK, int MT>
@@ -897,7 +919,7 @@ __device__ __forceinline__ void harm_lr_body(
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t c16 = lane & 15u, g = lane >> 4;
-  const uint32_t N = rad.N, KS = harm_mode_steps(N), MS = 4 * KS;
+  const uint32_t N = rad.N, MS = 8 * harm_order_steps(N);
   const uint32_t RS = MS * 16 + 8;
   const uint32_t hk = gr.trigt_k;
   const uint32_t nrow = F ? 4 * gr.legt_k : 2 * gr.legt_k;  // padded rings
@@ -913,9 +935,10 @@ __device__ __forceinline__ void harm_lr_body(
   const uint32_t az = static_cast<uint32_t>(2 * ncp * sizeof(T));
   const uint32_t nd = harm_dirs(gr);
   for (uint32_t pass = 0; pass < (F ? 1u : 2u); ++pass) {
-    // A row past the rings and an azimuth past the half ring repeat the last
-    // one (their factors are zero); the equator has no second half.
-    T va[RW][HK], vb[RW][HK];
+    // A row past the rings and an azimuth past pi / 2 repeat the last one
+    // (their factors are zero); the equator has no second half.  phi = 0 and
+    // pi / 2 have no partner at pi - phi.
+    T va[RW][HK], vb[RW][HK], wa[RW][HK], wb[RW][HK];
 #pragma unroll
     for (int w = 0; w < RW; ++w) {
       const uint32_t ring0 = F ? wave + w * NW : 2 * (wave + w * NW);
@@ -931,22 +954,25 @@ __device__ __forceinline__ void harm_lr_body(
         off = (c16 & 7u) * 8 + (next ? (eq ? gr.h : 2 * gr.h) * az : 0u);
         if (next) second = gr.h * az;
       }
-      const uint32_t end = off + (gr.h - 1) * az;
-      off += g * az;
 #pragma unroll
       for (int ks = 0; ks < HK; ++ks) {
-        const uint32_t o = off + 4 * ks * az;
-        const uint32_t oc = o < end ? o : end;
-        va[w][ks] = harm_at_byte(base, oc);
-        vb[w][ks] = harm_at_byte(base, oc + second);
+        const uint32_t k = 4 * ks + g < gr.h / 2 ? 4 * ks + g : gr.h / 2;
+        const bool two = k > 0 && 2 * k < gr.h;
+        const uint32_t o = off + k * az;
+        const uint32_t p = off + (two ? gr.h - k : k) * az;
+        va[w][ks] = harm_at_byte(base, o);
+        vb[w][ks] = harm_at_byte(base, o + second);
+        const T x = harm_at_byte(base, p), y = harm_at_byte(base, p + second);
+        wa[w][ks] = two ? x : T(0);
+        wb[w][ks] = two ? y : T(0);
       }
     }
     if (pass == 0) {
-      for (uint32_t e = wave; e < 2 * MT * HK; e += NW) {
+      for (uint32_t e = wave; e < 4 * MT * HK; e += NW) {
         const uint32_t sm = e / HK, ks = e - sm * HK;
-        const uint32_t set = sm / MT, mt = sm - set * MT;
+        const uint32_t sc = sm / MT, mt = sm - sc * MT;  // sc: 2 set + cs
         const T x = H.trigt[(static_cast<size_t>(gr.trigt) +
-                             (set * gr.trigt_m + mt) * hk +
+                             (sc * gr.trigt_m + mt) * hk +
                              (ks < hk ? ks : 0u)) * 64 + lane];
         tr[e * 64 + lane] = ks < hk ? x : T(0);
       }
@@ -969,30 +995,33 @@ __device__ __forceinline__ void harm_lr_body(
         const uint32_t row = wave + w * NW;
         const uint32_t ring = F ? row : 2 * row + (c16 >> 3);
         const T half2 = gr.equator && ring == 0 ? T(0) : set ? T(-1) : T(1);
-        // (partial sums: the rounding of a sum grows with its length)
-        constexpr int NA = F && MT == 1 ? 2 : 1;
-        v4 acc[MT * NA];
+        v4 acc[2][MT];  // cosines, sines
 #pragma unroll
-        for (int m = 0; m < MT * NA; ++m)
-          acc[m] = v4{T(0), T(0), T(0), T(0)};
-        const T *At = tr + set * MT * HK * 64 + lane;
+        for (int m = 0; m < MT; ++m)
+          acc[0][m] = acc[1][m] = v4{T(0), T(0), T(0), T(0)};
+        const T *At = tr + 2 * set * MT * HK * 64 + lane;
 #pragma unroll
         for (int ks = 0; ks < HK; ++ks) {
-          const T v = harm_fma(half2, vb[w][ks], va[w][ks]);
+          const T f = harm_fma(half2, vb[w][ks], va[w][ks]);
+          const T b = harm_fma(half2, wb[w][ks], wa[w][ks]);
+          const T v[2] = {set ? f - b : f + b, set ? f + b : f - b};
 #pragma unroll
-          for (int m = 0; m < MT; ++m)
-            acc[m + ks % NA] =
-                M::mfma(At[(m * HK + ks) * 64], v, acc[m + ks % NA]);
+          for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+              acc[c][m] =
+                  M::mfma(At[((c * MT + m) * HK + ks) * 64], v[c], acc[c][m]);
         }
-        if (NA > 1) acc[0] += acc[NA - 1];
         if (row < nrow) {
 #pragma unroll
-          for (int m = 0; m < MT; ++m)
+          for (int c = 0; c < 2; ++c)
 #pragma unroll
-            for (uint32_t r = 0; r < 4; ++r) {
-              const uint32_t mode = 16 * m + M::row(g, r);
-              if (mode < MS) Gm[row * RS + mode * 16 + c16] = acc[m][r];
-            }
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+              for (uint32_t r = 0; r < 4; ++r) {
+                const uint32_t mode = 2 * (16 * m + M::row(g, r)) + c;
+                if (mode < MS) Gm[row * RS + mode * 16 + c16] = acc[c][m][r];
+              }
         }
       }
       harm_barrier();
@@ -1054,13 +1083,27 @@ __device__ __forceinline__ void harm_lr_body(
   }
 }
 
-// Waves per SIMD that the registers of the rows' values leave room for.
+// Classes of groups by the steps of four azimuths up to pi / 2, which bound the
+// rings too: rows per wave, and steps, of class c.
 template <typename T>
-constexpr int harm_lr_waves(int hk) {
-  return sizeof(T) == 4 ? (hk <= 8 ? 5 : hk <= 12 ? 3 : 2) : (hk <= 8 ? 3 : 2);
+constexpr int harm_lr_rows(int c) {
+  return sizeof(T) == 4 ? c + 1 : c == 1 ? 1 : 2;
 }
-template <typename T, int RW, int HK>
-__global__ __launch_bounds__(kHarmBlock, harm_lr_waves<T>(HK)) void harm_lr_kernel(
+constexpr int harm_lr_steps(int c) { return c == 1 ? 4 : c == 2 ? 6 : 9; }
+__host__ __device__ constexpr int harm_lr_class(uint32_t hk) {
+  return hk <= 4 ? 1 : hk <= 6 ? 2 : 3;
+}
+// Waves per SIMD the registers are held to: two workgroups per CU pay for the
+// spills of the mixed class 2 (181 to 118 us at 10,000 waters, 2.55 to 1.70 ms
+// at 1.0M charges) and the FP64 class 1 (1,288 to 1,162 us at 288,000
+// charges), not for those of the others (FP64 class 2 410 to 828 us).
+template <typename T>
+constexpr int harm_lr_waves(int c) {
+  return sizeof(T) == 4 ? (c == 1 ? 5 : c == 2 ? 4 : 2) : (c == 1 ? 4 : 2);
+}
+// C: the largest class of the plan's groups.
+template <typename T, int C>
+__global__ __launch_bounds__(kHarmBlock, harm_lr_waves<T>(C)) void harm_lr_kernel(
     HarmDev<T> H, uint32_t ncell, const T *__restrict__ R,
     T *__restrict__ coef) {
   extern __shared__ char harm_smem[];
@@ -1070,15 +1113,20 @@ __global__ __launch_bounds__(kHarmBlock, harm_lr_waves<T>(HK)) void harm_lr_kern
     return;
   const HarmRad rad = H.rad[unit];
   const HarmGroup gr = H.grp[rad.group];
-  // tiles of 16 orders of a set; steps of four azimuths over half a ring
-  constexpr int MM = sizeof(T) == 4 ? 3 : 4;
-  harm_switch<MM>((harm_mode_steps(rad.N) + 3) / 4, [&](auto mt) {
-    constexpr int MT = decltype(mt)::value;
-    if (gr.trigt_k <= HK - 3)
-      harm_lr_body<T, RW, HK - 3, MT>(H, ncell, rad, gr, tile, R, coef,
-                                      harm_smem);
-    else
-      harm_lr_body<T, RW, HK, MT>(H, ncell, rad, gr, tile, R, coef, harm_smem);
+  harm_switch<C>(harm_lr_class(gr.trigt_k), [&](auto cls) {
+    constexpr int c = decltype(cls)::value;
+    constexpr int RW = harm_lr_rows<T>(c), HK = harm_lr_steps(c);
+    constexpr int LK = HK - (HK > 8 ? 2 : 1);
+    // tiles of 16 orders of a set
+    harm_switch<2>((harm_order_steps(rad.N) + 3) / 4, [&](auto mt) {
+      constexpr int MT = decltype(mt)::value;
+      if (gr.trigt_k <= LK)
+        harm_lr_body<T, RW, LK, MT>(H, ncell, rad, gr, tile, R, coef,
+                                    harm_smem);
+      else
+        harm_lr_body<T, RW, HK, MT>(H, ncell, rad, gr, tile, R, coef,
+                                    harm_smem);
+    });
   });
 }
 
@@ -1305,18 +1353,18 @@ void prepare_harmonic(size_t lds_limit) {
   allow(harm_moments_kernel<double, 16>);
   allow(harm_moments_kernel<double, 24>);
   allow(harm_moments_kernel<double, 32>);
+  allow(harm_sf_kernel<float, 1>);
   allow(harm_sf_kernel<float, 2>);
   allow(harm_sf_kernel<float, 3>);
-  allow(harm_sf_kernel<float, 4>);
+  allow(harm_sf_kernel<double, 1>);
   allow(harm_sf_kernel<double, 2>);
   allow(harm_sf_kernel<double, 3>);
-  allow(harm_sf_kernel<double, 4>);
-  allow(harm_lr_kernel<float, 2, 8>);
-  allow(harm_lr_kernel<float, 3, 12>);
-  allow(harm_lr_kernel<float, 4, 16>);
-  allow(harm_lr_kernel<double, 1, 8>);
-  allow(harm_lr_kernel<double, 2, 12>);
-  allow(harm_lr_kernel<double, 2, 16>);
+  allow(harm_lr_kernel<float, 1>);
+  allow(harm_lr_kernel<float, 2>);
+  allow(harm_lr_kernel<float, 3>);
+  allow(harm_lr_kernel<double, 1>);
+  allow(harm_lr_kernel<double, 2>);
+  allow(harm_lr_kernel<double, 3>);
 }
 
 template <typename T>
@@ -1330,18 +1378,17 @@ size_t harm_lds_moments(uint32_t N, uint32_t ksteps) {
 }
 template <typename T>
 size_t harm_lds_sf(uint32_t N, uint32_t h) {
-  const size_t KS = ((N + 1) / 2 + 1) / 2;
-  return ((sizeof(T) == 4 ? 16 : 8) * (4 * KS * 16 + 8) +
-          ((h + 15) / 16) * KS * 64) *
+  const size_t KC = harm_order_steps(N), npt = (h / 2 + 16) / 16;
+  return ((sizeof(T) == 4 ? 16 : 8) * (128 * KC + 24) + 2 * npt * KC * 64) *
          sizeof(T);
 }
 template <typename T>
 size_t harm_lds_lr(uint32_t N, uint32_t h, uint32_t nring) {
-  const size_t KS = ((N + 1) / 2 + 1) / 2, MS = 4 * KS;
+  const size_t KC = harm_order_steps(N);
   const size_t lk = std::max<size_t>(4, (nring + 3) / 4);
-  const size_t hk = (h + 3) / 4, top = hk <= 8 ? 8 : hk <= 12 ? 12 : 16;
-  return ((sizeof(T) == 4 ? 4 : 2) * lk * (MS * 16 + 8) +
-          2 * ((MS + 15) / 16) * top * 64) *
+  const size_t top = harm_lr_steps(harm_lr_class((h / 2 + 4) / 4));
+  return ((sizeof(T) == 4 ? 4 : 2) * lk * (128 * KC + 8) +
+          4 * ((KC + 3) / 4) * top * 64) *
          sizeof(T);
 }
 template size_t harm_lds_moments<float>(uint32_t, uint32_t);
@@ -1387,12 +1434,12 @@ void harm_sf(const HarmPlanDev &P, const HarmDev<T> &H, const void *atoms,
         static_cast<const typename HarmRecord<T>::type *>(atoms), start, k64,
         g.ny, g.nz, g.h, g.ncell, coef, outside, S);
   };
-  if (P.hsteps <= 8)
+  if (P.hsteps <= 4)
+    go(harm_sf_kernel<T, 1>);
+  else if (P.hsteps <= 8)
     go(harm_sf_kernel<T, 2>);
-  else if (P.hsteps <= 12)
-    go(harm_sf_kernel<T, 3>);
   else
-    go(harm_sf_kernel<T, 4>);
+    go(harm_sf_kernel<T, 3>);
 }
 
 template <typename T>
@@ -1403,14 +1450,13 @@ void harm_lr(const HarmPlanDev &P, const HarmDev<T> &H, const GridShape &g,
     kernel<<<harm_grid(nt, H.nrad), kHarmBlock, P.lds_lr, s>>>(H, g.ncell, R,
                                                                coef);
   };
-  // rows per wave and steps of four azimuths over half a ring
-  constexpr bool F = sizeof(T) == 4;
-  if (P.hsteps <= 8)
-    go(harm_lr_kernel<T, F ? 2 : 1, 8>);
-  else if (P.hsteps <= 12)
-    go(harm_lr_kernel<T, F ? 3 : 2, 12>);
+  const int c = harm_lr_class(P.hsteps);
+  if (c == 1)
+    go(harm_lr_kernel<T, 1>);
+  else if (c == 2)
+    go(harm_lr_kernel<T, 2>);
   else
-    go(harm_lr_kernel<T, F ? 4 : 2, 16>);
+    go(harm_lr_kernel<T, 3>);
   const uint32_t nw = nt * H.npair;
   harm_radial_kernel<T, true>
       <<<(nw + 3) / 4, 256, 0, s>>>(H, g.ncell, nw, coef, mom);

@@ -81,8 +81,10 @@ struct HarmGroup {
   uint32_t mup;        // first (mu, parity) entry of HarmDev::mup
   uint32_t leg, leg_n;    // Legendre, degrees -> rings: per ring tile of 16
   uint32_t legt, legt_k;  // rings -> degrees; steps over the rings
-  uint32_t trig, trig_k;  // Fourier, orders -> azimuths: [tile][set][step]
-  uint32_t trigt, trigt_m, trigt_k;  // azimuths -> orders: [set][tile][step]
+  // Fourier, azimuths up to pi / 2: orders -> azimuths [tile][cs][set][step]
+  // (cs 0: cosines, 1: sines), trig_t tiles, and back [set][cs][tile][step]
+  uint32_t trig, trig_k, trig_t;
+  uint32_t trigt, trigt_m, trigt_k;
 };
 
 // directions of a group

@@ -269,6 +269,7 @@ inline HarmTables plan_harmonic(const NodeTable &nodes, double h,
     T.lrow.push_back(r);
   }
   // Legendre functions on the rings and Fourier matrices
+  uint32_t hmax = 0;  // (one launch for all groups)
   for (size_t g = 0; g < ng; ++g) {
     dev::HarmGroup &G = T.grp[g];
     G.mup = static_cast<uint32_t>(T.mup.size());
@@ -335,42 +336,47 @@ inline HarmTables plan_harmonic(const NodeTable &nodes, double h,
       ct[k] = static_cast<double>(std::cos(kPi * k / G.h));
       sn[k] = static_cast<double>(std::sin(kPi * k / G.h));
     }
-    // mode 2 m + cs of a set: cosine or sine of order mu = 2 m + set
-    auto mode = [&](uint32_t k, uint32_t md, uint32_t set) {
-      const uint32_t mu = 2 * (md / 2) + set;
-      if (k >= G.h || mu >= G.N) return 0.0;
+    // cosine or sine of order 2 m + set at azimuth pi k / h, k <= h / 2
+    auto mode = [&](uint32_t k, uint32_t m, uint32_t set, uint32_t cs) {
+      const uint32_t mu = 2 * m + set;
+      if (2 * k > G.h || mu >= G.N) return 0.0;
       const uint32_t a = mu * k % (2 * G.h);
-      return md % 2 ? sn[a] : ct[a];
+      return cs ? sn[a] : ct[a];
     };
-    const uint32_t KS = ((G.N + 1) / 2 + 1) / 2, MS = 4 * KS;
     G.trig = static_cast<uint32_t>(T.trig.size() / 64);
-    G.trig_k = KS;
-    for (uint32_t pt = 0; pt < (G.h + 15) / 16; ++pt)
-      for (uint32_t set = 0; set < 2; ++set)
-        for (uint32_t k = 0; k < KS; ++k)
-          for (uint32_t a = 0; a < 64; ++a)
-            T.trig.push_back(mode(16 * pt + a % 16, 4 * k + a / 16, set));
+    G.trig_k = ((G.N + 1) / 2 + 3) / 4;
+    G.trig_t = (G.h / 2 + 16) / 16;
+    for (uint32_t pt = 0; pt < G.trig_t; ++pt)
+      for (uint32_t cs = 0; cs < 2; ++cs)
+        for (uint32_t set = 0; set < 2; ++set)
+          for (uint32_t k = 0; k < G.trig_k; ++k)
+            for (uint32_t a = 0; a < 64; ++a)
+              T.trig.push_back(
+                  mode(16 * pt + a % 16, 4 * k + a / 16, set, cs));
     G.trigt = static_cast<uint32_t>(T.trigt.size() / 64);
-    G.trigt_m = (MS + 15) / 16;
-    G.trigt_k = (G.h + 3) / 4;
+    G.trigt_m = (G.trig_k + 3) / 4;
+    G.trigt_k = (G.h / 2 + 4) / 4;
     T.hsteps = std::max(T.hsteps, G.trigt_k);
+    hmax = std::max(hmax, G.h);
     for (uint32_t set = 0; set < 2; ++set)
-      for (uint32_t mt = 0; mt < G.trigt_m; ++mt)
-        for (uint32_t k = 0; k < G.trigt_k; ++k)
-          for (uint32_t a = 0; a < 64; ++a)
-            T.trigt.push_back(mode(4 * k + a / 16, 16 * mt + a % 16, set));
+      for (uint32_t cs = 0; cs < 2; ++cs)
+        for (uint32_t mt = 0; mt < G.trigt_m; ++mt)
+          for (uint32_t k = 0; k < G.trigt_k; ++k)
+            for (uint32_t a = 0; a < 64; ++a)
+              T.trigt.push_back(
+                  mode(4 * k + a / 16, 16 * mt + a % 16, set, cs));
   }
   for (uint32_t i = 0; i < nrad; ++i) {
     const dev::HarmGroup &G = T.grp[T.rad[i].group];
     for (uint32_t rt = 0; rt < (G.nring + 15) / 16; ++rt)
       T.unit.push_back(make_uint2(i, rt));
     T.lds_sf = std::max(T.lds_sf, single
-                                      ? dev::harm_lds_sf<float>(T.rad[i].N, G.h)
-                                      : dev::harm_lds_sf<double>(T.rad[i].N, G.h));
+                                      ? dev::harm_lds_sf<float>(T.rad[i].N, hmax)
+                                      : dev::harm_lds_sf<double>(T.rad[i].N, hmax));
     T.lds_lr = std::max(
         T.lds_lr, single
-                      ? dev::harm_lds_lr<float>(T.rad[i].N, G.h, G.nring)
-                      : dev::harm_lds_lr<double>(T.rad[i].N, G.h, G.nring));
+                      ? dev::harm_lds_lr<float>(T.rad[i].N, hmax, G.nring)
+                      : dev::harm_lds_lr<double>(T.rad[i].N, hmax, G.nring));
   }
   // the kernels load whole groups of steps
   T.leg.resize(T.leg.size() + 8 * 64, 0.0);

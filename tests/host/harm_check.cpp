@@ -111,12 +111,18 @@ int main(int argc, char **argv) {
             for (uint32_t par = 0; par < 2; ++par) {
               const uint32_t l0 = m + ((m ^ par) & 1u);
               const uint2 o = T.mup[G.mup + 2 * m + par];
-              const size_t md = 2 * (m / 2), ks = G.trig_k;
-              const size_t ft =
-                  G.trig + (static_cast<size_t>(k / 16) * 2 + m % 2) * ks;
+              // azimuths past pi / 2 through the one at pi - phi: the cosine
+              // changes sign for odd orders, the sine for even ones
+              const uint32_t kk2 = 2 * k > G.h ? G.h - k : k;
+              const double sg[2] = {kk2 != k && m % 2 ? -1.0 : 1.0,
+                                    kk2 != k && m % 2 == 0 ? -1.0 : 1.0};
               auto mode = [&](size_t c) {
-                return T.trig[(ft + (md + c) / 4) * 64 + ((md + c) % 4) * 16 +
-                              k % 16];
+                const size_t ft =
+                    G.trig +
+                    ((static_cast<size_t>(kk2 / 16) * 2 + c) * 2 + m % 2) *
+                        G.trig_k;
+                return sg[c] * T.trig[(ft + m / 2 / 4) * 64 +
+                                      (m / 2 % 4) * 16 + kk2 % 16];
               };
               const double az = mode(0) * xc[m] + mode(1) * xs[m];
               double sum = 0.0;
