@@ -390,6 +390,9 @@ struct glst_engine {
   bool harmonic() const {
     return harm.ok() && sf_cheb && lr_atom_groups && rmt_shape != 2;
   }
+  // The path of the S at hand: the stages after calc_sf follow it, also where
+  // an option has changed since.
+  bool expanded() const { return field_layout == 1; }
   // Clears S when its layout changes: the kernels never write the slots of
   // the padded nodes.
   void set_field_layout() {
@@ -436,16 +439,16 @@ struct glst_engine {
 
   void sum_rmt_sf() {
     if (!has_lr || Kp == 0) return;
-    if (!sf_done || field_layout != (harmonic() ? 1 : 0))
+    if (!sf_done)
       throw StateError("sum_rmt_sf called before calc_sf");
     Scope sc(timer, "rmt", stream);
-    const bool nm = harmonic();
+    const bool nm = expanded();
     const double4 *kn = nm ? harm.k64 : k64.as<double4>();
-    if (rmt_mfma_path()) {
+    if (rmt_mfma_path(nm)) {
       dev::rmt_mfma(S.as<void>(), kn, group.as<uint32_t>(),
                     r_in.as<uint32_t>(), r_out.as<uint32_t>(), Kp, grid,
                     lds_limit, R.as<void>(), stream, 0, 0xffffffffu, nm);
-    } else if (rmt_wave_path()) {
+    } else if (rmt_wave_path(nm)) {
       dev::rmt_wave(S.as<void>(), kn, group.as<uint32_t>(),
                     r_in.as<uint32_t>(), r_out.as<uint32_t>(), Kp, grid,
                     R.as<void>(), stream, 0, 0xffffffffu, nm);
@@ -469,7 +472,7 @@ struct glst_engine {
 
   void calc_lr_ef() {
     if (!has_lr || Kp == 0 || natom == 0) return;
-    if (!rmt_done || field_layout != (harmonic() ? 1 : 0))
+    if (!rmt_done)
       throw StateError("calc_lr_ef called before sum_rmt_sf");
     lr_partials();
     reduce(false);
@@ -480,7 +483,7 @@ struct glst_engine {
   void reduce(bool with_near) {
     Scope sc(timer, "lr_reduce", stream);
     const bool lr = has_lr && Kp > 0;
-    dev::lr_reduce(partial.as<double4>(), lr ? (harmonic() ? 1u : nsplit) : 0,
+    dev::lr_reduce(partial.as<double4>(), lr ? (expanded() ? 1u : nsplit) : 0,
                    natom,
                    with_near ? near4.as<double4>() : nullptr, fx.as<double>(),
                    fy.as<double>(), fz.as<double>(), en.as<double>(), stream);
@@ -496,7 +499,7 @@ struct glst_engine {
 
   void lr_partials() {
     Scope sc(timer, "lr", stream);
-    if (harmonic()) {
+    if (expanded()) {
       auto run = [&](auto t) {
         using T = decltype(t);
         dev::harm_lr<T>(harm_plan, harm.dev<T>(), grid, R.as<T>(),
@@ -566,6 +569,7 @@ struct glst_engine {
     rmt_need = std::move(P.rmt_need);
   }
   void sf_stage() {
+    set_field_layout();
     if (!pipelined()) {
       calc_sf();
       return;
@@ -693,18 +697,19 @@ struct glst_engine {
                                     1) == 0;
   }
   // shell sums on the matrix cores (CT = float, nx and ny up to 16)
-  bool rmt_mfma_path() const {
+  bool rmt_mfma_path(bool nm = false) const {
     const bool want =
         rmt_shape == 3 ||
         (rmt_shape == 4 && grid.nx * grid.ny * 2 >= dev::kRmtMfmaMaxXY *
                                                         dev::kRmtMfmaMaxXY);
     return want && mixed() &&
-           dev::rmt_mfma_nodes(grid, lds_limit, harmonic()) > 0;
+           dev::rmt_mfma_nodes(grid, lds_limit, nm) > 0;
   }
   // shell sums as window sums of small grids (CT = float, every dimension
   // up to 8)
-  bool rmt_wave_path() const {
-    const bool want = rmt_shape == 5 || (rmt_shape == 4 && !rmt_mfma_path());
+  bool rmt_wave_path(bool nm = false) const {
+    const bool want =
+        rmt_shape == 5 || (rmt_shape == 4 && !rmt_mfma_path(nm));
     return want && mixed() && dev::rmt_wave_fits(grid);
   }
 
@@ -894,7 +899,7 @@ struct glst_engine {
   void field_to_host(const DeviceBuffer &buf, bool single, uint32_t fstride,
                      bool tiled, double *re, double *im) {
     const uint32_t ncp = dev::harm_row(grid.ncell);
-    const bool nm = harmonic();
+    const bool nm = expanded();
     const size_t n = static_cast<size_t>(nm ? ncp : grid.ncell) * Kp;
     std::vector<double> tmp(2 * n);
     if (single) {
@@ -1203,13 +1208,13 @@ glst_status_t glst_get_sf(glst_handle_t h, double *re, double *im) {
   NEED_HANDLE(h);
   return guarded(h, [&] {
     if (!h->has_lr || h->K == 0) return;
-    if (!h->sf_done || h->field_layout != (h->harmonic() ? 1 : 0))
+    if (!h->sf_done)
       throw StateError("glst_get_sf: no structure factors");
     const size_t n = static_cast<size_t>(h->grid.ncell) * h->K;
     std::vector<double> r(n), i(n);
     h->field_to_host(h->S, h->mixed(), 2, true, r.data(), i.data());
     const auto &g = h->grid;
-    if (h->mixed() || h->harmonic()) {
+    if (h->mixed() || h->expanded()) {
       // the field holds cell-local sums; apply exp(-i k.c)
       for (uint32_t c = 0; c < g.ncell; ++c) {
         const uint32_t x = c / (g.ny * g.nz), y = (c / g.nz) % g.ny,
@@ -1248,12 +1253,12 @@ glst_status_t glst_get_rmt(glst_handle_t h, double *re, double *im) {
   NEED_HANDLE(h);
   return guarded(h, [&] {
     if (!h->has_lr || h->K == 0) return;
-    if (!h->rmt_done || h->field_layout != (h->harmonic() ? 1 : 0))
+    if (!h->rmt_done)
       throw StateError("glst_get_rmt: no remote sums");
     const size_t n = static_cast<size_t>(h->grid.ncell) * h->K;
     std::vector<double> r(n), i(n);
     h->field_to_host(h->R, h->mixed(), 2, false, r.data(), i.data());
-    const bool polar = !h->harmonic();
+    const bool polar = !h->expanded();
     if (h->mixed() || !polar) {
       // the stored (kappa |V|, arg V / 2 pi) back to V = exp(+i k.c) R_c(k)
       // (node-major fields hold V itself), then undo the exp(+i k.c) factor

@@ -40,6 +40,8 @@ def _far(h, box, tol, ct, direct, torch, g):
         f.set_option("lr_atom_groups", 0)
     f.assign_atoms(*d)
     f.calc_sf()
+    if not direct:
+        f.set_option("sf_cheb", 0)  # the later stages follow the S at hand
     s = f.sf()
     f.sum_rmt_sf()
     f.calc_lr_ef()
