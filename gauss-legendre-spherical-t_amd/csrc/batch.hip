@@ -232,6 +232,8 @@ size_t ShapeTables::device_bytes() const {
 #define GLST_BATCH_RMT_LDS_DIV 4
 #endif
 constexpr size_t kBatchRmtLdsDiv = GLST_BATCH_RMT_LDS_DIV;
+// an expanded system has at least this part of the batch's pairs
+constexpr double kHarmShare = 200.0;
 
 BatchLayout pack_batch(int ct,
                        const std::vector<std::shared_ptr<const BatchSystem>> &cs,
@@ -250,6 +252,9 @@ BatchLayout pack_batch(int ct,
       tiles ? static_cast<uint32_t>(
                   std::max<uint64_t>(1, (lr_blocks + tiles - 1) / tiles))
             : 1;
+  double pairs = 0.0;
+  for (const auto &c : cs)
+    if (c->su().has_lr) pairs += static_cast<double>(c->natom) * c->su().K;
   std::vector<SplitPlan> splits(nsys);
   std::vector<uint32_t> task_first(nsys, 0);
   uint32_t split_base = 0;
@@ -287,10 +292,15 @@ BatchLayout pack_batch(int ct,
     d.partial0 = B.partial;
     d.ag0 = static_cast<uint32_t>(B.nag);
     d.agtile = 0;
-    // expanded far field: the rule of a handle (harm_worth)
+    // expanded far field: the rule of a handle (harm_worth), and no small part
+    // of the batch, whose launches per stage already fill the device (512
+    // mixed systems of 100 to 10,000 waters: 94.2 ms with all that a handle
+    // would expand, 86.4 with those of 8e8 pairs, 92.4 with none; 64 such
+    // systems 13.5, 13.4 and 16.1 ms; 16 systems 2.9, 4.2 and 4.7 ms)
     HarmSystem hs{s, 0, {}};
     if (cheb && lr && !cs[s]->direct &&
-        harm_worth(na, u.K, ct == GLST_CT_FLOAT)) {
+        harm_worth(na, u.K, ct == GLST_CT_FLOAT) &&
+        static_cast<double>(na) * u.K * kHarmShare >= pairs) {
       const HarmTables &t = cs[s]->shape->harm();
       if (t.ok)
         hs.plan = harm_fit(t, ct == GLST_CT_FLOAT, lds_limit, na, d.ncell);
