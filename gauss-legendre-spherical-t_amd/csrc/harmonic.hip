@@ -1477,8 +1477,9 @@ void harm_eval(const HarmPlanDev &P, const HarmDev<T> &H, const void *atoms,
   };
   // W MO >= N (N <= 8 ps).  FP32: four waves of twice the orders form the
   // radial values half as often (400 against 439 us at 3,375 cells), eight
-  // fill the device on small grids (69 against 102 us at 64 cells)
-  if (sizeof(T) == 4 && g.ncell * P.nset >= 512) {
+  // fill the device on smaller grids (69 against 102 us at 64 cells, 87
+  // against 106 at 512, two workgroups each)
+  if (sizeof(T) == 4 && g.ncell * P.nset >= 2048) {
     harm_host_switch<5>(ps, [&](auto k) {
       constexpr int PM = decltype(k)::value;
       if (H.N <= 8 * PM - 4)

@@ -23,9 +23,10 @@ constexpr double kHarmEps64 = 1e-15;
 // Systems with fewer (atom, node) pairs keep the direct sums: those are the
 // direct sums' work, while the passes here take 0.2 (mixed) to 0.5 ms (FP64)
 // however small the grid.  Measured in us per step, expansion against direct
-// sums: mixed 1,000 waters at tol 1e-5 (1.7e8 pairs) 350 to 333, 3,300 at 1e-4
-// (2.5e8) 279 to 317, 1,000 at 1e-6 (4e8) 479 to 518; FP64 3,300 at 1e-4 542
-// to 526, 5,500 at 1e-4 (4e8) 835 to 859, 1,000 at 1e-6 1,259 to 1,393.
+// sums: mixed 1,000 waters at tol 1e-5 (1.7e8 pairs) 334 to 333, 3,300 at 1e-4
+// (2.5e8) 272 to 317, 1,000 at 1e-6 (4e8) 461 to 517; FP64 1,000 at 1e-5 725
+// to 749 but 3,300 at 1e-4 525 to 528 and 1,800 at 1e-4 (1.3e8) 479 to 385,
+// 5,500 at 1e-4 (4e8) 828 to 858, 1,000 at 1e-6 1,213 to 1,403.
 constexpr double kHarmPairs32 = 2e8, kHarmPairs64 = 3e8;
 
 // j_0(z) .. j_{n-1}(z), z > 0: Miller's backward recurrence j_{m-1} =
