@@ -130,6 +130,18 @@ __device__ __forceinline__ HarmCentre harm_centre(uint32_t cell, uint32_t ny,
   return c;
 }
 
+// One wave: the atoms of [a0, a0 + na) outside the ball, in order, into list[1]
+// ...; their number into list[0].  na <= 64.
+template <typename T>
+__device__ __forceinline__ void harm_list_outside(
+    const HarmDev<T> &H, const typename HarmRecord<T>::type *atoms, uint32_t a0,
+    uint32_t na, const HarmCentre &cc, uint32_t *list) {
+  const uint32_t lane = threadIdx.x & 63u;
+  const bool out = lane < na && harm_atom(H, atoms, a0 + lane, cc).out;
+  const unsigned long long mask = __ballot(out);
+  if (out) list[1 + __popcll(mask & ((1ull << lane) - 1))] = a0 + lane;
+  if (lane == 0) list[0] = static_cast<uint32_t>(__popcll(mask));
+}
 // Workgroup barrier for data in LDS: waits for the LDS operations only, so that
 // loads issued ahead and stores stay in flight (__syncthreads drains them).
 __device__ __forceinline__ void harm_barrier() {
@@ -839,32 +851,51 @@ __device__ __forceinline__ void harm_sf_body(
   for (uint32_t c = 0; c < kHarmCells; ++c)
     if (cell0 + c < ncell) any |= outside[cell0 + c];
   if (!any) return;
-  // atoms outside the unit ball: their terms one by one
-  __syncthreads();
+  // atoms outside the unit ball: their terms one by one, 64 atoms of every cell
+  // at a time (wave c lists those of cell c)
+  uint32_t *list = reinterpret_cast<uint32_t *>(smem);
   const uint32_t d0 = rt ? 32 * gr.h * rt - (gr.equator ? gr.h : 0u) : 0u;
   const uint32_t d1 =
       32 * gr.h * (rt + 1) - (gr.equator ? gr.h : 0u) < nd
           ? 32 * gr.h * (rt + 1) - (gr.equator ? gr.h : 0u)
           : nd;
-  for (uint32_t e = tid; e < (d1 - d0) * kHarmCells; e += kHarmBlock) {
-    const uint32_t cell = cell0 + (e & (kHarmCells - 1));
-    if (cell >= ncell || !outside[cell]) continue;
-    const uint32_t node = gr.node0 + rad.idx * nd + d0 + e / kHarmCells;
-    const double4 k = k64[node];
-    const HarmCentre cc = harm_centre(cell, ny, nz, h);
-    double re = 0.0, im = 0.0;
-    for (uint32_t j = start[cell]; j < start[cell + 1]; ++j) {
-      if (harm_atom(H, atoms, j, cc).out) {
-        const HarmOffset d = harm_offset(atoms, j, cc);
+  uint32_t most = 0;
+  for (uint32_t c = 0; c < kHarmCells; ++c)
+    if (cell0 + c < ncell && outside[cell0 + c]) {
+      const uint32_t n = start[cell0 + c + 1] - start[cell0 + c];
+      most = n > most ? n : most;
+    }
+  for (uint32_t p0 = 0; p0 < most; p0 += 64) {
+    __syncthreads();
+    for (uint32_t c = wave; c < kHarmCells; c += NW) {
+      uint32_t n = 0;
+      if (cell0 + c < ncell && outside[cell0 + c])
+        n = start[cell0 + c + 1] - start[cell0 + c];
+      n = n > p0 ? n - p0 : 0u;
+      harm_list_outside(H, atoms, n ? start[cell0 + c] + p0 : 0u,
+                        n < 64 ? n : 64u, harm_centre(cell0 + c, ny, nz, h),
+                        list + 65 * c);
+    }
+    __syncthreads();
+    for (uint32_t e = tid; e < (d1 - d0) * kHarmCells; e += kHarmBlock) {
+      const uint32_t c = e & (kHarmCells - 1), cell = cell0 + c;
+      const uint32_t n = list[65 * c];
+      if (n == 0) continue;
+      const uint32_t node = gr.node0 + rad.idx * nd + d0 + e / kHarmCells;
+      const double4 k = k64[node];
+      const HarmCentre cc = harm_centre(cell, ny, nz, h);
+      double re = 0.0, im = 0.0;
+      for (uint32_t q = 0; q < n; ++q) {
+        const HarmOffset d = harm_offset(atoms, list[65 * c + 1 + q], cc);
         const double ph = k.x * d.x + k.y * d.y + k.z * d.z;
         re += d.q * cos(ph);
         im -= d.q * sin(ph);
       }
+      T *sr = S + harm_slot<T>(node, cell, 0, ncp);
+      T *si = S + harm_slot<T>(node, cell, 1, ncp);
+      *sr += static_cast<T>(re);
+      *si += static_cast<T>(im);
     }
-    T *sr = S + harm_slot<T>(node, cell, 0, ncp);
-    T *si = S + harm_slot<T>(node, cell, 1, ncp);
-    *sr += static_cast<T>(re);
-    *si += static_cast<T>(im);
   }
 }
 
@@ -1133,39 +1164,86 @@ __global__ __launch_bounds__(kHarmBlock, harm_lr_waves<T>(C)) void harm_lr_kerne
 // ---------------------------------------------------------------------------
 // coefficients -> energies and forces
 
-// Fields of an atom outside the unit ball: the direct sum over the nodes.
+// Fields of the atoms outside their cell's ball (cells without any return at
+// once): the direct sums over the nodes, four atoms and four nodes at a time
+// (the nodes' remote sums lie rows apart; with one of each at a time, inside the
+// evaluation, an FP64 step of 2,000 waters at rcut 8, tol 1e-6, with a molecule
+// across the box's corner took 4.60 ms instead of 2.82).
+constexpr uint32_t kHarmOutBlock = 512;
 template <typename T>
-__device__ void harm_outside_eval(const HarmOffset &a, uint32_t cell, const double4 *k64,
-                                  uint32_t K, const T *R, uint32_t ncp,
-                                  double *red, double4 *out) {
-  double e = 0.0, fx = 0.0, fy = 0.0, fz = 0.0;
-  for (uint32_t n = threadIdx.x; n < K; n += blockDim.x) {
-    const double4 k = k64[n];
-    const double ph = k.x * a.x + k.y * a.y + k.z * a.z;
-    const double vr = R[harm_slot<T>(n, cell, 0, ncp)];
-    const double vi = R[harm_slot<T>(n, cell, 1, ncp)];
-    const double c = cos(ph), s = sin(ph);
-    const double b = c * vi + s * vr;
-    e += c * vr - s * vi;
-    fx += k.x * b;
-    fy += k.y * b;
-    fz += k.z * b;
-  }
-  double v[4] = {fx, fy, fz, e};
-  for (int d = 0; d < 4; ++d) {
-    harm_barrier();
-    red[threadIdx.x] = v[d];
-    harm_barrier();
-    for (uint32_t o = 256; o > 0; o >>= 1) {
-      if (threadIdx.x < o && threadIdx.x + o < blockDim.x)
-        red[threadIdx.x] += red[threadIdx.x + o];
-      harm_barrier();
+__global__ __launch_bounds__(kHarmOutBlock) void harm_outside_kernel(
+    HarmDev<T> H, const typename HarmRecord<T>::type *__restrict__ atoms,
+    const uint32_t *__restrict__ start, const double4 *__restrict__ k64,
+    uint32_t K, uint32_t ny, uint32_t nz, double h, uint32_t ncell,
+    const T *__restrict__ R, const uint32_t *__restrict__ outside,
+    double4 *__restrict__ out) {
+  const uint32_t cell = blockIdx.x;
+  if (!outside[cell]) return;
+  __shared__ uint32_t list[65];
+  __shared__ double red[kHarmOutBlock / 64][16];
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+  const uint32_t ncp = harm_row(ncell);
+  const uint32_t a0 = start[cell], na = start[cell + 1] - a0;
+  const HarmCentre cc = harm_centre(cell, ny, nz, h);
+  for (uint32_t p0 = 0; p0 < na; p0 += 64) {
+    __syncthreads();
+    if (wave == 0)
+      harm_list_outside(H, atoms, a0 + p0, na - p0 < 64 ? na - p0 : 64u, cc,
+                        list);
+    __syncthreads();
+    const uint32_t cnt = list[0];
+    for (uint32_t q0 = 0; q0 < cnt; q0 += 4) {
+      HarmOffset a[4];
+      double v[16];
+#pragma unroll
+      for (uint32_t q = 0; q < 4; ++q)
+        a[q] = harm_offset(atoms, list[1 + (q0 + q < cnt ? q0 + q : q0)], cc);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) v[i] = 0.0;
+      for (uint32_t n0 = tid; n0 < K; n0 += 4 * kHarmOutBlock) {
+        double4 k[4];
+        double vr[4], vi[4];
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) {
+          const uint32_t n = n0 + u * kHarmOutBlock;
+          const uint32_t m = n < K ? n : n0;
+          k[u] = k64[m];
+          vr[u] = R[harm_slot<T>(m, cell, 0, ncp)];
+          vi[u] = R[harm_slot<T>(m, cell, 1, ncp)];
+          if (n >= K) vr[u] = vi[u] = 0.0;
+        }
+#pragma unroll
+        for (uint32_t q = 0; q < 4; ++q) {
+          if (q0 + q >= cnt) break;  // uniform
+#pragma unroll
+          for (uint32_t u = 0; u < 4; ++u) {
+            const double ph =
+                k[u].x * a[q].x + k[u].y * a[q].y + k[u].z * a[q].z;
+            const double c = cos(ph), s = sin(ph);
+            const double b = c * vi[u] + s * vr[u];
+            v[4 * q] += k[u].x * b;
+            v[4 * q + 1] += k[u].y * b;
+            v[4 * q + 2] += k[u].z * b;
+            v[4 * q + 3] += c * vr[u] - s * vi[u];
+          }
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        for (int o = 32; o > 0; o >>= 1) v[i] += __shfl_xor(v[i], o, 64);
+        if (lane == 0) red[wave][i] = v[i];
+      }
+      __syncthreads();
+      if (tid < 4 && q0 + tid < cnt) {
+        double t[4] = {0.0, 0.0, 0.0, 0.0};
+        for (uint32_t w = 0; w < kHarmOutBlock / 64; ++w)
+          for (uint32_t d = 0; d < 4; ++d) t[d] += red[w][4 * tid + d];
+        const uint32_t i = list[1 + q0 + tid];
+        const double q = harm_offset(atoms, i, cc).q;
+        out[i] = make_double4(q * t[0], q * t[1], q * t[2], q * t[3]);
+      }
+      __syncthreads();
     }
-    v[d] = red[0];
-  }
-  harm_barrier();
-  if (threadIdx.x == 0) {
-    *out = make_double4(a.q * v[0], a.q * v[1], a.q * v[2], a.q * v[3]);
   }
 }
 
@@ -1307,10 +1385,8 @@ __device__ __forceinline__ void harm_eval_body(
 template <typename T, int W, int MO, int PM>
 __global__ __launch_bounds__(64 * W) void harm_eval_kernel(
     HarmDev<T> H, const typename HarmRecord<T>::type *__restrict__ atoms,
-    const uint32_t *__restrict__ start, const double4 *__restrict__ k64,
-    uint32_t K, uint32_t ny, uint32_t nz, double h, uint32_t ncell,
-    uint32_t nset, const T *__restrict__ mom, const T *__restrict__ R,
-    const uint32_t *__restrict__ outside, double4 *__restrict__ out) {
+    const uint32_t *__restrict__ start, uint32_t ny, uint32_t nz, double h,
+    uint32_t nset, const T *__restrict__ mom, double4 *__restrict__ out) {
   __shared__ double red[W * 256];
   const uint32_t nb = gridDim.x, b = blockIdx.x;
   const uint32_t q = nb >> 3, r = nb & 7u, x = b & 7u;
@@ -1329,11 +1405,6 @@ __global__ __launch_bounds__(64 * W) void harm_eval_kernel(
   for (uint32_t p0 = 64 * set; p0 < na; p0 += 64 * nset) {
     const uint32_t cnt = na - p0 < 64 ? na - p0 : 64u;
     harm_eval_body<T, W, MO, PM>(H, atoms, a0 + p0, cnt, cc, U, out, red);
-    if (outside[cell])  // uniform; the same wave stores again
-      for (uint32_t i = a0 + p0; i < a0 + p0 + cnt; ++i)
-        if (harm_atom(H, atoms, i, cc).out)
-          harm_outside_eval<T>(harm_offset(atoms, i, cc), cell, k64, K, R,
-                               harm_row(ncell), red, out + i);
   }
   asm volatile("" ::"v"(touch[0]), "v"(touch[1]));
 }
@@ -1467,13 +1538,13 @@ void harm_eval(const HarmPlanDev &P, const HarmDev<T> &H, const void *atoms,
                const uint32_t *start, const double4 *k64, uint32_t K,
                const GridShape &g, const T *mom, const T *R,
                const uint32_t *outside, double4 *out, hipStream_t s) {
+  auto *at = static_cast<const typename HarmRecord<T>::type *>(atoms);
   const uint32_t ps = harm_psteps(0, H.N);
   auto go = [&](auto waves, auto orders, auto steps) {
     constexpr int W = decltype(waves)::value, MO = decltype(orders)::value;
     harm_eval_kernel<T, W, MO, decltype(steps)::value>
         <<<g.ncell * P.nset, 64 * W, 0, s>>>(
-            H, static_cast<const typename HarmRecord<T>::type *>(atoms), start,
-            k64, K, g.ny, g.nz, g.h, g.ncell, P.nset, mom, R, outside, out);
+            H, at, start, g.ny, g.nz, g.h, P.nset, mom, out);
   };
   // W MO >= N (N <= 8 ps).  FP32: four waves of twice the orders form the
   // radial values half as often (400 against 439 us at 3,375 cells), eight
@@ -1491,6 +1562,8 @@ void harm_eval(const HarmPlanDev &P, const HarmDev<T> &H, const void *atoms,
     harm_host_switch<sizeof(T) == 4 ? 5 : 7>(
         ps, [&](auto k) { go(HarmInt<8>{}, k, k); });
   }
+  harm_outside_kernel<T><<<g.ncell, kHarmOutBlock, 0, s>>>(
+      H, at, start, k64, K, g.ny, g.nz, g.h, g.ncell, R, outside, out);
 }
 
 #define GLST_HARM(T)                                                          \
