@@ -10,7 +10,7 @@ synchronisation.
 
 Prints ONE JSON line: atom-steps/s of the mixed FP32/FP64 path (value), the
 plain FP64 path beside it, the relative force error of both against the
-direct FP64 all-pairs sum, the roofline of the dominant kernel (HIP events on
+direct FP64 all-pairs sum, the roofline of the back-projection (HIP events on
 the handle's stream), a CPU baseline (the oracle's FP64 restatement of the
 reference path, one full step on the host cores), the served p50/p99 latency
 of the continuous-batching server under Poisson arrivals, the throughput
@@ -37,8 +37,6 @@ NWATER, BOX, RCUT, TOL, SEED = 96000, 142.0, 10.0, 1e-4, 1
 # an order at an accidental zero of its error for these cell edges.
 SERVE_RCUT, SERVE_TOL = 9.0, 2e-5
 ERR_BAR = 1e-5  # the metric's relative force error bar
-PEAK_FP32_VALU_TFLOPS = 157.3   # MI355X published FP32 vector peak
-PEAK_FP64_VALU_TFLOPS = 78.6    # MI355X published FP64 vector peak
 PEAK_HBM_GBS = 8000.0
 STAGES = ["bin", "sort", "sf", "rmt", "lr", "lr_reduce", "sr"]
 # Schedules (overlap_near, lr_blocks, rmt_shape, pipeline, graph) the
@@ -536,59 +534,33 @@ def main():
     log(f"relative force error vs direct FP64 sum: mixed {err_mixed:.3e} "
         f"fp64 {err_fp64:.3e}")
 
-    # Roofline of the dominant kernel, the back-projection (calc_lr_ef:
-    # lr_ag_kernel<NR> over atom groups, one launch per alpha group; avg_ms
-    # is the sum of the group launches of one step, HIP events on the
-    # handle's stream around them, from the steps run one stage after
-    # another).
-    # Algorithmic work: 20 flops (sin and cos counted as one each) per
-    # (atom, node) pair, the count of the reference's per-pair formulation,
-    # over the K nodes of the cubature (the table's padding to a multiple of
-    # 256 nodes is never visited).
+    # Roofline of the back-projection (calc_lr_ef through the harmonic
+    # expansion: harm_lr, harm_radial and harm_eval; avg_ms is their sum in one
+    # step, HIP events on the handle's stream around them, from the steps run
+    # one stage after another).  The bytes it cannot do without: the remote
+    # sums of every (cell, node) once, 8 B (16 B in FP64) each.
     K = info.num_nodes
-    pairs = natom * K
-    lr_ms = tm["kernel"].get("lr", float("nan"))
-    achieved = 20.0 * pairs / (lr_ms * 1e-3) / 1e12
-    # HBM traffic is not measured in this run: it is read from the committed
-    # summary of two rocprofv3 --pmc passes (FETCH_SIZE, WRITE_SIZE) over
-    # the same kernel on this workload
-    traffic, traffic_src = None, None
-    tf = os.path.join(REPO, "profiles", "lr_ag_288k_traffic.json")
-    if os.path.exists(tf):
-        with open(tf) as fh:
-            traffic = json.load(fh).get("bytes_per_step")
-        traffic_src = ("profiles/lr_ag_288k_traffic.json: rocprofv3 --pmc "
-                       "FETCH_SIZE and WRITE_SIZE of this kernel on this "
-                       "workload, committed; not measured in this run")
-    roof = {
-        "kernel": "lr_ag_kernel<NR> (calc_lr_ef back-projection over atom "
-                  "groups, all alpha-group launches of one step)",
-        "bound": "valu",
-        "achieved": achieved,
-        "peak": PEAK_FP32_VALU_TFLOPS,
-        "unit": "TFLOP/s",
-        "frac": achieved / PEAK_FP32_VALU_TFLOPS,
-        "traffic": traffic,
-        "traffic_source": traffic_src,
-        "avg_ms": lr_ms,
-        "pairs": pairs,
-        "pair_rate_per_s": pairs / (lr_ms * 1e-3),
-    }
+    ncell = int(np.prod(info.ncell))
 
-    # the FP64 path's back-projection (lr_f64_kernel, one launch per step)
-    # at the same 20 flops per pair against the FP64 vector peak
-    lr64_ms = t64["kernel"].get("lr", float("nan"))
-    ach64 = 20.0 * pairs / (lr64_ms * 1e-3) / 1e12
-    roof64 = {
-        "kernel": "lr_f64_kernel (calc_lr_ef back-projection, FP64)",
-        "bound": "valu",
-        "achieved": ach64,
-        "peak": PEAK_FP64_VALU_TFLOPS,
-        "unit": "TFLOP/s",
-        "frac": ach64 / PEAK_FP64_VALU_TFLOPS,
-        "avg_ms": lr64_ms,
-        "pairs": pairs,
-    }
+    def lr_roofline(ms, per_pair):
+        need = ncell * K * per_pair
+        gbs = need / (ms * 1e-3) / 1e9
+        return {
+            "kernel": "harm_lr, harm_radial and harm_eval (calc_lr_ef through "
+                      "the harmonic expansion)",
+            "bound": "hbm",
+            "achieved": gbs,
+            "peak": PEAK_HBM_GBS,
+            "unit": "GB/s",
+            "frac": gbs / PEAK_HBM_GBS,
+            "bytes": need,
+            "avg_ms": ms,
+            "cell_node_pairs": ncell * K,
+            "atom_node_pairs": natom * K,
+        }
+
+    roof = lr_roofline(tm["kernel"].get("lr", float("nan")), 8)
+    roof64 = lr_roofline(t64["kernel"].get("lr", float("nan")), 16)
 
     configs = config_errors(g, torch)
     log(f"configs: {configs}")
