@@ -207,7 +207,8 @@ struct glst_engine {
       // no room for the expansion's work fields: the direct sums need less
       if (!harm.ok()) throw;
       harm.release();
-      for (DeviceBuffer *b : {&harm_coef, &harm_mom, &harm_out, &S, &R})
+      for (DeviceBuffer *b :
+           {&harm_coef, &harm_mom, &harm_out, &S, &R, &rmt_work})
         b->release();
       allocate();
     }
@@ -226,7 +227,9 @@ struct glst_engine {
   size_t harm_coef_len = 0, harm_mom_len = 0;
   std::vector<uint32_t> harm_row_of;  // row of the fields of a node
   void plan_far_field() {
-    if (!has_lr || Kp == 0 || !harm_worth(natom, K, mixed())) return;
+    if (!has_lr || Kp == 0 || !harm_worth(natom, K, mixed()) ||
+        !harm_shell_sums(mixed(), rmt_shape, grid, lds_limit))
+      return;
     const HarmTables t = plan_harmonic(nodes, grid.h, spherical_rule, mixed());
     if (!t.ok) return;
     harm_plan = harm_fit(t, mixed(), lds_limit, natom, grid.ncell);
@@ -279,6 +282,9 @@ struct glst_engine {
           harm_coef.resize(harm_coef_len * real);
           harm_mom.resize(harm_mom_len * real);
           harm_out.resize(static_cast<size_t>(grid.ncell) * 4);
+          // (here, so that a handle without room for it takes direct sums)
+          if (rmt_global_path(true))
+            rmt_work.resize(field * sizeof(double2));
         }
         const uint32_t ntile = (natom + 255) / 256;
         // enough workgroups to fill the chip several times over
@@ -386,9 +392,11 @@ struct glst_engine {
   }
 
   // Far field through spherical harmonics: for handles that planned it,
-  // unless the options ask for the direct sums or for the global tables.
+  // unless the options ask for the direct sums or for the global tables, or
+  // only the expansion would need those (harm_shell_sums).
   bool harmonic() const {
-    return harm.ok() && sf_cheb && lr_atom_groups && rmt_shape != 2;
+    return harm.ok() && sf_cheb && lr_atom_groups && rmt_shape != 2 &&
+           harm_shell_sums(mixed(), rmt_shape, grid, lds_limit);
   }
   // The path of the S at hand: the stages after calc_sf follow it, also where
   // an option has changed since.
@@ -444,27 +452,32 @@ struct glst_engine {
     Scope sc(timer, "rmt", stream);
     const bool nm = expanded();
     const double4 *kn = nm ? harm.k64 : k64.as<double4>();
-    if (rmt_mfma_path(nm)) {
-      dev::rmt_mfma(S.as<void>(), kn, group.as<uint32_t>(),
-                    r_in.as<uint32_t>(), r_out.as<uint32_t>(), Kp, grid,
-                    lds_limit, R.as<void>(), stream, 0, 0xffffffffu, nm);
-    } else if (rmt_wave_path(nm)) {
-      dev::rmt_wave(S.as<void>(), kn, group.as<uint32_t>(),
-                    r_in.as<uint32_t>(), r_out.as<uint32_t>(), Kp, grid,
-                    R.as<void>(), stream, 0, 0xffffffffu, nm);
-    } else if (rmt_shape == 2 ||
-        !dev::rmt_lds(mixed(), rmt_shape == 1 ? 1 : dev::kRmtMaxNodes,
-                      S.as<void>(),
-                      kn, group.as<uint32_t>(),
+    switch (rmt_path(nm)) {
+      case dev::RmtPath::kMfma:
+        dev::rmt_mfma(S.as<void>(), kn, group.as<uint32_t>(),
                       r_in.as<uint32_t>(), r_out.as<uint32_t>(), Kp, grid,
-                      lds_limit, R.as<void>(), stream, 0, 0xffffffffu,
-                      nm)) {
-      // tables too large for LDS: FP64 work field, allocated on first use
-      rmt_work.resize(static_cast<size_t>(grid.ncell) * Kp * sizeof(double2));
-      dev::rmt_global(mixed(), S.as<void>(), rmt_work.as<double2>(),
-                      kn, group.as<uint32_t>(),
+                      lds_limit, R.as<void>(), stream, 0, 0xffffffffu, nm);
+        break;
+      case dev::RmtPath::kWave:
+        dev::rmt_wave(S.as<void>(), kn, group.as<uint32_t>(),
                       r_in.as<uint32_t>(), r_out.as<uint32_t>(), Kp, grid,
-                      R.as<void>(), stream, nm);
+                      R.as<void>(), stream, 0, 0xffffffffu, nm);
+        break;
+      case dev::RmtPath::kLds:
+        dev::rmt_lds(mixed(), rmt_shape == 1 ? 1 : dev::kRmtMaxNodes,
+                     S.as<void>(), kn, group.as<uint32_t>(),
+                     r_in.as<uint32_t>(), r_out.as<uint32_t>(), Kp, grid,
+                     lds_limit, R.as<void>(), stream, 0, 0xffffffffu, nm);
+        break;
+      case dev::RmtPath::kGlobal:
+        // tables too large for LDS: FP64 work field, allocated on first use
+        rmt_work.resize(static_cast<size_t>(grid.ncell) * Kp *
+                        sizeof(double2));
+        dev::rmt_global(mixed(), S.as<void>(), rmt_work.as<double2>(), kn,
+                        group.as<uint32_t>(), r_in.as<uint32_t>(),
+                        r_out.as<uint32_t>(), Kp, grid, R.as<void>(), stream,
+                        nm);
+        break;
     }
     check_launch("rmt");
     rmt_done = true;
@@ -552,14 +565,14 @@ struct glst_engine {
     return pipeline && !harmonic() && mixed() && has_lr && Kp > 0 &&
            !sf_groups.empty() &&
            ev_sf.size() == sf_groups.size() &&
-           lr_groups.size() == sf_groups.size() && !rmt_global_path();
+           lr_groups.size() == sf_groups.size() && !rmt_global_path(false);
   }
   void plan_pipeline() {
     pipe_tmax = rmt_shape == 1 ? 1 : dev::kRmtMaxNodes;
     const uint32_t T =
-        rmt_mfma_path()
+        rmt_path(false) == dev::RmtPath::kMfma
             ? dev::rmt_mfma_nodes(grid, lds_limit)
-        : rmt_wave_path()
+        : rmt_path(false) == dev::RmtPath::kWave
             ? dev::kRmtWaveNodes
             : dev::rmt_nodes_per_group(grid.nx, grid.ny, grid.nz, lds_limit,
                                        pipe_tmax);
@@ -602,12 +615,12 @@ struct glst_engine {
         if (g > 0) GLST_HIP(hipStreamWaitEvent(rmt_stream, ev_sf[g], 0));
         const uint32_t t0 = g > 0 ? tile_end[g - 1] : 0;
         const bool ok =
-            rmt_mfma_path()
+            rmt_path(false) == dev::RmtPath::kMfma
                 ? dev::rmt_mfma(S.as<void>(), k64.as<double4>(),
                                 group.as<uint32_t>(), r_in.as<uint32_t>(),
                                 r_out.as<uint32_t>(), Kp, grid, lds_limit,
                                 R.as<void>(), rmt_stream, t0, tile_end[g])
-            : rmt_wave_path()
+            : rmt_path(false) == dev::RmtPath::kWave
                 ? dev::rmt_wave(S.as<void>(), k64.as<double4>(),
                                 group.as<uint32_t>(), r_in.as<uint32_t>(),
                                 r_out.as<uint32_t>(), Kp, grid, R.as<void>(),
@@ -688,29 +701,12 @@ struct glst_engine {
     graph_exec = nullptr;
   }
 
-  // shell sums through the global-memory tables (one node's table does not
-  // fit in LDS, or forced)
-  bool rmt_global_path() const {
-    if (rmt_mfma_path() || rmt_wave_path()) return false;
-    return rmt_shape == 2 ||
-           dev::rmt_nodes_per_group(grid.nx, grid.ny, grid.nz, lds_limit,
-                                    1) == 0;
+  // the kernel of the shell sums on fields of this layout
+  dev::RmtPath rmt_path(bool nm) const {
+    return dev::rmt_path(mixed(), rmt_shape, grid, lds_limit, nm);
   }
-  // shell sums on the matrix cores (CT = float, nx and ny up to 16)
-  bool rmt_mfma_path(bool nm = false) const {
-    const bool want =
-        rmt_shape == 3 ||
-        (rmt_shape == 4 && grid.nx * grid.ny * 2 >= dev::kRmtMfmaMaxXY *
-                                                        dev::kRmtMfmaMaxXY);
-    return want && mixed() &&
-           dev::rmt_mfma_nodes(grid, lds_limit, nm) > 0;
-  }
-  // shell sums as window sums of small grids (CT = float, every dimension
-  // up to 8)
-  bool rmt_wave_path(bool nm = false) const {
-    const bool want =
-        rmt_shape == 5 || (rmt_shape == 4 && !rmt_mfma_path(nm));
-    return want && mixed() && dev::rmt_wave_fits(grid);
+  bool rmt_global_path(bool nm) const {
+    return rmt_path(nm) == dev::RmtPath::kGlobal;
   }
 
   // New back-projection split target: splits, their table and the partials.
@@ -741,7 +737,7 @@ struct glst_engine {
       // nothing may allocate inside the capture, and a change of layout
       // belongs before it
       if (has_lr && Kp > 0) set_field_layout();
-      if (has_lr && Kp > 0 && rmt_global_path())
+      if (has_lr && Kp > 0 && rmt_global_path(harmonic()))
         rmt_work.resize(static_cast<size_t>(grid.ncell) * Kp * sizeof(double2));
       const bool timing = timer.enabled;
       timer.enabled = false;
@@ -839,7 +835,7 @@ struct glst_engine {
              apply_lr_blocks();
            },
            {1024, 2048, 4096, 8192, 16384, 32768, 65536});
-      if (!rmt_global_path())
+      if (!rmt_global_path(harmonic()))
         knob([&] { return static_cast<int64_t>(rmt_shape); },
              [&](int64_t v) {
                rmt_shape = static_cast<int>(v);

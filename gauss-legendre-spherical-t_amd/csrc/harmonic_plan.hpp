@@ -393,6 +393,22 @@ inline bool harm_worth(uint32_t natom, uint32_t K, bool single) {
          (single ? kHarmPairs32 : kHarmPairs64);
 }
 
+// Whether the shell sums of node-major fields run on tables no worse than
+// those of the direct sums' fields: not where only they need the FP64 tables
+// in global memory, because the node-major matrix-core kernel takes z slices
+// too (mixed grids of up to 16 x 16 cells whose long axis in z leaves no room
+// in LDS).  345,000 charges on 16 x 16 x 33 cells: shell sums 10.8 ms against
+// 1.8 on the matrix cores, steps 13.8 against 5.0, and 2.5 GB of tables.  Up
+// to 32 cells in z the tables fit in LDS and the expansion keeps its gain
+// (251,000 charges on 16 x 16 x 24: 3.13 ms against 3.52).
+inline bool harm_shell_sums(bool mixed, int rmt_shape,
+                            const dev::GridShape &g, size_t lds_limit) {
+  auto path = [&](bool nm) {
+    return dev::rmt_path(mixed, rmt_shape, g, lds_limit, nm);
+  };
+  return path(true) == path(false) || path(true) != dev::RmtPath::kGlobal;
+}
+
 // Launch sizes for a system of natom atoms in ncell cells; nrad 0 where a
 // kernel's LDS does not fit.
 inline dev::HarmPlanDev harm_fit(const HarmTables &t, bool single,

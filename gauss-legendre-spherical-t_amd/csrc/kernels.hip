@@ -3681,20 +3681,6 @@ bool rmt_lds(bool mixed, uint32_t tmax, const void *S, const double4 *k64,
   return true;
 }
 
-// Nodes per tile of the matrix-core shell sums: two (two workgroups of 63 KB
-// share a CU at 15^3) where they fit, else one.
-#ifndef GLST_RMT_MFMA_NPW
-#define GLST_RMT_MFMA_NPW 2
-#endif
-uint32_t rmt_mfma_nodes(const GridShape &g, size_t lds_limit, bool nm) {
-  if (g.nx > kRmtMfmaMaxXY || g.ny > kRmtMfmaMaxXY || g.ncell == 0) return 0;
-  if (nm && g.nz > kRmtMfmaMaxXY) return 0;
-  const uint32_t a = nm ? g.nz : g.nx, c = nm ? g.nx : g.nz;
-  for (uint32_t npw = GLST_RMT_MFMA_NPW; npw >= 1; npw >>= 1)
-    if (rmt_mfma_lds_bytes(a, g.ny, c, npw) <= lds_limit) return npw;
-  return 0;
-}
-
 bool rmt_mfma(const void *S, const double4 *k64, const uint32_t *group,
               const uint32_t *r_in, const uint32_t *r_out, uint32_t Kp,
               const GridShape &g, size_t lds_limit, void *R, hipStream_t s,

@@ -223,11 +223,23 @@ inline size_t rmt_mfma_lds_bytes(uint32_t nx, uint32_t ny, uint32_t nz,
   const size_t nline = static_cast<size_t>(nx) * ny;
   return npw * (nline * (rmt_zpitch(nz) + 1) + nx + ny + nz) * 8;
 }
-// Nodes per workgroup tile of the matrix-core shell sums on this grid (0:
+// Nodes per workgroup tile of the matrix-core shell sums on this grid: two
+// (two workgroups of 63 KB share a CU at 15^3) where they fit, else one (0:
 // the grid is too wide for them, or one node's table does not fit).  On
 // node-major fields the slices are (z, y) planes, so that a slice's cells are
 // consecutive in the rows, and nz is limited as well.
-uint32_t rmt_mfma_nodes(const GridShape &g, size_t lds_limit, bool nm = false);
+#ifndef GLST_RMT_MFMA_NPW
+#define GLST_RMT_MFMA_NPW 2
+#endif
+inline uint32_t rmt_mfma_nodes(const GridShape &g, size_t lds_limit,
+                               bool nm = false) {
+  if (g.nx > kRmtMfmaMaxXY || g.ny > kRmtMfmaMaxXY || g.ncell == 0) return 0;
+  if (nm && g.nz > kRmtMfmaMaxXY) return 0;
+  const uint32_t a = nm ? g.nz : g.nx, c = nm ? g.nx : g.nz;
+  for (uint32_t npw = GLST_RMT_MFMA_NPW; npw >= 1; npw >>= 1)
+    if (rmt_mfma_lds_bytes(a, g.ny, c, npw) <= lds_limit) return npw;
+  return 0;
+}
 // Tiles [tile0, tile1) of rmt_mfma_nodes() nodes (tile1 clamped to
 // Kp / nodes).  False: the grid is not supported (nothing launched).
 bool rmt_mfma(const void *S, const double4 *k64, const uint32_t *group,
@@ -246,6 +258,23 @@ constexpr uint32_t kRmtWaveBlock = 256;
 inline bool rmt_wave_fits(const GridShape &g) {
   return g.ncell > 0 && g.nx <= kRmtWaveMaxDim && g.ny <= kRmtWaveMaxDim &&
          g.nz <= kRmtWaveMaxDim;
+}
+// The kernel a handle's shell sums run on, for its option rmt_shape (0 .. 5,
+// glst_hip.h) and the layout of its fields: the one place that decides, for
+// the launches, the work field that the global tables need (which a captured
+// step cannot allocate) and the choice of the far field (harmonic_plan.hpp).
+enum class RmtPath { kMfma, kWave, kLds, kGlobal };
+inline RmtPath rmt_path(bool mixed, int shape, const GridShape &g,
+                        size_t lds_limit, bool nm) {
+  const bool wide = g.nx * g.ny * 2 >= kRmtMfmaMaxXY * kRmtMfmaMaxXY;
+  if (mixed && (shape == 3 || (shape == 4 && wide)) &&
+      rmt_mfma_nodes(g, lds_limit, nm) > 0)
+    return RmtPath::kMfma;
+  if (mixed && (shape == 4 || shape == 5) && rmt_wave_fits(g))
+    return RmtPath::kWave;
+  if (shape == 2 || rmt_nodes_per_group(g.nx, g.ny, g.nz, lds_limit, 1) == 0)
+    return RmtPath::kGlobal;
+  return RmtPath::kLds;
 }
 // Tiles [tile0, tile1) of kRmtWaveNodes nodes (tile1 clamped to
 // Kp / kRmtWaveNodes).  False: the grid does not fit (nothing launched).

@@ -1,0 +1,75 @@
+// Host check of the rules that choose a handle's kernels: the shell sums' path
+// (rmt_path) on both field layouts, and the far field's expansion, which must
+// not bring in FP64 tables in global memory where the direct sums' fields need
+// none.  Prints one line per failure and the counts.
+#include "harmonic_plan.hpp"
+
+#include <cstdio>
+
+namespace glst {
+std::string tdesign_dir() { return ""; }
+namespace dev {
+template <typename T>
+size_t harm_lds_sf(uint32_t, uint32_t) { return 0; }
+template <typename T>
+size_t harm_lds_lr(uint32_t, uint32_t, uint32_t) { return 0; }
+template size_t harm_lds_sf<float>(uint32_t, uint32_t);
+template size_t harm_lds_sf<double>(uint32_t, uint32_t);
+template size_t harm_lds_lr<float>(uint32_t, uint32_t, uint32_t);
+template size_t harm_lds_lr<double>(uint32_t, uint32_t, uint32_t);
+}  // namespace dev
+}  // namespace glst
+
+int main() {
+  using namespace glst;
+  using dev::RmtPath;
+  constexpr size_t kLds = 160 * 1024;
+  int failures = 0;
+  long checks = 0, refused = 0;
+  const uint32_t dims[] = {3, 4, 8, 9, 12, 15, 16, 17, 20, 21, 24, 33, 38, 64};
+  for (bool mixed : {true, false})
+    for (int shape = 0; shape <= 5; ++shape)
+      for (uint32_t nx : dims)
+        for (uint32_t ny : dims)
+          for (uint32_t nz : dims) {
+            const dev::GridShape g{nx, ny, nz, nx * ny * nz, 9.0};
+            const RmtPath a = dev::rmt_path(mixed, shape, g, kLds, false);
+            const RmtPath b = dev::rmt_path(mixed, shape, g, kLds, true);
+            const bool fits = dev::rmt_nodes_per_group(nx, ny, nz, kLds, 1) > 0;
+            // each path where its kernel takes the grid
+            bool good = true;
+            for (bool nm : {false, true}) {
+              const RmtPath p = nm ? b : a;
+              if (p == RmtPath::kMfma)
+                good = good && mixed && dev::rmt_mfma_nodes(g, kLds, nm) > 0;
+              if (p == RmtPath::kWave)
+                good = good && mixed && dev::rmt_wave_fits(g);
+              if (p == RmtPath::kLds) good = good && fits && shape != 2;
+              if (p == RmtPath::kGlobal) good = good && (!fits || shape == 2);
+            }
+            const bool takes = harm_shell_sums(mixed, shape, g, kLds);
+            const bool worse = b == RmtPath::kGlobal && a != RmtPath::kGlobal;
+            if (!good || takes == worse) {
+              std::printf("FAIL mixed %d shape %d grid %u x %u x %u: paths %d "
+                          "%d takes %d\n", mixed, shape, nx, ny, nz,
+                          static_cast<int>(a), static_cast<int>(b), takes);
+              ++failures;
+            }
+            ++checks;
+            refused += !takes;
+          }
+  auto refuses = [&](uint32_t nx, uint32_t ny, uint32_t nz, bool want) {
+    const dev::GridShape g{nx, ny, nz, nx * ny * nz, 9.0};
+    if (harm_shell_sums(true, 4, g, kLds) == want) {
+      std::printf("FAIL %u x %u x %u\n", nx, ny, nz);
+      ++failures;
+    }
+  };
+  refuses(16, 16, 40, true);
+  refuses(16, 16, 33, true);
+  refuses(16, 16, 24, false);
+  refuses(15, 15, 15, false);
+  refuses(21, 21, 21, false);  // global tables on either layout
+  std::printf("checks %ld refused %ld failures %d\n", checks, refused, failures);
+  return failures ? 1 : 0;
+}
