@@ -299,7 +299,7 @@ BatchLayout pack_batch(int ct,
     // systems 13.5, 13.4 and 16.1 ms; 16 systems 2.9, 4.2 and 4.7 ms)
     HarmSystem hs{s, 0, {}};
     if (cheb && lr && !cs[s]->direct &&
-        harm_worth(na, u.K, ct == GLST_CT_FLOAT) &&
+        harm_worth(na, d.ncell, u.K, ct == GLST_CT_FLOAT) &&
         static_cast<double>(na) * u.K * kHarmShare >= pairs) {
       const HarmTables &t = cs[s]->shape->harm();
       if (t.ok)

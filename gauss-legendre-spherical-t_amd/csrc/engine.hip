@@ -227,7 +227,8 @@ struct glst_engine {
   size_t harm_coef_len = 0, harm_mom_len = 0;
   std::vector<uint32_t> harm_row_of;  // row of the fields of a node
   void plan_far_field() {
-    if (!has_lr || Kp == 0 || !harm_worth(natom, K, mixed()) ||
+    if (!has_lr || Kp == 0 ||
+        !harm_worth(natom, grid.ncell, K, mixed()) ||
         !harm_shell_sums(mixed(), rmt_shape, grid, lds_limit))
       return;
     const HarmTables t = plan_harmonic(nodes, grid.h, spherical_rule, mixed());

@@ -28,6 +28,17 @@ constexpr double kHarmEps64 = 1e-15;
 // to 749 but 3,300 at 1e-4 525 to 528 and 1,800 at 1e-4 (1.3e8) 479 to 385,
 // 5,500 at 1e-4 (4e8) 828 to 858, 1,000 at 1e-6 1,213 to 1,403.
 constexpr double kHarmPairs32 = 2e8, kHarmPairs64 = 3e8;
+// So do dilute ones: the direct sums cost (atom, node) work, the expansion
+// (cell, node) work, whatever the cells hold.  Fewest atoms per cell on grids
+// of up to 512 cells, where the direct sums' launches leave the device partly
+// idle, and beyond.  Steps in ms, expansion against direct sums, at so many
+// atoms per cell: mixed 6^3 cells (tol 1e-6) 0.75 to 0.88 at 10, 8^3 (1e-5)
+// 0.70 to 0.84 at 5; 10^3 (1e-4) 0.56 to 0.66 at 22, 15^3 1.24 to 1.27 at 22,
+// 1.22 to 1.07 at 12, 1.22 to 0.98 at 6.  FP64 6^3 2.14 to 2.53 at 23 and to
+// 1.67 at 10, 8^3 2.31 to 2.82 at 21 and to 2.09 at 11; 10^3 1.39 to 2.05 at
+// 39, 1.29 to 1.30 at 22, 15^3 3.63 to 3.51 at 22, 3.60 to 2.31 at 12.
+constexpr uint32_t kHarmSmallGrid = 512;
+constexpr double kHarmFill32[2] = {0.0, 22.0}, kHarmFill64[2] = {17.0, 24.0};
 
 // j_0(z) .. j_{n-1}(z), z > 0: Miller's backward recurrence j_{m-1} =
 // (2m + 1) / z j_m - j_{m+1} from well above max(n, z), normalised by
@@ -388,9 +399,13 @@ inline HarmTables plan_harmonic(const NodeTable &nodes, double h,
   return T;
 }
 
-inline bool harm_worth(uint32_t natom, uint32_t K, bool single) {
+inline bool harm_worth(uint32_t natom, uint32_t ncell, uint32_t K,
+                       bool single) {
+  const double fill =
+      (single ? kHarmFill32 : kHarmFill64)[ncell > kHarmSmallGrid];
   return static_cast<double>(natom) * K >=
-         (single ? kHarmPairs32 : kHarmPairs64);
+             (single ? kHarmPairs32 : kHarmPairs64) &&
+         natom >= fill * ncell;
 }
 
 // Whether the shell sums of node-major fields run on tables no worse than

@@ -70,6 +70,24 @@ int main() {
   refuses(16, 16, 24, false);
   refuses(15, 15, 15, false);
   refuses(21, 21, 21, false);  // global tables on either layout
+  // dilute systems keep the direct sums: (charges, cells, nodes, mixed, taken)
+  auto worth = [&](uint32_t n, uint32_t ncell, uint32_t K, bool mixed,
+                   bool want) {
+    if (harm_worth(n, ncell, K, mixed) != want) {
+      std::printf("FAIL %u charges in %u cells\n", n, ncell);
+      ++failures;
+    }
+  };
+  worth(288000, 3375, 27453, true, true);
+  worth(288000, 3375, 27453, false, true);
+  worth(39304, 3375, 14718, true, false);
+  worth(39304, 3375, 14718, false, false);
+  worth(8000, 3375, 27453, true, false);
+  worth(32928, 6144, 17862, true, false);
+  worth(2744, 512, 74032, true, true);   // small grid
+  worth(2744, 512, 200000, false, false);
+  worth(10648, 512, 74032, false, true);
+  worth(3000, 64, 20000, true, false);   // few pairs
   std::printf("checks %ld refused %ld failures %d\n", checks, refused, failures);
   return failures ? 1 : 0;
 }

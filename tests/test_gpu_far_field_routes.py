@@ -1,5 +1,5 @@
 """Which far field a handle takes, and that every route gives the same fields:
-grids with one long edge, captured and eager.
+grids with one long edge, captured and eager; dilute systems.
 
 lr_blocks cuts the direct sums' back-projection into other partial sums and
 has no effect on the expansion, so "the same bits under another lr_blocks"
@@ -43,7 +43,7 @@ def same(a, b):
 def expands(f, d):
     """Whether this handle's steps expand the far field."""
     keep, a = f.get_option("lr_blocks"), step(f, d)
-    f.set_option("lr_blocks", 4 * keep)
+    f.set_option("lr_blocks", 1)
     b = step(f, d)
     f.set_option("lr_blocks", keep)
     return same(a, b)
@@ -76,3 +76,19 @@ def test_long_grids_captured_and_eager(cuda, nz, want):
     f.close()
     assert rel_err(eager[:3], ref[:3]) < 2e-6
     assert rel_err(eager[3:], ref[3:]) < 2e-6
+
+
+@pytest.mark.parametrize("ct,n,spacing,tol,want", [
+    ("float", 12, 3.0, 1e-4, True), ("float", 12, 4.0, 1e-4, False),
+    ("float", 8, 4.0, 1e-5, True),
+    ("double", 8, 3.0, 1e-5, True), ("double", 8, 4.0, 1e-5, False)])
+def test_dilute_systems_keep_direct_sums(cuda, ct, n, spacing, tol, want):
+    """Atoms per cell of n^3 grids: 27 (spacing 3) and 11.4 (spacing 4)."""
+    import torch
+    import glst_amd as g
+    box = (9.0 * n - 0.5,) * 3
+    h = lattice(box, spacing, 5)
+    f, d = handle(g, torch, h, box, tol, ct=ct)
+    assert f.info().ncell_total == n ** 3
+    assert expands(f, d) == want
+    f.close()

@@ -1,7 +1,8 @@
 """The rules that choose a handle's kernels, on the CPU under AddressSanitizer
 and UBSan (tests/host/route_check.cpp): the expansion of the far field is not
 taken where only its field layout would send the shell sums to FP64 tables in
-global memory, which a captured step cannot allocate.
+global memory, which a captured step cannot allocate, nor by dilute systems,
+whose direct sums are the faster.
 """
 import os
 import shutil
