@@ -92,3 +92,35 @@ def test_dilute_systems_keep_direct_sums(cuda, ct, n, spacing, tol, want):
     assert f.info().ncell_total == n ** 3
     assert expands(f, d) == want
     f.close()
+
+
+@pytest.mark.parametrize("ct,bar", [("double", 1e-11), ("float", 2e-6)])
+def test_global_tables_on_node_major_fields(cuda, ct, bar):
+    """17 x 18 x 31 cells, whose shell-sum tables fit no LDS (nor do the
+    matrix-core slices): the expansion through the tables in global memory,
+    tiles of 16 cells in z with a remainder, against the FP64 direct sums."""
+    import torch
+    import glst_amd as g
+    box, tol = (152.0, 161.0, 278.0), 1e-4
+    h = lattice(box, 2.95, 9)
+    f, d = handle(g, torch, h, box, tol, ct=ct)
+    assert tuple(f.info().ncell) == (17, 18, 31)
+    assert expands(f, d)
+    f.assign_atoms(*d)
+    f.calc_sf()
+    f.sum_rmt_sf()
+    r = f.rmt()
+    ef = step(f, d)
+    f.close()
+    f, d = handle(g, torch, h, box, tol, ct="double", lr_atom_groups=0)
+    f.assign_atoms(*d)
+    f.calc_sf()
+    f.sum_rmt_sf()
+    r0 = f.rmt()
+    ef0 = step(f, d)
+    f.close()
+    scale = max(np.abs(a).max() for a in r0)
+    assert max(np.abs(a - b).max() for a, b in zip(r, r0)) < \
+        (1e-11 if ct == "double" else 1e-5) * scale
+    assert rel_err(ef[:3], ef0[:3]) < bar
+    assert rel_err(ef[3:], ef0[3:]) < bar
