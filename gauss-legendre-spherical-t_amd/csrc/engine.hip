@@ -203,6 +203,7 @@ struct glst_engine {
     plan_far_field();
     try {
       allocate();
+      upload_nodes();
     } catch (const AllocError &) {
       // no room for the expansion's work fields: the direct sums need less
       if (!harm.ok()) throw;
@@ -211,8 +212,8 @@ struct glst_engine {
            {&harm_coef, &harm_mom, &harm_out, &S, &R, &rmt_work})
         b->release();
       allocate();
+      upload_nodes();
     }
-    upload_nodes();
     dev::fill_f64(fx.as<double>(), 0.0, natom, stream);
     dev::fill_f64(fy.as<double>(), 0.0, natom, stream);
     dev::fill_f64(fz.as<double>(), 0.0, natom, stream);
