@@ -59,9 +59,8 @@ size_t BatchLayout::device_bytes() const {
   b += field * (mixed() ? 8 : 16) * 2;  // S and R
   b += partial * sizeof(double4);
   b += (sys.size() + sys_harm.size()) * sizeof(dev::SysDev);
-  b += std::min<size_t>(harm.size(), kHarmSlots) *
-           (harm_coef + harm_mom + harm_out) +
-       harm_bytes;
+  for (const HarmSlot &f : harm_slot) b += f.coef + f.mom + f.out;
+  b += harm_bytes;
   size_t nseg = bin.seg.size() + hist_p.seg.size() + scatter.seg.size() +
                 sr.seg.size() + reduce.seg.size() + rmt.seg.size() +
                 rmt_small.seg.size() + rmt_rest.seg.size() +
@@ -297,7 +296,8 @@ BatchLayout pack_batch(int ct,
     // mixed systems of 100 to 10,000 waters: 94.2 ms with all that a handle
     // would expand, 86.4 with those of 8e8 pairs, 92.4 with none; 64 such
     // systems 13.5, 13.4 and 16.1 ms; 16 systems 2.9, 4.2 and 4.7 ms)
-    HarmSystem hs{s, 0, {}};
+    HarmSystem hs{};
+    hs.sys = s;
     if (cheb && lr && !cs[s]->direct &&
         harm_worth(na, d.ncell, u.K, ct == GLST_CT_FLOAT) &&
         static_cast<double>(na) * u.K * kHarmShare >= pairs) {
@@ -306,9 +306,9 @@ BatchLayout pack_batch(int ct,
         hs.plan = harm_fit(t, ct == GLST_CT_FLOAT, lds_limit, na, d.ncell);
       if (hs.plan.nrad) {
         const size_t real = ct == GLST_CT_FLOAT ? 4 : 8;
-        B.harm_coef = std::max(B.harm_coef, harm_coef_len(t, d.ncell) * real);
-        B.harm_mom = std::max(B.harm_mom, harm_mom_len(t, d.ncell) * real);
-        B.harm_out = std::max<size_t>(B.harm_out, size_t{4} * d.ncell);
+        hs.coef = harm_coef_len(t, d.ncell) * real;
+        hs.mom = harm_mom_len(t, d.ncell) * real;
+        hs.out = size_t{4} * d.ncell;
         if (!expanded[cs[s]->shape.get()]) B.harm_bytes += t.bytes(real);
         expanded[cs[s]->shape.get()] = true;
         B.harm.push_back(hs);
@@ -377,6 +377,10 @@ BatchLayout pack_batch(int ct,
     h.slot = static_cast<uint32_t>(
         std::min_element(load, load + kHarmSlots) - load);
     load[h.slot] += kHarmPairs32 + work(h);
+    HarmSlot &f = B.harm_slot[h.slot];
+    f.coef = std::max(f.coef, h.coef);
+    f.mom = std::max(f.mom, h.mom);
+    f.out = std::max(f.out, h.out);
   }
   if (!B.harm.empty()) {
     B.sys_harm = B.sys;
@@ -541,9 +545,9 @@ void glst_batch::configure(
   partial.grow(B.partial * sizeof(double4), hr);
   const size_t nslot = std::min<size_t>(B.harm.size(), kHarmSlots);
   for (size_t i = 0; i < nslot; ++i) {
-    harm_coef[i].grow(B.harm_coef, hr);
-    harm_mom[i].grow(B.harm_mom, hr);
-    harm_out[i].grow(B.harm_out, hr);
+    harm_coef[i].grow(B.harm_slot[i].coef, hr);
+    harm_mom[i].grow(B.harm_slot[i].mom, hr);
+    harm_out[i].grow(B.harm_slot[i].out, hr);
     if (!harm_stream[i])
       GLST_HIP(hipStreamCreateWithFlags(&harm_stream[i],
                                         hipStreamNonBlocking));

@@ -128,7 +128,9 @@ struct Plan {
 };
 
 // Systems with an expanded far field (harmonic.hpp) run their passes on this
-// many streams, each with work fields for its largest system: a pass of one
+// many streams, each with work fields for the largest of its systems (so that a
+// batch needs no more than its systems do alone, one slot each: the sum by
+// which a server admits them): a pass of one
 // system is too short to fill the device.  The rule of a single handle decides
 // which (the launches per stage keep the others): 64 mixed systems of 100 to
 // 10,000 waters take 14.6 ms, 16.0 with direct sums for all; 12 FP64 systems
@@ -137,6 +139,10 @@ constexpr uint32_t kHarmSlots = 4;
 struct HarmSystem {
   uint32_t sys, slot;
   dev::HarmPlanDev plan;
+  size_t coef, mom, out;  // bytes of its work fields
+};
+struct HarmSlot {
+  size_t coef = 0, mom = 0, out = 0;  // bytes of the work fields
 };
 
 // Host layout of a whole batch: SysDev records (offsets into the shape
@@ -156,12 +162,13 @@ struct BatchLayout {
   // whose grids fit dev::rmt_wave (rmt_small, when asked for) and the rest
   // (rmt_rest); rmt holds every system (the fused step's phase)
   Plan rmt_small, rmt_rest;
-  // the expanded systems, in launch order, and the work fields of a slot in
-  // bytes; the launches per stage (S(k), back-projection, rmt_*_direct) leave
+  // the expanded systems, in launch order, and the slots' work fields; the
+  // launches per stage (S(k), back-projection, rmt_*_direct) leave
   // them out, and the sum over the back-projection's rows reads one
   // (sys_harm: `sys` with nsplit 1).  The other modes sum all directly.
   std::vector<HarmSystem> harm;
-  size_t harm_coef = 0, harm_mom = 0, harm_out = 0, harm_bytes = 0;
+  HarmSlot harm_slot[kHarmSlots];
+  size_t harm_bytes = 0;  // the shapes' tables
   std::vector<dev::SysDev> sys_harm;
   Plan rmt_small_direct, rmt_rest_direct;
   std::map<uint32_t, Plan> sf_nr, lr_nr;  // radial count (0: any) -> plan
