@@ -519,6 +519,19 @@ void glst_batch::configure(
     GLST_HIP(hipDeviceSynchronize());
     tables->clear();
   }
+  try {
+    set_up(ct, cs);
+  } catch (const AllocError &) {
+    // no room for the expansions' work fields: the direct sums need fewer
+    if (B.harm.empty()) throw;
+    release_arenas();
+    for (auto &c : cs) c = make_batch_system(c->natom, c->shape, true);
+    set_up(ct, cs);
+  }
+}
+
+void glst_batch::set_up(
+    int ct, const std::vector<std::shared_ptr<const glst::BatchSystem>> &cs) {
   B = pack_batch(ct, cs, *tables, lds_limit, lr_blocks, sf_cheb != 0,
                  rmt_wave != 0);
   tables->upload(stream);

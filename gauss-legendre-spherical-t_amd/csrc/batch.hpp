@@ -271,7 +271,8 @@ struct glst_batch {
   // device, streams and events (once)
   void open(void *stream_);
   // (re)pack for these systems: uploads tables and run tables, grows arenas,
-  // clears S and the accumulators
+  // clears S and the accumulators; with direct sums for all where the
+  // expansions' work fields find no room
   void configure(int ct,
                  std::vector<std::shared_ptr<const glst::BatchSystem>> cs);
   void zero_ef();
@@ -303,6 +304,9 @@ struct glst_batch {
   size_t device_bytes() const;
 
  private:
+  void set_up(
+      int ct,
+      const std::vector<std::shared_ptr<const glst::BatchSystem>> &cs);
   glst::dev::LrTaskArgs task_args() const;
   void near_field(hipStream_t s);
   // clears S where the next step's layout differs from what it holds (not
