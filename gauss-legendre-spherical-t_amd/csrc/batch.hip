@@ -798,12 +798,12 @@ void glst_batch::step_async(const double *rx, const double *ry,
                             const double *rz, const double *qc) {
   if (!rx || !ry || !rz || !qc)
     throw ArgError("calc_ener_force: null coordinate or charge pointer");
+  set_field_layout();
   if (use_fused()) {
     step_fused(rx, ry, rz, qc);
     assigned = true;
     return;
   }
-  set_field_layout();
   const bool expand = fused == 0 && !B.harm.empty();
   const dev::SysDev *sys = d_sys.as<dev::SysDev>();
   // assign_atoms of every system

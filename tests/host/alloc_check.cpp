@@ -5,6 +5,7 @@
 //            the direct sums, up to the bytes those need
 //   batch    the same for a batch
 //   slots    a batch of expanded systems needs no more than they do alone
+//   layout   a batch clears S where a step's layout of it differs from the last
 // Prints "ok" and returns 0, or one line per failure.
 #include "fake_hip.hpp"
 #include "glst_batch.h"
@@ -98,8 +99,7 @@ void handle() {
     }
 }
 
-size_t batch_run(int ct, const std::vector<Sys> &v, size_t limit, int *route,
-                 int fused = 0) {
+size_t batch_run(int ct, const std::vector<Sys> &v, size_t limit, int *route) {
   std::vector<uint32_t> n;
   std::vector<double> box, rcut;
   for (const Sys &s : v) {
@@ -114,7 +114,6 @@ size_t batch_run(int ct, const std::vector<Sys> &v, size_t limit, int *route,
   glst_status_t s =
       glst_batch_create(ct, static_cast<uint32_t>(n.size()), n.data(),
                         box.data(), rcut.data(), v[0].tol, nullptr, &b);
-  if (s == GLST_OK && fused) s = glst_batch_set_option(b, "fused", fused);
   if (s == GLST_OK)
     s = glst_batch_calc_ener_force(b, arr(0), arr(1), arr(2), arr(3));
   const size_t peak = st.peak;
@@ -170,6 +169,32 @@ void slots() {
   }
 }
 
+// fused 0 expands, the other launch modes do not
+void layout() {
+  const uint32_t n = 100000;
+  const double box[] = {135, 135, 135}, rcut = 9;
+  glst_batch_t b = nullptr;
+  CHECK(glst_batch_create(GLST_CT_FLOAT, 1, &n, box, &rcut, 1e-4, nullptr,
+                          &b) == GLST_OK, "%s", glst_global_last_error());
+  int last = -1;
+  for (int graph : {0, 1})
+    for (int fused : {0, 0, 1, 1, 0, 2, 0, 3, 2, 0}) {
+      glst_batch_set_option(b, "graph", graph);
+      CHECK(glst_batch_set_option(b, "fused", fused) == GLST_OK, "%s",
+            glst_batch_last_error(b));
+      st.reset();
+      CHECK(glst_batch_calc_ener_force(b, arr(0), arr(1), arr(2), arr(3)) ==
+                GLST_OK, "%s", glst_batch_last_error(b));
+      const int now = fused == 0;
+      CHECK((st.harm > 0) == (now == 1), "fused %d", fused);
+      // S: more than the 4 n doubles of the accumulators
+      CHECK((st.filled > 4 * n) == (last >= 0 && now != last),
+            "fused %d graph %d: %zu doubles filled", fused, graph, st.filled);
+      last = now;
+    }
+  glst_batch_destroy(b);
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -178,6 +203,7 @@ int main(int argc, char **argv) {
   else if (what == "handle") handle();
   else if (what == "batch") batch();
   else if (what == "slots") slots();
+  else if (what == "layout") layout();
   else return 2;
   if (failures || st.failures) return 1;
   std::printf("ok\n");

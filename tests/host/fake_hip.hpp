@@ -10,6 +10,7 @@
 
 #include <sys/mman.h>
 
+#include <algorithm>
 #include <cstdio>
 #include <cstring>
 #include <map>
@@ -23,7 +24,8 @@ struct State {
   long refused_in_capture = 0, failures = 0;
   // launches since reset(): expanded and direct far fields, shell sums by path
   long harm = 0, direct = 0, global = 0, steps = 0;
-  void reset() { harm = direct = global = steps = 0; }
+  size_t filled = 0;  // doubles of the largest fill
+  void reset() { harm = direct = global = steps = filled = 0; }
 };
 inline State st;
 
@@ -161,6 +163,7 @@ void prepare_kernels(size_t) {}
 void fill_u32(uint32_t *, uint32_t, size_t, hipStream_t) {}
 void fill_f64(double *p, double, size_t n, hipStream_t) {
   if (n) fake::require(p, n * 8, "fill_f64");
+  fake::st.filled = std::max(fake::st.filled, n);
 }
 void bin_chunks(bool, const double *, const double *, const double *, uint32_t,
                 double, const GridShape &, uint32_t *, uint32_t *, uint32_t *,

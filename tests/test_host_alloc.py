@@ -29,7 +29,7 @@ def alloc_check(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("what", ["handle", "capture", "batch", "slots"])
+@pytest.mark.parametrize("what", ["handle", "capture", "batch", "slots", "layout"])
 def test_allocations(alloc_check, what):
     r = subprocess.run([alloc_check, what], capture_output=True, text=True,
                        timeout=300)
