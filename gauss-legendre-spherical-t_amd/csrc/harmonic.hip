@@ -19,6 +19,7 @@
 #include "harmonic.hpp"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace glst {
 namespace dev {
@@ -253,8 +254,10 @@ __device__ __forceinline__ void harm_switch(uint32_t n, F f) {
 // tabulated in LDS by all waves; the recurrence constants of a round are
 // loaded during the one before and go through LDS too (a load inside the loop
 // over the degrees would wait for the stores before it).  Cells of more than
-// 4 KS atoms take several passes that add up in `mom`.  336 and 1,637 us
-// (422 and 1,560 with the constants loaded per degree), bound by the latency
+// 4 KS atoms take several passes that add up in `mom`.  The mixed path sums the
+// degrees below kHarmExactL in FP64: the terms of a cell's low moments mostly
+// cancel, and the rest is common to all nodes.  345 and 1,637 us
+// (336 with all sums in FP32, 422 and 1,560 with the constants loaded per degree), bound by the latency
 // of the LDS reads between the products: 59 % of the wave cycles wait.  FP32
 // takes 64 atoms a pass (more registers leave fewer waves: 388 us at 128),
 // FP64 up to 128 (1,880 us at 64).
@@ -293,6 +296,8 @@ __device__ __forceinline__ void harm_moments_body(
   const uint32_t pr = M::perm(c16);  // radial index of this lane's A row
   const uint32_t row0 = (pr < prow ? pr : prow - 1) * AS + g;
   const uint32_t row1 = (16 + pr < prow ? 16 + pr : prow - 1) * AS + g;
+  const uint32_t low0 = (c16 < prow ? c16 : prow - 1) * AS + g;
+  const uint32_t low1 = (16 + c16 < prow ? 16 + c16 : prow - 1) * AS + g;
   const uint32_t mu = 8 * t + (c16 >> 1);
   for (uint32_t p0 = 0; p0 == 0 || p0 < na; p0 += CH) {
     const uint32_t cnt = na - p0 < CH ? na - p0 : CH;
@@ -344,27 +349,35 @@ __device__ __forceinline__ void harm_moments_body(
       const T *rc = H.rec + (static_cast<size_t>(rl) * 64 + rm) * 2;
       T rnext = rl < LB ? rc[0] : T(0);
       T *o = out + (H.qoff[t] + H.crow[8 * t]) * 16 + lane;
-      // one degree: PT row tiles of radial polynomials
+      // one degree: PT row tiles of radial polynomials, LOW: the sums in FP64
       // A: Y of the degree before; B: of the one before that, then of this
-      auto degree = [&](auto tiles, uint32_t l, T(&A)[NK], T(&B)[NK]) {
+      auto degree = [&](auto tiles, auto low, uint32_t l, T(&A)[NK],
+                        T(&B)[NK]) {
         constexpr int PT = decltype(tiles)::value;
+        constexpr bool LOW = decltype(low)::value != 0;
         const uint32_t PK = harm_psteps(l, N);
         const T *zl = zt + (l % LB) * prow * AS;
         const T rb = rec[(l % LB) * 8 * nwave + mu];
         const T ra = l > mu ? T(1) : T(0), one = T(1) - ra;
         // (partial sums: the rounding of a sum grows with its length)
-        constexpr int NA = sizeof(T) == 4 ? 4 / PT : 1;
-        v4 a0s[NA], a1s[NA];
+        constexpr int NA = sizeof(T) == 4 && !LOW ? 4 / PT : 1;
+        using S = std::conditional_t<LOW, double, T>;
+        using MS = Harm<S>;
+        using s4 = typename MS::v4;
+        s4 a0s[NA], a1s[NA];
 #pragma unroll
         for (int i = 0; i < NA; ++i)
-          a0s[i] = a1s[i] = v4{T(0), T(0), T(0), T(0)};
+          a0s[i] = a1s[i] = s4{S(0), S(0), S(0), S(0)};
 #pragma unroll
         for (int k = 0; k < NK; ++k) {
           const T z = zs[2 * (4 * k + g)], s = zs[2 * (4 * k + g) + 1];
           const T y = harm_fma(harm_fma(ra, z, one), A[k], -(rb * s) * B[k]);
           B[k] = y;
-          a0s[k % NA] = M::mfma(zl[row0 + 4 * k], y, a0s[k % NA]);
-          if (PT > 1) a1s[k % NA] = M::mfma(zl[row1 + 4 * k], y, a1s[k % NA]);
+          a0s[k % NA] = MS::mfma(static_cast<S>(zl[(LOW ? low0 : row0) + 4 * k]),
+                                 static_cast<S>(y), a0s[k % NA]);
+          if (PT > 1)
+            a1s[k % NA] = MS::mfma(static_cast<S>(zl[(LOW ? low1 : row1) + 4 * k]),
+                                   static_cast<S>(y), a1s[k % NA]);
         }
 #pragma unroll
         for (int w = NA / 2; w > 0; w /= 2)
@@ -373,7 +386,12 @@ __device__ __forceinline__ void harm_moments_body(
             a0s[i] += a0s[i + w];
             if (PT > 1) a1s[i] += a1s[i + w];
           }
-        v4 acc0 = a0s[0], acc1 = a1s[0];
+        v4 acc0, acc1;
+#pragma unroll
+        for (uint32_t r = 0; r < 4; ++r) {
+          acc0[r] = static_cast<T>(a0s[0][r]);
+          acc1[r] = static_cast<T>(a1s[0][r]);
+        }
         // orders above the degree are zero; register r holds the rows
         // p = 4 r + g
 #pragma unroll
@@ -413,16 +431,20 @@ __device__ __forceinline__ void harm_moments_body(
         }
         harm_barrier();
         for (uint32_t l = l0 < 8 * t ? 8 * t : l0; l < l0 + nl; l += 2) {
-          if (harm_psteps(l, N) > 4)
-            degree(HarmInt<2>{}, l, Y1, Y2);
-          else
-            degree(HarmInt<1>{}, l, Y1, Y2);
-          if (l + 1 < N) {
-            if (harm_psteps(l + 1, N) > 4)
-              degree(HarmInt<2>{}, l + 1, Y2, Y1);
-            else
-              degree(HarmInt<1>{}, l + 1, Y2, Y1);
-          }
+          auto one = [&](uint32_t d, T(&A)[NK], T(&B)[NK]) {
+            if (sizeof(T) == 4 && d < kHarmExactL) {
+              if (harm_psteps(d, N) > 4)
+                degree(HarmInt<2>{}, HarmInt<1>{}, d, A, B);
+              else
+                degree(HarmInt<1>{}, HarmInt<1>{}, d, A, B);
+            } else if (harm_psteps(d, N) > 4) {
+              degree(HarmInt<2>{}, HarmInt<0>{}, d, A, B);
+            } else {
+              degree(HarmInt<1>{}, HarmInt<0>{}, d, A, B);
+            }
+          };
+          one(l, Y1, Y2);
+          if (l + 1 < N) one(l + 1, Y2, Y1);
         }
         harm_barrier();
       }
@@ -458,127 +480,159 @@ constexpr int harm_max_psteps() {
 // One wave: degree l and order tile t of the eight cells of a tile.  Forward:
 // B_i = sum_p gam_l[i][p] Q[p] for the radial nodes with more than l degrees,
 // the moments in registers for all eight cells; a lane ends with the eight
-// cells' values of one (node, column), adjacent in the coefficients.  73 and
-// 369 us forward, 108 and 286 us backward: memory traffic of the coefficients
-// (0.25 and 1.0 GB).
-template <typename T>
+// cells' values of one (node, column), adjacent in the coefficients.  74 and
+// 369 us forward, 107 and 286 us backward: memory traffic of the coefficients
+// (0.25 and 1.0 GB), behind which the FP64 products of the mixed path's low
+// degrees (see kHarmExactL) cost nothing.
+// CT: the type of the products; with FP64 products of FP32 data (the low
+// degrees) four cells at a time, so that the registers stay those of the rest.
+template <typename T, typename CT>
 __device__ __forceinline__ void harm_forward_wave(const HarmDev<T> &H,
                                                   uint32_t ncell, uint32_t tile,
                                                   uint32_t l, uint32_t t,
                                                   const T *mom, T *coef) {
-  using M = Harm<T>;
+  using M = Harm<CT>;
   using v4 = typename M::v4;
+  using o4 = typename Harm<T>::v4;
   constexpr int MAXPK = harm_max_psteps<T>();
+  constexpr bool LOW = sizeof(CT) != sizeof(T);
+  constexpr uint32_t NC = LOW ? 4 : 8;
   const uint32_t lane = threadIdx.x & 63u, c16 = lane & 15u, g = lane >> 4;
   const uint4 lr = H.lrow[l];
   const size_t cs = static_cast<size_t>(H.rows) * 16;
   const T *Q = mom + static_cast<size_t>(H.qoff[t] + H.crow[l]) * 16 + lane;
   T *out = coef + static_cast<size_t>(tile) * H.stride * 8;
+  const CT *gam;
+  if constexpr (LOW)
+    gam = H.gam64 + static_cast<size_t>(H.lrow64[l].x) * 64 + lane;
+  else
+    gam = H.gam + static_cast<size_t>(lr.x) * 64 + lane;
   harm_switch<MAXPK>(harm_psteps(l, H.N), [&](auto steps) {
     constexpr int PK = decltype(steps)::value;
-    T q[8][PK];
+#pragma unroll 1
+    for (uint32_t c0 = 0; c0 < 8; c0 += NC) {
+      CT q[NC][PK];
 #pragma unroll
-    for (uint32_t c = 0; c < 8; ++c) {
-      const uint32_t cell = tile * 8 + c < ncell ? tile * 8 + c : ncell - 1;
-      const T *p = Q + cell * cs;
+      for (uint32_t c = 0; c < NC; ++c) {
+        const uint32_t k = tile * 8 + c0 + c;
+        const T *p = Q + (k < ncell ? k : ncell - 1) * cs;
 #pragma unroll
-      for (int r = 0; r < PK; ++r) q[c][r] = p[r * 64];
-    }
-    const T *G = H.gam + static_cast<size_t>(lr.x) * 64 + lane;
-    T gm[PK];
-#pragma unroll
-    for (int r = 0; r < PK; ++r) gm[r] = G[r * 64];
-    for (uint32_t i0 = 0; i0 < lr.z; i0 += 16) {
-      T gx[PK];
-#pragma unroll
-      for (int r = 0; r < PK; ++r) gx[r] = gm[r];
-      G += PK * 64;  // (the table has room for one more load)
+        for (int r = 0; r < PK; ++r) q[c][r] = p[r * 64];
+      }
+      const CT *G = gam;
+      CT gm[PK];
 #pragma unroll
       for (int r = 0; r < PK; ++r) gm[r] = G[r * 64];
-      HarmRad ri[4];
+      for (uint32_t i0 = 0; i0 < lr.z; i0 += 16) {
+        CT gx[PK];
 #pragma unroll
-      for (uint32_t r = 0; r < 4; ++r) {
-        const uint32_t i = i0 + M::row(g, r);
-        ri[r] = H.rad[i < H.nrad ? i : H.nrad - 1];
-      }
-      v4 d[8];
+        for (int r = 0; r < PK; ++r) gx[r] = gm[r];
+        G += PK * 64;  // (the table has room for one more load)
 #pragma unroll
-      for (uint32_t c = 0; c < 8; ++c) d[c] = v4{T(0), T(0), T(0), T(0)};
+        for (int r = 0; r < PK; ++r) gm[r] = G[r * 64];
+        HarmRad ri[4];
 #pragma unroll
-      for (int r = 0; r < PK; ++r)
-#pragma unroll
-        for (uint32_t c = 0; c < 8; ++c) d[c] = M::mfma(gx[r], q[c][r], d[c]);
-#pragma unroll
-      for (uint32_t r = 0; r < 4; ++r)
-        if (i0 + M::row(g, r) < lr.z) {
-          v4 *o = reinterpret_cast<v4 *>(
-              out + (ri[r].off + harm_block(t, l, ri[r].N) * 16 + c16) * 8);
-          o[0] = v4{d[0][r], d[1][r], d[2][r], d[3][r]};
-          o[1] = v4{d[4][r], d[5][r], d[6][r], d[7][r]};
+        for (uint32_t r = 0; r < 4; ++r) {
+          const uint32_t i = i0 + M::row(g, r);
+          ri[r] = H.rad[i < H.nrad ? i : H.nrad - 1];
         }
+        v4 d[NC];
+#pragma unroll
+        for (uint32_t c = 0; c < NC; ++c)
+          d[c] = v4{CT(0), CT(0), CT(0), CT(0)};
+#pragma unroll
+        for (int r = 0; r < PK; ++r)
+#pragma unroll
+          for (uint32_t c = 0; c < NC; ++c)
+            d[c] = M::mfma(gx[r], q[c][r], d[c]);
+#pragma unroll
+        for (uint32_t r = 0; r < 4; ++r)
+          if (i0 + M::row(g, r) < lr.z) {
+            T *o = out +
+                   (ri[r].off + harm_block(t, l, ri[r].N) * 16 + c16) * 8 + c0;
+#pragma unroll
+            for (uint32_t c = 0; c < NC; c += 4)
+              *reinterpret_cast<o4 *>(o + c) =
+                  o4{static_cast<T>(d[c][r]), static_cast<T>(d[c + 1][r]),
+                     static_cast<T>(d[c + 2][r]), static_cast<T>(d[c + 3][r])};
+          }
+      }
     }
   });
 }
 
 // Backward: U[p] = sum_i gam_l[i][p] C_i, per (l, order) the pairs (cosine,
 // sine) of the rows p side by side.
-template <typename T>
+template <typename T, typename CT>
 __device__ __forceinline__ void harm_backward_wave(const HarmDev<T> &H,
                                                    uint32_t ncell,
                                                    uint32_t tile, uint32_t l,
                                                    uint32_t t, const T *coef,
                                                    T *mom) {
-  using M = Harm<T>;
+  using M = Harm<CT>;
   using v4 = typename M::v4;
+  using i4 = typename Harm<T>::v4;
+  constexpr bool LOW = sizeof(CT) != sizeof(T);
+  constexpr uint32_t NC = LOW ? 4 : 8;
   const uint32_t lane = threadIdx.x & 63u, c16 = lane & 15u, g = lane >> 4;
   const uint32_t PK = harm_psteps(l, H.N);
   const uint4 lr = H.lrow[l];
   const uint32_t mu = 8 * t + (c16 >> 1);
-  const T *G = H.gamt + static_cast<size_t>(lr.y) * 64 + lane;
+  const CT *gamt;
+  if constexpr (LOW)
+    gamt = H.gamt64 + static_cast<size_t>(H.lrow64[l].y) * 64 + lane;
+  else
+    gamt = H.gamt + static_cast<size_t>(lr.y) * 64 + lane;
   const T *in = coef + static_cast<size_t>(tile) * H.stride * 8 + c16 * 8;
   T *o = mom + 8 * (H.urow[l] + mu * PK) + 2 * g + (c16 & 1u);
   harm_switch<2>(PK > 4 ? 2u : 1u, [&](auto tiles) {
     constexpr int PT = decltype(tiles)::value;
-    v4 d[PT][8];
+#pragma unroll 1
+    for (uint32_t c0 = 0; c0 < 8; c0 += NC) {
+      const CT *G = gamt;
+      v4 d[PT][NC];
 #pragma unroll
-    for (int p = 0; p < PT; ++p)
+      for (int p = 0; p < PT; ++p)
 #pragma unroll
-      for (uint32_t c = 0; c < 8; ++c) d[p][c] = v4{T(0), T(0), T(0), T(0)};
-    // four radial nodes a step, two steps in flight; nodes past the last
-    // have zero factors and repeat it
-    for (uint32_t i0 = 0; i0 < lr.z; i0 += 8) {
-      v4 b[2][2];
-      T ga[2][PT];
+        for (uint32_t c = 0; c < NC; ++c)
+          d[p][c] = v4{CT(0), CT(0), CT(0), CT(0)};
+      // four radial nodes a step, two steps in flight; nodes past the last
+      // have zero factors and repeat it
+      for (uint32_t i0 = 0; i0 < lr.z; i0 += 8) {
+        i4 b[2][NC / 4];
+        CT ga[2][PT];
 #pragma unroll
-      for (uint32_t u = 0; u < 2; ++u) {
-        const uint32_t i = i0 + 4 * u + g;
-        const HarmRad ri = H.rad[i < lr.z ? i : lr.z - 1];
-        const v4 *p = reinterpret_cast<const v4 *>(
-            in + (ri.off + harm_block(t, l, ri.N) * 16) * 8);
-        b[u][0] = p[0];
-        b[u][1] = p[1];
+        for (uint32_t u = 0; u < 2; ++u) {
+          const uint32_t i = i0 + 4 * u + g;
+          const HarmRad ri = H.rad[i < lr.z ? i : lr.z - 1];
+          const i4 *p = reinterpret_cast<const i4 *>(
+              in + (ri.off + harm_block(t, l, ri.N) * 16) * 8 + c0);
 #pragma unroll
-        for (int p2 = 0; p2 < PT; ++p2) {
-          const T x = G[(u * PT + p2) * 64];
-          ga[u][p2] = i0 + 4 * u < lr.z ? x : T(0);
+          for (uint32_t c = 0; c < NC / 4; ++c) b[u][c] = p[c];
+#pragma unroll
+          for (int p2 = 0; p2 < PT; ++p2) {
+            const CT x = G[(u * PT + p2) * 64];
+            ga[u][p2] = i0 + 4 * u < lr.z ? x : CT(0);
+          }
         }
+        G += 2 * PT * 64;
+#pragma unroll
+        for (uint32_t u = 0; u < 2; ++u)
+#pragma unroll
+          for (int p = 0; p < PT; ++p)
+#pragma unroll
+            for (uint32_t c = 0; c < NC; ++c)
+              d[p][c] = M::mfma(ga[u][p], static_cast<CT>(b[u][c >> 2][c & 3u]),
+                                d[p][c]);
       }
-      G += 2 * PT * 64;
 #pragma unroll
-      for (uint32_t u = 0; u < 2; ++u)
+      for (uint32_t c = 0; c < NC; ++c) {
+        if (tile * 8 + c0 + c >= ncell) break;
+        T *p = o + static_cast<size_t>(tile * 8 + c0 + c) * H.ustride;
 #pragma unroll
-        for (int p = 0; p < PT; ++p)
-#pragma unroll
-          for (uint32_t c = 0; c < 8; ++c)
-            d[p][c] = M::mfma(ga[u][p], b[u][c >> 2][c & 3u], d[p][c]);
-    }
-#pragma unroll
-    for (uint32_t c = 0; c < 8; ++c) {
-      if (tile * 8 + c >= ncell) break;
-      T *p = o + static_cast<size_t>(tile * 8 + c) * H.ustride;
-#pragma unroll
-      for (uint32_t r = 0; r < 4 * PT; ++r)
-        if (r < PK && mu <= l) p[r * 8] = d[r >> 2][c][r & 3u];
+        for (uint32_t r = 0; r < 4 * PT; ++r)
+          if (r < PK && mu <= l) p[r * 8] = static_cast<T>(d[r >> 2][c][r & 3u]);
+      }
     }
   });
 }
@@ -586,7 +640,7 @@ __device__ __forceinline__ void harm_backward_wave(const HarmDev<T> &H,
 // Wave w of a launch: tile w / (pairs) and the (l, t) pair w % pairs of the
 // plan.
 template <typename T, bool BACK>
-__global__ __launch_bounds__(256) void harm_radial_kernel(
+__global__ __launch_bounds__(256, sizeof(T) == 4 ? 4 : 2) void harm_radial_kernel(
     HarmDev<T> H, uint32_t ncell, uint32_t nwave, const T *__restrict__ in,
     T *__restrict__ out) {
   const uint32_t nb = gridDim.x, b = blockIdx.x;
@@ -597,14 +651,21 @@ __global__ __launch_bounds__(256) void harm_radial_kernel(
   if (w >= nwave) return;
   const uint32_t tile = w / H.npair;
   const uint2 lt = H.pair[w - tile * H.npair];
-  if (BACK)
-    harm_backward_wave(H, ncell, tile, lt.x, lt.y, in, out);
-  else
-    harm_forward_wave(H, ncell, tile, lt.x, lt.y, in, out);
+  if (sizeof(T) == 4 && lt.x < kHarmExactL) {
+    if (BACK)
+      harm_backward_wave<T, double>(H, ncell, tile, lt.x, lt.y, in, out);
+    else
+      harm_forward_wave<T, double>(H, ncell, tile, lt.x, lt.y, in, out);
+  } else if (BACK) {
+    harm_backward_wave<T, T>(H, ncell, tile, lt.x, lt.y, in, out);
+  } else {
+    harm_forward_wave<T, T>(H, ncell, tile, lt.x, lt.y, in, out);
+  }
 }
 
 // ---------------------------------------------------------------------------
-// coefficients -> structure factors (374 and 943 us, 400 and 1,131 with the
+// coefficients -> structure factors (397 and 943 us; mixed 374 with the lowest
+// orders in FP32 too, before that 400 and 1,131 with the
 // azimuths up to pi summed one by one, 415 and 1,194 before that with a select
 // per coefficient; the workgroups' phases between barriers, two to three
 // workgroups per CU, against 0.15 and 0.29 ms of stores)
@@ -679,6 +740,15 @@ __device__ __forceinline__ void harm_sf_body(
   constexpr uint32_t kRow = 256 * sizeof(T);  // from a degree to the next but one
   const uint32_t brow = g * kRow + c16 * sizeof(T);
   const T *leg = H.leg + (static_cast<size_t>(gr.leg) + rt * gr.leg_n) * 64 + lane;
+  // the FP64 factors of the sets' lowest orders (mixed, the last two waves)
+  const bool low = F && wave >= NW - 2;
+  uint32_t at64[2] = {0u, 0u};
+  if (low) {
+#pragma unroll
+    for (uint32_t set = 0; set < 2; ++set)
+      at64[set] = gr.leg64 + rt * gr.leg64_n +
+                  H.mup64[gr.mup64 + 2 * set + wave - (NW - 2)].x;
+  }
   for (uint32_t pass = 0; pass < (F ? 1u : 2u); ++pass) {
     v4 E[2][NR][NPT];
 #pragma unroll
@@ -713,8 +783,35 @@ __device__ __forceinline__ void harm_sf_body(
           }
         }
       };
-      if (2 * wave + set < N) fetch(2 * wave + set);
-      for (uint32_t m = wave; m < MH; m += NW) {
+      // the lowest order of the set (mixed): the same products in FP64, by
+      // the last two waves, which have fewer orders than the first ones
+      const uint32_t m0 = F && wave == 0 ? NW : wave;
+      if (2 * m0 + set < N) fetch(2 * m0 + set);
+      if (low) {
+        const uint32_t par = wave - (NW - 2);
+        uint32_t l0;
+        const uint32_t n = degrees(set, par, l0);
+        const double *A = H.leg64 + static_cast<size_t>(at64[set]) * 64 + lane;
+        const T *B = cf + (n ? harm_block(0, l0, N) * 16 + 2 * set : 0u) * 8;
+        harm_d4 acc = {0.0, 0.0, 0.0, 0.0};
+        for (uint32_t k = 0; k < n; k += 16) {
+          double x[4];
+          T y[4];
+#pragma unroll
+          for (uint32_t u = 0; u < 4; ++u) {
+            x[u] = A[(k + 4 * u) * 16];  // (four more steps in the table)
+            y[u] = harm_ranged(B, n * kRow, brow + (k + 4 * u) * kRow);
+          }
+#pragma unroll
+          for (uint32_t u = 0; u < 4; ++u)
+            acc = Harm<double>::mfma(x[u], static_cast<double>(y[u]), acc);
+        }
+#pragma unroll
+        for (uint32_t r = 0; r < 4; ++r)
+          Gm[Harm<double>::row(g, r) * RS + cs * sines + c8 * 2 + par] =
+              static_cast<T>(acc[r]);
+      }
+      for (uint32_t m = m0; m < MH; m += NW) {
         const uint32_t mu = 2 * m + set;
         const uint32_t mode = cs * sines + m * 16;
         v4 acc[NP];
@@ -924,7 +1021,8 @@ __global__ __launch_bounds__(kHarmBlock) void harm_sf_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// remote sums -> coefficients (420 and 1,162 us, 438 and 1,311 with the azimuths
+// remote sums -> coefficients (436 and 1,162 us; mixed 420 with the lowest
+// orders in FP32 too, before that 438 and 1,311 with the azimuths
 // up to pi summed one by one and every group in the registers of the largest;
 // reads R once, 0.15 and 0.29 ms, all loads of a workgroup in flight, then the
 // phases between barriers as in harm_sf)
@@ -937,7 +1035,12 @@ __global__ __launch_bounds__(kHarmBlock) void harm_sf_kernel(
 // V(phi) +- V(phi + pi), and f(phi) +- f(pi - phi) summed over the azimuths up
 // to pi / 2 against the cosines and, with the other sign, the sines;
 // (2) per order and parity, the sums over the rings against the Legendre
-// functions, stored as the cells' coefficients.
+// functions, stored as the cells' coefficients.  The mixed path keeps the ring
+// sums of each set's lowest order apart (`low`) and sums them over the rings in
+// FP64 at the end, when the registers of the loaded values are free (inside
+// the loop over the sets it spilled 120 of them: 3,824 against 4,461 us for
+// the way back at 1.0M charges).
+constexpr uint32_t kHarmLowRow = 40;  // scalars of a ring
 template <typename T, int RW, int HK, int MT>
 __device__ __forceinline__ void harm_lr_body(
     const HarmDev<T> &H, uint32_t ncell, const HarmRad &rad,
@@ -955,7 +1058,8 @@ __device__ __forceinline__ void harm_lr_body(
   const uint32_t hk = gr.trigt_k;
   const uint32_t nrow = F ? 4 * gr.legt_k : 2 * gr.legt_k;  // padded rings
   T *Gm = reinterpret_cast<T *>(smem);
-  T *tr = Gm + nrow * RS;
+  T *low = Gm + nrow * RS;  // mixed: [set][ring], the set's lowest order
+  T *tr = low + (F ? 2 * nrow * kHarmLowRow : 0u);
   const uint32_t cell0 = tile * kHarmCells;
   const uint32_t ncp = harm_row(ncell);
   // columns of (2): the cosines of the eight cells, then the sines
@@ -965,6 +1069,15 @@ __device__ __forceinline__ void harm_lr_body(
   // bytes of an azimuth: a row's offsets stay below 4 h of them (32 bits)
   const uint32_t az = static_cast<uint32_t>(2 * ncp * sizeof(T));
   const uint32_t nd = harm_dirs(gr);
+  // the FP64 factors of a set's lowest order, waves (set, parity)
+  // (asked for ahead of the last phase, except where the registers are held
+  // to most waves)
+  constexpr bool PRE = F && RW > 2;
+  auto factors64 = [&] {
+    return H.legt64 + lane +
+           (static_cast<size_t>(gr.legt64) + H.mup64[gr.mup64 + wave].y) * 64;
+  };
+  double x64[4] = {};
   for (uint32_t pass = 0; pass < (F ? 1u : 2u); ++pass) {
     // A row past the rings and an azimuth past pi / 2 repeat the last one
     // (their factors are zero); the equator has no second half.  phi = 0 and
@@ -1019,7 +1132,9 @@ __device__ __forceinline__ void harm_lr_body(
           for (uint32_t u = 0; u < 4; ++u) la[pp][u] = A[u * 64];
         }
       };
-      if (2 * wave + set < N) fetch(2 * wave + set);
+      // (mixed: the lowest order comes last, in FP64)
+      const uint32_t m0 = F && wave == 0 ? NW : wave;
+      if (2 * m0 + set < N) fetch(2 * m0 + set);
       // (1)
 #pragma unroll
       for (int w = 0; w < RW; ++w) {
@@ -1051,13 +1166,21 @@ __device__ __forceinline__ void harm_lr_body(
 #pragma unroll
               for (uint32_t r = 0; r < 4; ++r) {
                 const uint32_t mode = 2 * (16 * m + M::row(g, r)) + c;
-                if (mode < MS) Gm[row * RS + mode * 16 + c16] = acc[c][m][r];
+                uint32_t to = row * RS + mode * 16 + c16;
+                if (F && m == 0 && r == 0 && g == 0)  // order `set`
+                  to = (nrow * RS + (set * nrow + row) * kHarmLowRow) +
+                       c * 16 + c16;
+                if (mode < MS) Gm[to] = acc[c][m][r];
               }
         }
       }
       harm_barrier();
       // (2)
-      for (uint32_t m = wave; 2 * m + set < N; m += NW) {
+      if (PRE && set == 1 && wave < 4) {
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) x64[u] = factors64()[u * 64];
+      }
+      for (uint32_t m = m0; 2 * m + set < N; m += NW) {
         const uint32_t mu = 2 * m + set;
         const uint32_t mode = 2 * m + cs;
         T xa[NP][4];
@@ -1110,6 +1233,40 @@ __device__ __forceinline__ void harm_lr_body(
         }
       }
       harm_barrier();
+    }
+  }
+  if constexpr (F) {
+    // (2) of the lowest order of each set in FP64, wave (set, parity)
+    const uint32_t set = wave >> 1, par = wave & 1u;
+    const uint32_t l0 = set + ((set ^ par) & 1u);
+    if (set < 2 && l0 < N) {
+      const uint32_t n = (N - l0 + 1) / 2;
+      const double *A = factors64();
+      const T *sums = low + set * nrow * kHarmLowRow + cs * 16 + c8 * 2 + par;
+      T *o = cf + (harm_block(0, l0, N) * 16 + 2 * set) * 8;
+      for (uint32_t i0 = 0; i0 < n; i0 += 16) {
+        harm_d4 acc = {0.0, 0.0, 0.0, 0.0};
+        for (uint32_t k = 0; k < gr.legt_k; k += 4) {
+          if (!PRE || i0 + k > 0) {
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u)
+              x64[u] = A[(k + u < gr.legt_k ? k + u : k) * 64];
+          }
+#pragma unroll
+          for (uint32_t u = 0; u < 4; ++u)
+            if (k + u < gr.legt_k)
+              acc = Harm<double>::mfma(
+                  x64[u],
+                  static_cast<double>(sums[(4 * (k + u) + g) * kHarmLowRow]),
+                  acc);
+        }
+#pragma unroll
+        for (uint32_t r = 0; r < 4; ++r) {
+          const uint32_t i = i0 + Harm<double>::row(g, r);
+          if (i < n) o[i * 256] = static_cast<T>(acc[r]);
+        }
+        A += gr.legt_k * 64;
+      }
     }
   }
 }
@@ -1459,6 +1616,7 @@ size_t harm_lds_lr(uint32_t N, uint32_t h, uint32_t nring) {
   const size_t lk = std::max<size_t>(4, (nring + 3) / 4);
   const size_t top = harm_lr_steps(harm_lr_class((h / 2 + 4) / 4));
   return ((sizeof(T) == 4 ? 4 : 2) * lk * (128 * KC + 8) +
+          (sizeof(T) == 4 ? 2 * 4 * lk * kHarmLowRow : 0) +
           4 * ((KC + 3) / 4) * top * 64) *
          sizeof(T);
 }

@@ -62,6 +62,15 @@ __host__ __device__ inline uint32_t harm_psteps(uint32_t l, uint32_t N) {
   return ((N - 1 - l) / 2 + 4) / 4;
 }
 
+// Mixed path: the products of the lowest degrees (radial) and orders (Legendre)
+// that are formed in FP64, from FP32 operands and FP64 tables, and stored in
+// FP32.  Their rounding is common to all directions of a radial node (degree
+// 0) or all azimuths of a ring (order 0) and so does not average out: with FP32
+// products it was nearly all of the far field's error, whose rms over 15 water
+// boxes was 3.2e-7 in the forces and 2.9e-7 in the energies against 2.6e-7 and
+// 1.4e-7 of the direct sums, and is 2.0e-7 and 1.3e-7.
+constexpr uint32_t kHarmExactL = 4, kHarmExactMu = 2;
+
 // One radial node.
 struct HarmRad {
   uint32_t N;      // degrees
@@ -85,6 +94,9 @@ struct HarmGroup {
   // (cs 0: cosines, 1: sines), trig_t tiles, and back [set][cs][tile][step]
   uint32_t trig, trig_k, trig_t;
   uint32_t trigt, trigt_m, trigt_k;
+  // the FP64 copies of leg and legt for the orders below kHarmExactMu, and
+  // their offsets, four (order, parity) entries of HarmDev::mup64
+  uint32_t leg64, leg64_n, legt64, mup64;
 };
 
 // directions of a group
@@ -102,6 +114,10 @@ struct HarmDev {
   const T *gam, *gamt;    // radial matrices: moments -> radial nodes and back
   const uint4 *lrow;      // per degree l: gam, gamt offsets, radial nodes with
                           // N_i > l
+  // mixed: FP64 tables of the low degrees and orders; offsets by degree into
+  // gam64 and gamt64, by (group, order, parity) into leg64 and legt64
+  const double *leg64, *legt64, *gam64, *gamt64;
+  const uint2 *lrow64, *mup64;
   const uint2 *pair;      // npair (degree, order tile) pairs
   const uint32_t *crow;   // rows of the degrees below l
   const uint32_t *urow;   // groups of the contracted coefficients below l

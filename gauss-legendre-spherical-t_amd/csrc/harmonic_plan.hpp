@@ -93,6 +93,8 @@ struct HarmTables {
   std::vector<dev::HarmGroup> grp;
   std::vector<uint2> mup;
   std::vector<double> leg, legt, trig, trigt, gam, gamt, jac, rec;
+  std::vector<double> leg64, legt64, gam64, gamt64;  // mixed (HarmDev)
+  std::vector<uint2> lrow64, mup64;
   std::vector<uint4> lrow;
   std::vector<uint2> pair;  // (degree, order tile)
   std::vector<uint32_t> crow, urow, qoff;
@@ -107,11 +109,13 @@ struct HarmTables {
   size_t bytes(size_t real) const {
     return (leg.size() + legt.size() + trig.size() + trigt.size() +
             gam.size() + gamt.size() + jac.size() + rec.size()) * real +
+           (leg64.size() + legt64.size() + gam64.size() + gamt64.size()) * 8 +
+           (lrow64.size() + mup64.size()) * sizeof(uint2) +
            rad.size() * sizeof(rad[0]) + grp.size() * sizeof(grp[0]) +
            (mup.size() + pair.size() + unit.size()) * sizeof(uint2) +
            lrow.size() * sizeof(uint4) + (crow.size() + urow.size()) * 4 +
            (node_of_row.size() + 256) * sizeof(double4) +
-           20 * 256;
+           26 * 256;
   }
 };
 
@@ -261,32 +265,43 @@ inline HarmTables plan_harmonic(const NodeTable &nodes, double h,
     const double v = static_cast<double>(gn[i][n] * kap[l][p]);
     return p % 2 ? -v : v;
   };
-  // row R of a chained product stands for this index (Harm<T>::perm)
-  auto perm = [&](uint32_t R) { return single ? 4 * (R & 3u) + (R >> 2) : R; };
+  // row R of a chained FP32 product stands for index 4 (R % 4) + R / 4
+  // (Harm<float>::perm)
+  auto radial = [&](uint32_t l, bool fp32, std::vector<double> &gam,
+                    std::vector<double> &gamt) {
+    auto perm = [&](uint32_t R) { return fp32 ? 4 * (R & 3u) + (R >> 2) : R; };
+    const uint32_t PK = dev::harm_psteps(l, N);
+    uint32_t above = 0;  // radial nodes with more than l degrees
+    while (above < nrad && T.rad[above].N > l) ++above;
+    for (uint32_t i0 = 0; i0 < above; i0 += 16)
+      for (uint32_t k = 0; k < PK; ++k)
+        for (uint32_t a = 0; a < 64; ++a)
+          gam.push_back(gamma(i0 + a % 16, l, 4 * k + a / 16));
+    for (uint32_t i0 = 0; i0 < above; i0 += 4)
+      for (uint32_t t = 0; t < (PK > 4 ? 2u : 1u); ++t)
+        for (uint32_t a = 0; a < 64; ++a)
+          gamt.push_back(gamma(i0 + a / 16, l, 16 * t + perm(a % 16)));
+    return above;
+  };
+  auto at = [](const std::vector<double> &v) {
+    return static_cast<uint32_t>(v.size() / 64);
+  };
   for (uint32_t l = 0; l < N; ++l) {
-    uint4 r = make_uint4(static_cast<uint32_t>(T.gam.size() / 64),
-                         static_cast<uint32_t>(T.gamt.size() / 64), 0, 0);
-    {
-      const uint32_t PK = dev::harm_psteps(l, N);
-      while (r.z < nrad && T.rad[r.z].N > l) ++r.z;
-      for (uint32_t i0 = 0; i0 < r.z; i0 += 16)
-        for (uint32_t k = 0; k < PK; ++k)
-          for (uint32_t a = 0; a < 64; ++a)
-            T.gam.push_back(gamma(i0 + a % 16, l, 4 * k + a / 16));
-      for (uint32_t i0 = 0; i0 < r.z; i0 += 4)
-        for (uint32_t t = 0; t < (PK > 4 ? 2u : 1u); ++t)
-          for (uint32_t a = 0; a < 64; ++a)
-            T.gamt.push_back(gamma(i0 + a / 16, l, 16 * t + perm(a % 16)));
-    }
+    uint4 r = make_uint4(at(T.gam), at(T.gamt), 0, 0);
+    r.z = radial(l, single, T.gam, T.gamt);
     T.lrow.push_back(r);
+    if (single && l < dev::kHarmExactL) {
+      T.lrow64.push_back(make_uint2(at(T.gam64), at(T.gamt64)));
+      radial(l, false, T.gam64, T.gamt64);
+    }
   }
   // Legendre functions on the rings and Fourier matrices
   uint32_t hmax = 0;  // (one launch for all groups)
   for (size_t g = 0; g < ng; ++g) {
     dev::HarmGroup &G = T.grp[g];
     G.mup = static_cast<uint32_t>(T.mup.size());
-    G.leg = static_cast<uint32_t>(T.leg.size() / 64);
-    G.legt = static_cast<uint32_t>(T.legt.size() / 64);
+    G.leg = at(T.leg);
+    G.legt = at(T.legt);
     G.legt_k = std::max<uint32_t>(4, (G.nring + 3) / 4);
     const uint32_t nrt = (G.nring + 15) / 16;
     // pl[ring][mu][l], with the sign of (-i)^l: even degrees give the real
@@ -319,29 +334,38 @@ inline HarmTables plan_harmonic(const NodeTable &nodes, double h,
                  ? pl[(static_cast<size_t>(j) * G.N + m) * G.N + l]
                  : 0.0;
     };
-    std::vector<double> one;  // one ring tile
-    for (uint32_t rt = 0; rt < nrt; ++rt) {
-      one.clear();
-      for (uint32_t m = 0; m < G.N; ++m)
-        for (uint32_t par = 0; par < 2; ++par) {
-          const uint32_t l0 = m + ((m ^ par) & 1u);
-          const uint32_t n = l0 < G.N ? (G.N - l0 + 1) / 2 : 0u;
-          if (rt == 0)
-            T.mup.push_back(make_uint2(
-                static_cast<uint32_t>(one.size() / 64),
-                static_cast<uint32_t>(T.legt.size() / 64) - G.legt));
-          for (uint32_t k = 0; k < n; k += 4)
-            for (uint32_t a = 0; a < 64; ++a)
-              one.push_back(P(16 * rt + a % 16, m, l0 + 2 * (k + a / 16)));
-          if (rt == 0)
-            for (uint32_t i0 = 0; i0 < n; i0 += 16)
-              for (uint32_t ks = 0; ks < G.legt_k; ++ks)
-                for (uint32_t a = 0; a < 64; ++a)
-                  T.legt.push_back(
-                      P(4 * ks + a / 16, m, l0 + 2 * (i0 + a % 16)));
-        }
-      G.leg_n = static_cast<uint32_t>(one.size() / 64);
-      T.leg.insert(T.leg.end(), one.begin(), one.end());
+    // orders below `orders` of every ring tile; returns the length of one
+    auto legendre = [&](uint32_t orders, std::vector<double> &leg,
+                        std::vector<double> &legt, std::vector<uint2> &off) {
+      std::vector<double> one;  // one ring tile
+      const uint32_t base = at(legt);
+      for (uint32_t rt = 0; rt < nrt; ++rt) {
+        one.clear();
+        for (uint32_t m = 0; m < orders; ++m)
+          for (uint32_t par = 0; par < 2; ++par) {
+            const uint32_t l0 = m + ((m ^ par) & 1u);
+            const uint32_t n = l0 < G.N ? (G.N - l0 + 1) / 2 : 0u;
+            if (rt == 0) off.push_back(make_uint2(at(one), at(legt) - base));
+            for (uint32_t k = 0; k < n; k += 4)
+              for (uint32_t a = 0; a < 64; ++a)
+                one.push_back(P(16 * rt + a % 16, m, l0 + 2 * (k + a / 16)));
+            if (rt == 0)
+              for (uint32_t i0 = 0; i0 < n; i0 += 16)
+                for (uint32_t ks = 0; ks < G.legt_k; ++ks)
+                  for (uint32_t a = 0; a < 64; ++a)
+                    legt.push_back(
+                        P(4 * ks + a / 16, m, l0 + 2 * (i0 + a % 16)));
+          }
+        leg.insert(leg.end(), one.begin(), one.end());
+      }
+      return at(one);
+    };
+    G.leg_n = legendre(G.N, T.leg, T.legt, T.mup);
+    if (single) {
+      G.mup64 = static_cast<uint32_t>(T.mup64.size());
+      G.leg64 = at(T.leg64);
+      G.legt64 = at(T.legt64);
+      G.leg64_n = legendre(dev::kHarmExactMu, T.leg64, T.legt64, T.mup64);
     }
     std::vector<double> ct(2 * G.h), sn(2 * G.h);
     for (uint32_t k = 0; k < 2 * G.h; ++k) {
@@ -391,10 +415,9 @@ inline HarmTables plan_harmonic(const NodeTable &nodes, double h,
                       : dev::harm_lds_lr<double>(T.rad[i].N, hmax, G.nring));
   }
   // the kernels load whole groups of steps
-  T.leg.resize(T.leg.size() + 8 * 64, 0.0);
-  T.legt.resize(T.legt.size() + 8 * 64, 0.0);
-  T.gam.resize(T.gam.size() + 8 * 64, 0.0);
-  T.gamt.resize(T.gamt.size() + 8 * 64, 0.0);
+  for (auto *t : {&T.leg, &T.legt, &T.gam, &T.gamt, &T.leg64, &T.legt64,
+                  &T.gam64, &T.gamt64})
+    t->resize(t->size() + 8 * 64, 0.0);
   T.ok = true;
   return T;
 }
@@ -501,6 +524,13 @@ class HarmDevice {
     const size_t trig = real(t.trig), trigt = real(t.trigt);
     const size_t gam = real(t.gam), gamt = real(t.gamt);
     const size_t jac = real(t.jac), rec = real(t.rec);
+    auto fp64 = [&](const std::vector<double> &v) {
+      return raw(v.data(), v.size() * 8);
+    };
+    const size_t leg64 = fp64(t.leg64), legt64 = fp64(t.legt64);
+    const size_t gam64 = fp64(t.gam64), gamt64 = fp64(t.gamt64);
+    const size_t lrow64 = raw(t.lrow64.data(), t.lrow64.size() * sizeof(uint2));
+    const size_t mup64 = raw(t.mup64.data(), t.mup64.size() * sizeof(uint2));
     buf_.resize(host.size());
     GLST_HIP(hipMemcpy(buf_.as<void>(), host.data(), host.size(),
                        hipMemcpyHostToDevice));
@@ -523,6 +553,12 @@ class HarmDevice {
       d.gamt = at(gamt);
       d.jac = at(jac);
       d.rec = at(rec);
+      d.leg64 = reinterpret_cast<const double *>(b + leg64);
+      d.legt64 = reinterpret_cast<const double *>(b + legt64);
+      d.gam64 = reinterpret_cast<const double *>(b + gam64);
+      d.gamt64 = reinterpret_cast<const double *>(b + gamt64);
+      d.lrow64 = reinterpret_cast<const uint2 *>(b + lrow64);
+      d.mup64 = reinterpret_cast<const uint2 *>(b + mup64);
       d.nrad = static_cast<uint32_t>(t.rad.size());
       d.N = t.N;
       d.stride = t.stride;
