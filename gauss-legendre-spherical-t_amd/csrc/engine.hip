@@ -200,10 +200,12 @@ struct glst_engine {
       ev_rmt.push_back(nullptr);
       GLST_HIP(hipEventCreateWithFlags(&ev_rmt.back(), hipEventDisableTiming));
     }
-    plan_far_field();
+    const NodeLayout layout =
+        Kp > 0 ? layout_nodes(nodes, K, Kp) : NodeLayout{};
+    plan_far_field(layout);
     try {
       allocate();
-      upload_nodes();
+      upload_nodes(layout);
     } catch (const AllocError &) {
       // no room for the expansion's work fields: the direct sums need less
       if (!harm.ok()) throw;
@@ -212,7 +214,7 @@ struct glst_engine {
            {&harm_coef, &harm_mom, &harm_out, &S, &R, &rmt_work})
         b->release();
       allocate();
-      upload_nodes();
+      upload_nodes(layout);
     }
     dev::fill_f64(fx.as<double>(), 0.0, natom, stream);
     dev::fill_f64(fy.as<double>(), 0.0, natom, stream);
@@ -227,7 +229,7 @@ struct glst_engine {
   // and the nodes and the device can hold it.
   size_t harm_coef_len = 0, harm_mom_len = 0;
   std::vector<uint32_t> harm_row_of;  // row of the fields of a node
-  void plan_far_field() {
+  void plan_far_field(const NodeLayout &layout) {
     if (!has_lr || Kp == 0 ||
         !harm_worth(natom, grid.ncell, K, mixed()) ||
         !harm_shell_sums(mixed(), rmt_shape, grid, lds_limit))
@@ -237,7 +239,7 @@ struct glst_engine {
     harm_plan = harm_fit(t, mixed(), lds_limit, natom, grid.ncell);
     if (harm_plan.nrad == 0) return;
     try {
-      harm.upload(t, mixed(), layout_nodes(nodes, K, Kp).k64);
+      harm.upload(t, mixed(), layout.k64);
     } catch (const AllocError &) {
       harm.release();
       return;
@@ -321,10 +323,9 @@ struct glst_engine {
     return sf_cheb && mixed() && cheb.bytes() ? cheb.as<float>() : nullptr;
   }
 
-  void upload_nodes() {
+  void upload_nodes(const NodeLayout &L) {
     if (Kp == 0) return;
-    NodeLayout L = layout_nodes(nodes, K, Kp);
-    dev_of_ref = std::move(L.dev_of_ref);
+    dev_of_ref = L.dev_of_ref;
     ntask = static_cast<uint32_t>(L.node0.size());
     if (split_host.empty()) set_splits(1);
     const std::vector<uint32_t> &split = split_host;

@@ -10,6 +10,7 @@
 #include <cmath>
 #include <cstdint>
 #include <cstring>
+#include <memory>
 #include <type_traits>
 #include <vector>
 
@@ -496,17 +497,25 @@ class HarmDevice {
   void upload(const HarmTables &t, bool single,
               const std::vector<double4> &nodes) {
     // one buffer, every table on a 256-byte boundary
-    std::vector<char> host;
+    const size_t room = t.bytes(single ? 4 : 8) + nodes.size() * sizeof(double4);
+    const std::unique_ptr<char[]> host(new char[room]);  // (not cleared)
+    size_t size = 0;
+    auto place = [&](size_t bytes) {
+      const size_t at = (size + 255) / 256 * 256;
+      size = at + bytes;
+      return at;
+    };
     auto raw = [&](const void *p, size_t bytes) {
-      const size_t at = (host.size() + 255) / 256 * 256;
-      host.resize(at + bytes);
-      if (bytes) std::memcpy(host.data() + at, p, bytes);
+      const size_t at = place(bytes);
+      if (bytes) std::memcpy(host.get() + at, p, bytes);
       return at;
     };
     auto real = [&](const std::vector<double> &v) {
       if (!single) return raw(v.data(), v.size() * 8);
-      std::vector<float> f(v.begin(), v.end());
-      return raw(f.data(), f.size() * 4);
+      const size_t at = place(v.size() * 4);
+      float *f = reinterpret_cast<float *>(host.get() + at);
+      for (size_t i = 0; i < v.size(); ++i) f[i] = static_cast<float>(v[i]);
+      return at;
     };
     const size_t rad = raw(t.rad.data(), t.rad.size() * sizeof(t.rad[0]));
     const size_t grp = raw(t.grp.data(), t.grp.size() * sizeof(t.grp[0]));
@@ -515,10 +524,10 @@ class HarmDevice {
     const size_t pair = raw(t.pair.data(), t.pair.size() * sizeof(uint2));
     const size_t crow = raw(t.crow.data(), t.crow.size() * 4);
     const size_t urow = raw(t.urow.data(), t.urow.size() * 4);
-    std::vector<double4> k(nodes);
-    for (size_t r = 0; r < t.node_of_row.size(); ++r)
-      k[r] = nodes[t.node_of_row[r]];
-    const size_t kat = raw(k.data(), k.size() * sizeof(double4));
+    const size_t kat = place(nodes.size() * sizeof(double4));
+    double4 *k = reinterpret_cast<double4 *>(host.get() + kat);
+    for (size_t r = 0; r < nodes.size(); ++r)
+      k[r] = nodes[r < t.node_of_row.size() ? t.node_of_row[r] : r];
     const size_t units = raw(t.unit.data(), t.unit.size() * sizeof(uint2));
     const size_t leg = real(t.leg), legt = real(t.legt);
     const size_t trig = real(t.trig), trigt = real(t.trigt);
@@ -531,8 +540,8 @@ class HarmDevice {
     const size_t gam64 = fp64(t.gam64), gamt64 = fp64(t.gamt64);
     const size_t lrow64 = raw(t.lrow64.data(), t.lrow64.size() * sizeof(uint2));
     const size_t mup64 = raw(t.mup64.data(), t.mup64.size() * sizeof(uint2));
-    buf_.resize(host.size());
-    GLST_HIP(hipMemcpy(buf_.as<void>(), host.data(), host.size(),
+    buf_.resize(size);
+    GLST_HIP(hipMemcpy(buf_.as<void>(), host.get(), size,
                        hipMemcpyHostToDevice));
     auto fill = [&](auto &d) {
       using T = std::remove_const_t<std::remove_reference_t<decltype(*d.leg)>>;
