@@ -997,7 +997,11 @@ double glst_batch::autotune(const double *rx, const double *ry,
     }
     overlap_near = pick_overlap;
     drop_graph();
-    if (B.partial > 0) {
+    // (the splits have no effect on the expanded systems)
+    const size_t nlr = std::count_if(
+        B.sys.begin(), B.sys.end(),
+        [](const dev::SysDev &d) { return d.Kp > 0; });
+    if (fused != 0 ? nlr > 0 : nlr > B.harm.size()) {
       const uint32_t keep = lr_blocks;
       uint32_t pick = keep;
       for (uint32_t v : {1024u, 2048u, 4096u, 8192u, 16384u, 32768u, 65536u}) {

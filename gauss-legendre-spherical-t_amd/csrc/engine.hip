@@ -832,12 +832,13 @@ struct glst_engine {
          },
          {0, 1, 2});
     if (has_lr && Kp > 0) {
-      knob([&] { return static_cast<int64_t>(lr_blocks); },
-           [&](int64_t v) {
-             lr_blocks = static_cast<uint32_t>(v);
-             apply_lr_blocks();
-           },
-           {1024, 2048, 4096, 8192, 16384, 32768, 65536});
+      if (!harmonic())  // (no effect on the expansion)
+        knob([&] { return static_cast<int64_t>(lr_blocks); },
+             [&](int64_t v) {
+               lr_blocks = static_cast<uint32_t>(v);
+               apply_lr_blocks();
+             },
+             {1024, 2048, 4096, 8192, 16384, 32768, 65536});
       if (!rmt_global_path(harmonic()))
         knob([&] { return static_cast<int64_t>(rmt_shape); },
              [&](int64_t v) {

@@ -5,6 +5,8 @@
 //            the direct sums, up to the bytes those need
 //   batch    the same for a batch
 //   slots    a batch of expanded systems needs no more than they do alone
+//   tune     tuning an expanded handle or batch tries no splits of the direct
+//            sums' back-projection, which would allocate their rows again
 //   layout   a batch clears S where a step's layout of it differs from the last
 // Prints "ok" and returns 0, or one line per failure.
 #include "fake_hip.hpp"
@@ -169,6 +171,34 @@ void slots() {
   }
 }
 
+void tune() {
+  const double box[] = {135, 135, 135}, rcut = 9;
+  for (uint32_t n : {100000u, 20000u}) {  // expanded, and dilute
+    glst_handle_t h = nullptr;
+    CHECK(glst_create(GLST_CT_DOUBLE, n, 1e-4, 135, 135, 135, 9, nullptr, &h) ==
+              GLST_OK, "%s", glst_global_last_error());
+    long before = st.allocations;
+    double ms = 0.0;
+    st.reset();
+    CHECK(glst_autotune(h, arr(0), arr(1), arr(2), arr(3), 2, &ms) == GLST_OK,
+          "%s", glst_last_error(h));
+    CHECK((st.harm > 0) == (n == 100000), "%u charges", n);
+    CHECK((st.allocations == before) == (st.harm > 0), "%ld allocations",
+          st.allocations - before);
+    glst_destroy(h);
+    glst_batch_t b = nullptr;
+    CHECK(glst_batch_create(GLST_CT_DOUBLE, 1, &n, box, &rcut, 1e-4, nullptr,
+                            &b) == GLST_OK, "%s", glst_global_last_error());
+    before = st.allocations;
+    st.reset();
+    CHECK(glst_batch_autotune(b, arr(0), arr(1), arr(2), arr(3), 2, &ms) ==
+              GLST_OK, "%s", glst_batch_last_error(b));
+    CHECK((st.allocations == before) == (st.harm > 0), "batch: %ld allocations",
+          st.allocations - before);
+    glst_batch_destroy(b);
+  }
+}
+
 // fused 0 expands, the other launch modes do not
 void layout() {
   const uint32_t n = 100000;
@@ -203,6 +233,7 @@ int main(int argc, char **argv) {
   else if (what == "handle") handle();
   else if (what == "batch") batch();
   else if (what == "slots") slots();
+  else if (what == "tune") tune();
   else if (what == "layout") layout();
   else return 2;
   if (failures || st.failures) return 1;

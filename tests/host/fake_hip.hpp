@@ -21,7 +21,7 @@ struct State {
   std::map<const char *, size_t> mem;  // allocations
   size_t used = 0, peak = 0, limit = SIZE_MAX;
   int capturing = 0;
-  long refused_in_capture = 0, failures = 0;
+  long refused_in_capture = 0, failures = 0, allocations = 0;
   // launches since reset(): expanded and direct far fields, shell sums by path
   long harm = 0, direct = 0, global = 0, steps = 0;
   size_t filled = 0;  // doubles of the largest fill
@@ -56,6 +56,7 @@ hipError_t hipMalloc(void **p, size_t n) {
   if (a == MAP_FAILED) return hipErrorOutOfMemory;
   st.mem[static_cast<const char *>(a)] = n;
   st.used += n;
+  ++st.allocations;
   st.peak = st.used > st.peak ? st.used : st.peak;
   *p = a;
   return hipSuccess;

@@ -29,7 +29,8 @@ def alloc_check(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("what", ["handle", "capture", "batch", "slots", "layout"])
+@pytest.mark.parametrize("what", ["handle", "capture", "batch", "slots", "layout",
+                                  "tune"])
 def test_allocations(alloc_check, what):
     r = subprocess.run([alloc_check, what], capture_output=True, text=True,
                        timeout=300)
