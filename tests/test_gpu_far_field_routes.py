@@ -1,5 +1,6 @@
 """Which far field a handle takes, and that every route gives the same fields:
-grids with one long edge, captured and eager; dilute systems.
+grids with one long edge, captured and eager; dilute systems; global tables;
+the matrix-core shell sums of expanded grids with unequal edges; most azimuths.
 
 lr_blocks cuts the direct sums' back-projection into other partial sums and
 has no effect on the expansion, so "the same bits under another lr_blocks"
@@ -124,3 +125,58 @@ def test_global_tables_on_node_major_fields(cuda, ct, bar):
         (1e-11 if ct == "double" else 1e-5) * scale
     assert rel_err(ef[:3], ef0[:3]) < bar
     assert rel_err(ef[3:], ef0[3:]) < bar
+
+
+def fields(f, d):
+    f.assign_atoms(*d)
+    f.calc_sf()
+    s = f.sf()
+    f.sum_rmt_sf()
+    r = f.rmt()
+    return s, r, step(f, d)
+
+
+def off(a, b):
+    return max(np.abs(x - y).max() for x, y in zip(a, b)) / \
+        max(np.abs(y).max() for y in b)
+
+
+# 12 x 13 x 15 cells: matrix-core shell sums whose x and z axes differ, and
+# 2,340 workgroups of the evaluation, which takes four waves from 2,048 on.
+# 6^3 cells at tol 3e-7: the most azimuths (59 half azimuths) and, mixed, the
+# most degrees (40) the kernels take.
+# FP64 terms left out stay under 1e-15 of a wave and sums of up to 56 terms of
+# a recurrence round under 1e-13; 1e-12 leaves room for the cancellation of a
+# neutral system.  Mixed: the bars of the path.
+@pytest.mark.parametrize("box,spacing,tol,ncell", [
+    ((107.5, 116.5, 134.5), 3.0, 1e-4, (12, 13, 15)),
+    ((46.2, 46.2, 46.2), 2.3, 3e-7, (6, 6, 6))])
+def test_expansion_matches_direct_sums(cuda, box, spacing, tol, ncell):
+    import torch
+    import glst_amd as g
+    h = lattice(box, spacing, 17)
+    f, d = handle(g, torch, h, box, tol, ct="double", lr_atom_groups=0)
+    s0, r0, ef0 = fields(f, d)
+    f.close()
+    for ct, sbar, bar in (("double", 1e-12, 1e-12), ("float", 1e-5, 2e-6)):
+        f, d = handle(g, torch, h, box, tol, ct=ct)
+        assert tuple(f.info().ncell) == ncell
+        assert expands(f, d)
+        s, r, ef = fields(f, d)
+        f.close()
+        assert off(s, s0) < sbar, ct
+        assert off(r, r0) < sbar, ct
+        assert rel_err(ef[:3], ef0[:3]) < bar, ct
+        assert rel_err(ef[3:], ef0[3:]) < bar, ct
+        # the same system in a batch beside a small one
+        small = lattice((31.0, 40.0, 36.0), 2.6, 3)
+        n = [h[0].size, small[0].size]
+        b = g.GLSTBatch(n, [box, (31.0, 40.0, 36.0)], 9.0, tol, ct=ct)
+        packed = [torch.as_tensor(np.concatenate([x, y]), dtype=torch.float64,
+                                  device="cuda") for x, y in zip(h, small)]
+        b.zero_ef()
+        b.calc_ener_force(*packed)
+        got = [t.cpu().numpy()[:n[0]] for t in b.get_ef()]
+        b.close()
+        assert rel_err(got[:3], ef0[:3]) < bar, ct
+        assert rel_err(got[3:], ef0[3:]) < bar, ct
