@@ -1277,7 +1277,7 @@ template <typename T>
 constexpr int harm_lr_rows(int c) {
   return sizeof(T) == 4 ? c + 1 : c == 1 ? 1 : 2;
 }
-constexpr int harm_lr_steps(int c) { return c == 1 ? 4 : c == 2 ? 6 : 9; }
+constexpr int harm_lr_steps(int c) { return c == 1 ? 4 : c == 2 ? 6 : 8; }
 __host__ __device__ constexpr int harm_lr_class(uint32_t hk) {
   return hk <= 4 ? 1 : hk <= 6 ? 2 : 3;
 }
@@ -1303,8 +1303,7 @@ __global__ __launch_bounds__(kHarmBlock, harm_lr_waves<T>(C)) void harm_lr_kerne
   const HarmGroup gr = H.grp[rad.group];
   harm_switch<C>(harm_lr_class(gr.trigt_k), [&](auto cls) {
     constexpr int c = decltype(cls)::value;
-    constexpr int RW = harm_lr_rows<T>(c), HK = harm_lr_steps(c);
-    constexpr int LK = HK - (HK > 8 ? 2 : 1);
+    constexpr int RW = harm_lr_rows<T>(c), HK = harm_lr_steps(c), LK = HK - 1;
     // tiles of 16 orders of a set
     harm_switch<2>((harm_order_steps(rad.N) + 3) / 4, [&](auto mt) {
       constexpr int MT = decltype(mt)::value;
@@ -1583,10 +1582,8 @@ void prepare_harmonic(size_t lds_limit) {
   allow(harm_moments_kernel<double, 32>);
   allow(harm_sf_kernel<float, 1>);
   allow(harm_sf_kernel<float, 2>);
-  allow(harm_sf_kernel<float, 3>);
   allow(harm_sf_kernel<double, 1>);
   allow(harm_sf_kernel<double, 2>);
-  allow(harm_sf_kernel<double, 3>);
   allow(harm_lr_kernel<float, 1>);
   allow(harm_lr_kernel<float, 2>);
   allow(harm_lr_kernel<float, 3>);
@@ -1665,10 +1662,8 @@ void harm_sf(const HarmPlanDev &P, const HarmDev<T> &H, const void *atoms,
   };
   if (P.hsteps <= 4)
     go(harm_sf_kernel<T, 1>);
-  else if (P.hsteps <= 8)
-    go(harm_sf_kernel<T, 2>);
   else
-    go(harm_sf_kernel<T, 3>);
+    go(harm_sf_kernel<T, 2>);
 }
 
 template <typename T>

@@ -39,7 +39,8 @@ namespace dev {
 
 constexpr uint32_t kHarmMaxN = 56;   // expansion degrees 0 .. N - 1
 constexpr uint32_t kHarmMaxN32 = 40; // in FP32 (reached at phases of 20 radians)
-constexpr uint32_t kHarmMaxH = 64;   // half azimuths of a ring
+constexpr uint32_t kHarmMaxH = 63;   // half azimuths of a ring (reached with
+                                     // 56 degrees; more need more)
 constexpr uint32_t kHarmCells = 8;   // cells per tile of the transforms
 constexpr uint32_t kHarmMu = 8;      // azimuthal orders per tile of 16 columns
 
