@@ -787,7 +787,7 @@ void glst_batch::harm_step(const HarmSystem &h) {
   dev::harm_lr<T>(h.plan, H, g, Rs, coef, mom, s);
   // the atoms' indices count from the batch's first atom
   dev::harm_eval<T>(
-      h.plan, H, atoms, start, k64, B.cs[h.sys]->su().K, g, mom, Rs, out,
+      h.plan, H, atoms, start, k64, B.cs[h.sys]->su().K, g, mom, Rs, out, coef,
       reinterpret_cast<double4 *>(
           reinterpret_cast<uintptr_t>(partial.as<double4>()) +
           (d.partial0 - d.atom0) * sizeof(double4)),

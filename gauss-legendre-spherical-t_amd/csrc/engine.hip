@@ -523,8 +523,8 @@ struct glst_engine {
         dev::harm_eval<T>(harm_plan, harm.dev<T>(), lr_atoms(),
                           cell_start.as<uint32_t>(), harm.k64, K,
                           grid, harm_mom.as<T>(), R.as<T>(),
-                          harm_out.as<uint32_t>(), partial.as<double4>(),
-                          stream);
+                          harm_out.as<uint32_t>(), harm_coef.as<T>(),
+                          partial.as<double4>(), stream);
       };
       if (mixed())
         run(0.0f);

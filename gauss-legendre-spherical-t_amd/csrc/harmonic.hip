@@ -214,7 +214,7 @@ template <typename T>
 constexpr uint32_t harm_lb() {
   return sizeof(T) == 4 ? 4 : 2;
 }
-constexpr int kHarmBlock = 512;  // threads of the transform kernels
+constexpr uint32_t kHarmBlock = 512;  // threads of the transform kernels
 
 template <int V>
 struct HarmInt {
@@ -1320,85 +1320,119 @@ __global__ __launch_bounds__(kHarmBlock, harm_lr_waves<T>(C)) void harm_lr_kerne
 // ---------------------------------------------------------------------------
 // coefficients -> energies and forces
 
-// Fields of the atoms outside their cell's ball (cells without any return at
-// once): the direct sums over the nodes, four atoms and four nodes at a time
-// (the nodes' remote sums lie rows apart; with one of each at a time, inside the
-// evaluation, an FP64 step of 2,000 waters at rcut 8, tol 1e-6, with a molecule
-// across the box's corner took 4.60 ms instead of 2.82).
-constexpr uint32_t kHarmOutBlock = 512;
+// Fields of the atoms outside their cell's ball: the direct sums over the nodes,
+// four atoms and four nodes at a time (the nodes' remote sums lie rows apart),
+// before the evaluation.  The nodes of a cell are shared out to kHarmSlices
+// workgroups: workgroup b takes slice j of cell b - j, so that the grid stays
+// one workgroup per cell and most find nothing to do.  The slices' sums go to
+// the cell's coefficients, which are free by then, and the evaluation adds them
+// up; a cell of more atoms than fit there is left to one workgroup, which
+// stores the fields itself.  With an atom beyond the box's corner, an FP64 step
+// of 2,000 waters at rcut 8, tol 1e-6 takes 2.38 ms, 2.94 with one workgroup for
+// all nodes of a cell, 2.73 with direct sums for all (1.83 without that atom).
+constexpr uint32_t kHarmSlices = 16;
 template <typename T>
-__global__ __launch_bounds__(kHarmOutBlock) void harm_outside_kernel(
+__device__ __forceinline__ bool harm_sliced(const HarmDev<T> &H, uint32_t na) {
+  return na * kHarmSlices * sizeof(double4) <= H.stride * sizeof(T);
+}
+// [atom of the cell][slice]
+template <typename T>
+__device__ __forceinline__ double4 *harm_slices(const HarmDev<T> &H, T *coef,
+                                                uint32_t cell) {
+  return reinterpret_cast<double4 *>(coef + static_cast<size_t>(cell) * H.stride);
+}
+template <typename T>
+__global__ __launch_bounds__(kHarmBlock) void harm_outside_kernel(
     HarmDev<T> H, const typename HarmRecord<T>::type *__restrict__ atoms,
     const uint32_t *__restrict__ start, const double4 *__restrict__ k64,
     uint32_t K, uint32_t ny, uint32_t nz, double h, uint32_t ncell,
     const T *__restrict__ R, const uint32_t *__restrict__ outside,
-    double4 *__restrict__ out) {
-  const uint32_t cell = blockIdx.x;
-  if (!outside[cell]) return;
-  __shared__ uint32_t list[65];
-  __shared__ double red[kHarmOutBlock / 64][16];
+    T *__restrict__ coef, double4 *__restrict__ out) {
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+  // (a far field has at least 27 cells, more than the slices)
+  auto cell_of = [&](uint32_t j) {
+    return blockIdx.x < j ? blockIdx.x + ncell - j : blockIdx.x - j;
+  };
+  unsigned long long todo =
+      __ballot(lane < kHarmSlices && outside[cell_of(lane % kHarmSlices)]);
+  if (!todo) return;
+  __shared__ uint32_t list[65];
+  __shared__ double red[kHarmBlock / 64][16];
   const uint32_t ncp = harm_row(ncell);
-  const uint32_t a0 = start[cell], na = start[cell + 1] - a0;
-  const HarmCentre cc = harm_centre(cell, ny, nz, h);
-  for (uint32_t p0 = 0; p0 < na; p0 += 64) {
-    __syncthreads();
-    if (wave == 0)
-      harm_list_outside(H, atoms, a0 + p0, na - p0 < 64 ? na - p0 : 64u, cc,
-                        list);
-    __syncthreads();
-    const uint32_t cnt = list[0];
-    for (uint32_t q0 = 0; q0 < cnt; q0 += 4) {
-      HarmOffset a[4];
-      double v[16];
+  for (; todo; todo &= todo - 1) {
+    const uint32_t slice = static_cast<uint32_t>(__ffsll(todo)) - 1;
+    const uint32_t cell = cell_of(slice);
+    const uint32_t a0 = start[cell], na = start[cell + 1] - a0;
+    const bool sliced = harm_sliced(H, na);
+    if (!sliced && slice > 0) continue;
+    const uint32_t per = sliced ? (K + kHarmSlices - 1) / kHarmSlices : K;
+    const uint32_t k0 = slice * per < K ? slice * per : K;
+    const uint32_t k1 = k0 + per < K ? k0 + per : K;
+    const HarmCentre cc = harm_centre(cell, ny, nz, h);
+    for (uint32_t p0 = 0; p0 < na; p0 += 64) {
+      __syncthreads();
+      if (wave == 0)
+        harm_list_outside(H, atoms, a0 + p0, na - p0 < 64 ? na - p0 : 64u, cc,
+                          list);
+      __syncthreads();
+      const uint32_t cnt = list[0];
+      for (uint32_t q0 = 0; q0 < cnt; q0 += 4) {
+        HarmOffset a[4];
+        double v[16];
 #pragma unroll
-      for (uint32_t q = 0; q < 4; ++q)
-        a[q] = harm_offset(atoms, list[1 + (q0 + q < cnt ? q0 + q : q0)], cc);
+        for (uint32_t q = 0; q < 4; ++q)
+          a[q] = harm_offset(atoms, list[1 + (q0 + q < cnt ? q0 + q : q0)], cc);
 #pragma unroll
-      for (int i = 0; i < 16; ++i) v[i] = 0.0;
-      for (uint32_t n0 = tid; n0 < K; n0 += 4 * kHarmOutBlock) {
-        double4 k[4];
-        double vr[4], vi[4];
-#pragma unroll
-        for (uint32_t u = 0; u < 4; ++u) {
-          const uint32_t n = n0 + u * kHarmOutBlock;
-          const uint32_t m = n < K ? n : n0;
-          k[u] = k64[m];
-          vr[u] = R[harm_slot<T>(m, cell, 0, ncp)];
-          vi[u] = R[harm_slot<T>(m, cell, 1, ncp)];
-          if (n >= K) vr[u] = vi[u] = 0.0;
-        }
-#pragma unroll
-        for (uint32_t q = 0; q < 4; ++q) {
-          if (q0 + q >= cnt) break;  // uniform
+        for (int i = 0; i < 16; ++i) v[i] = 0.0;
+        for (uint32_t n0 = k0 + tid; n0 < k1; n0 += 4 * kHarmBlock) {
+          double4 k[4];
+          double vr[4], vi[4];
 #pragma unroll
           for (uint32_t u = 0; u < 4; ++u) {
-            const double ph =
-                k[u].x * a[q].x + k[u].y * a[q].y + k[u].z * a[q].z;
-            const double c = cos(ph), s = sin(ph);
-            const double b = c * vi[u] + s * vr[u];
-            v[4 * q] += k[u].x * b;
-            v[4 * q + 1] += k[u].y * b;
-            v[4 * q + 2] += k[u].z * b;
-            v[4 * q + 3] += c * vr[u] - s * vi[u];
+            const uint32_t n = n0 + u * kHarmBlock;
+            const uint32_t m = n < k1 ? n : n0;
+            k[u] = k64[m];
+            vr[u] = R[harm_slot<T>(m, cell, 0, ncp)];
+            vi[u] = R[harm_slot<T>(m, cell, 1, ncp)];
+            if (n >= k1) vr[u] = vi[u] = 0.0;
+          }
+#pragma unroll
+          for (uint32_t q = 0; q < 4; ++q) {
+            if (q0 + q >= cnt) break;  // uniform
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) {
+              const double ph =
+                  k[u].x * a[q].x + k[u].y * a[q].y + k[u].z * a[q].z;
+              const double c = cos(ph), s = sin(ph);
+              const double b = c * vi[u] + s * vr[u];
+              v[4 * q] += k[u].x * b;
+              v[4 * q + 1] += k[u].y * b;
+              v[4 * q + 2] += k[u].z * b;
+              v[4 * q + 3] += c * vr[u] - s * vi[u];
+            }
           }
         }
-      }
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        for (int o = 32; o > 0; o >>= 1) v[i] += __shfl_xor(v[i], o, 64);
-        if (lane == 0) red[wave][i] = v[i];
+        for (int i = 0; i < 16; ++i) {
+          for (int o = 32; o > 0; o >>= 1) v[i] += __shfl_xor(v[i], o, 64);
+          if (lane == 0) red[wave][i] = v[i];
+        }
+        __syncthreads();
+        if (tid < 4 && q0 + tid < cnt) {
+          double t[4] = {0.0, 0.0, 0.0, 0.0};
+          for (uint32_t w = 0; w < kHarmBlock / 64; ++w)
+            for (uint32_t d = 0; d < 4; ++d) t[d] += red[w][4 * tid + d];
+          const uint32_t i = list[1 + q0 + tid];
+          if (sliced) {
+            harm_slices(H, coef, cell)[(i - a0) * kHarmSlices + slice] =
+                make_double4(t[0], t[1], t[2], t[3]);
+          } else {
+            const double q = harm_offset(atoms, i, cc).q;
+            out[i] = make_double4(q * t[0], q * t[1], q * t[2], q * t[3]);
+          }
+        }
+        __syncthreads();
       }
-      __syncthreads();
-      if (tid < 4 && q0 + tid < cnt) {
-        double t[4] = {0.0, 0.0, 0.0, 0.0};
-        for (uint32_t w = 0; w < kHarmOutBlock / 64; ++w)
-          for (uint32_t d = 0; d < 4; ++d) t[d] += red[w][4 * tid + d];
-        const uint32_t i = list[1 + q0 + tid];
-        const double q = harm_offset(atoms, i, cc).q;
-        out[i] = make_double4(q * t[0], q * t[1], q * t[2], q * t[3]);
-      }
-      __syncthreads();
     }
   }
 }
@@ -1424,7 +1458,8 @@ __device__ __forceinline__ HarmConst<T> *harm_const(const T *p) {
 template <typename T, int W, int MO, int PM>
 __device__ __forceinline__ void harm_eval_body(
     const HarmDev<T> &H, const typename HarmRecord<T>::type *atoms, uint32_t a0,
-    uint32_t na, const HarmCentre &cc, const T *U, double4 *out, double *red) {
+    uint32_t na, const HarmCentre &cc, const T *U, const double4 *slices,
+    double4 *out, double *red) {
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t N = H.N;
@@ -1527,8 +1562,23 @@ __device__ __forceinline__ void harm_eval_body(
     for (int w = 1; w < W; ++w)
 #pragma unroll
       for (int d = 0; d < 4; ++d) v[d] += red[(4 * w + d) * 64 + lane];
-    const double q = a.q, f = -q * H.scale;
-    out[a0 + lane] = make_double4(f * v[0], f * v[1], f * v[2], q * v[3]);
+    const double q = a.q;
+    double f = -q * H.scale;
+    if (a.out && slices) {  // (the sums over the nodes)
+      f = q;
+#pragma unroll
+      for (int d = 0; d < 4; ++d) v[d] = 0.0;
+#pragma unroll 1
+      for (uint32_t j = 0; j < kHarmSlices; ++j) {
+        const double4 t = slices[lane * kHarmSlices + j];
+        v[0] += t.x;
+        v[1] += t.y;
+        v[2] += t.z;
+        v[3] += t.w;
+      }
+    }
+    if (!a.out || slices)
+      out[a0 + lane] = make_double4(f * v[0], f * v[1], f * v[2], q * v[3]);
   }
   harm_barrier();
 }
@@ -1542,7 +1592,8 @@ template <typename T, int W, int MO, int PM>
 __global__ __launch_bounds__(64 * W) void harm_eval_kernel(
     HarmDev<T> H, const typename HarmRecord<T>::type *__restrict__ atoms,
     const uint32_t *__restrict__ start, uint32_t ny, uint32_t nz, double h,
-    uint32_t nset, const T *__restrict__ mom, double4 *__restrict__ out) {
+    uint32_t nset, const T *__restrict__ mom, T *__restrict__ coef,
+    double4 *__restrict__ out) {
   __shared__ double red[W * 256];
   const uint32_t nb = gridDim.x, b = blockIdx.x;
   const uint32_t q = nb >> 3, r = nb & 7u, x = b & 7u;
@@ -1560,7 +1611,11 @@ __global__ __launch_bounds__(64 * W) void harm_eval_kernel(
   }
   for (uint32_t p0 = 64 * set; p0 < na; p0 += 64 * nset) {
     const uint32_t cnt = na - p0 < 64 ? na - p0 : 64u;
-    harm_eval_body<T, W, MO, PM>(H, atoms, a0 + p0, cnt, cc, U, out, red);
+    const double4 *slices =
+        harm_sliced(H, na) ? harm_slices(H, coef, cell) + p0 * kHarmSlices
+                           : nullptr;
+    harm_eval_body<T, W, MO, PM>(H, atoms, a0 + p0, cnt, cc, U, slices, out,
+                                 red);
   }
   asm volatile("" ::"v"(touch[0]), "v"(touch[1]));
 }
@@ -1690,33 +1745,35 @@ template <typename T>
 void harm_eval(const HarmPlanDev &P, const HarmDev<T> &H, const void *atoms,
                const uint32_t *start, const double4 *k64, uint32_t K,
                const GridShape &g, const T *mom, const T *R,
-               const uint32_t *outside, double4 *out, hipStream_t s) {
+               const uint32_t *outside, T *coef, double4 *out, hipStream_t s) {
   auto *at = static_cast<const typename HarmRecord<T>::type *>(atoms);
   const uint32_t ps = harm_psteps(0, H.N);
   auto go = [&](auto waves, auto orders, auto steps) {
     constexpr int W = decltype(waves)::value, MO = decltype(orders)::value;
     harm_eval_kernel<T, W, MO, decltype(steps)::value>
         <<<g.ncell * P.nset, 64 * W, 0, s>>>(
-            H, at, start, g.ny, g.nz, g.h, P.nset, mom, out);
+            H, at, start, g.ny, g.nz, g.h, P.nset, mom, coef, out);
   };
+  harm_outside_kernel<T><<<g.ncell, kHarmBlock, 0, s>>>(
+      H, at, start, k64, K, g.ny, g.nz, g.h, g.ncell, R, outside, coef, out);
   // W MO >= N (N <= 8 ps).  FP32: four waves of twice the orders form the
   // radial values half as often (400 against 439 us at 3,375 cells), eight
   // fill the device on smaller grids (69 against 102 us at 64 cells, 87
   // against 106 at 512, two workgroups each)
-  if (sizeof(T) == 4 && g.ncell * P.nset >= 2048) {
-    harm_host_switch<5>(ps, [&](auto k) {
-      constexpr int PM = decltype(k)::value;
-      if (H.N <= 8 * PM - 4)
-        go(HarmInt<4>{}, HarmInt<2 * PM - 1>{}, k);
-      else
-        go(HarmInt<4>{}, HarmInt<2 * PM>{}, k);
-    });
-  } else {
-    harm_host_switch<sizeof(T) == 4 ? 5 : 7>(
-        ps, [&](auto k) { go(HarmInt<8>{}, k, k); });
+  if constexpr (sizeof(T) == 4) {
+    if (g.ncell * P.nset >= 2048) {
+      harm_host_switch<5>(ps, [&](auto k) {
+        constexpr int PM = decltype(k)::value;
+        if (H.N <= 8 * PM - 4)
+          go(HarmInt<4>{}, HarmInt<2 * PM - 1>{}, k);
+        else
+          go(HarmInt<4>{}, HarmInt<2 * PM>{}, k);
+      });
+      return;
+    }
   }
-  harm_outside_kernel<T><<<g.ncell, kHarmOutBlock, 0, s>>>(
-      H, at, start, k64, K, g.ny, g.nz, g.h, g.ncell, R, outside, out);
+  harm_host_switch<sizeof(T) == 4 ? 5 : 7>(
+      ps, [&](auto k) { go(HarmInt<8>{}, k, k); });
 }
 
 #define GLST_HARM(T)                                                          \
@@ -1734,7 +1791,7 @@ void harm_eval(const HarmPlanDev &P, const HarmDev<T> &H, const void *atoms,
   template void harm_eval<T>(const HarmPlanDev &, const HarmDev<T> &,         \
                              const void *, const uint32_t *, const double4 *, \
                              uint32_t, const GridShape &, const T *,          \
-                             const T *, const uint32_t *, double4 *,          \
+                             const T *, const uint32_t *, T *, double4 *,     \
                              hipStream_t);
 GLST_HARM(float)
 GLST_HARM(double)

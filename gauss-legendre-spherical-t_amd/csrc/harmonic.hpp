@@ -168,7 +168,7 @@ template <typename T>
 void harm_eval(const HarmPlanDev &P, const HarmDev<T> &H, const void *atoms,
                const uint32_t *start, const double4 *k64, uint32_t K,
                const GridShape &g, const T *mom, const T *R,
-               const uint32_t *outside, double4 *out, hipStream_t s);
+               const uint32_t *outside, T *coef, double4 *out, hipStream_t s);
 // Once per process and device (see prepare_kernels).
 void prepare_harmonic(size_t lds_limit);
 

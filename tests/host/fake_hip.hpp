@@ -304,7 +304,7 @@ template <typename T>
 void harm_eval(const HarmPlanDev &, const HarmDev<T> &, const void *,
                const uint32_t *, const double4 *k64, uint32_t K,
                const GridShape &g, const T *, const T *R, const uint32_t *,
-               double4 *, hipStream_t) {
+               T *, double4 *, hipStream_t) {
   fake::require(k64, K * sizeof(double4), "k64");
   fake::require(R, static_cast<size_t>(harm_row(g.ncell)) * K * 2 * sizeof(T),
                 "R");
@@ -327,7 +327,7 @@ void harm_eval(const HarmPlanDev &, const HarmDev<T> &, const void *,
   template void harm_eval<T>(const HarmPlanDev &, const HarmDev<T> &,         \
                              const void *, const uint32_t *, const double4 *, \
                              uint32_t, const GridShape &, const T *,          \
-                             const T *, const uint32_t *, double4 *,          \
+                             const T *, const uint32_t *, T *, double4 *,     \
                              hipStream_t);
 FAKE_HARM(float)
 FAKE_HARM(double)

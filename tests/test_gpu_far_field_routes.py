@@ -180,3 +180,45 @@ def test_expansion_matches_direct_sums(cuda, box, spacing, tol, ncell):
         b.close()
         assert rel_err(got[:3], ef0[:3]) < bar, ct
         assert rel_err(got[3:], ef0[3:]) < bar, ct
+
+
+@pytest.mark.parametrize("ct,bar", [("double", 1e-12), ("float", 2e-6)])
+@pytest.mark.parametrize("tol,crowd", [(2e-5, 3), (2e-5, 1000), (1e-5, 70)])
+def test_atoms_outside_their_ball(cuda, ct, bar, tol, crowd):
+    """Atoms beyond a corner of the box, which the binning puts into the corner
+    cell but whose plane waves its expansion does not hold: 3 and 70 of them
+    with the nodes shared out to workgroups (one or two lists of 64), 1,000 in one
+    cell that one workgroup takes; and one across the opposite corner."""
+    import torch
+    import glst_amd as g
+    box = (53.0, 49.0, 62.0)
+    h = lattice(box, 2.6, 21)
+    rng = np.random.default_rng(4)
+    out = rng.uniform(-3.5, -0.5, (crowd, 3))
+    out = np.concatenate([out, [[54.5, 54.5, 63.5]]])
+    q = rng.uniform(-1.0, 1.0, len(out))
+    h = [np.concatenate([a, b]) for a, b in zip(h, [*out.T, q])]
+    f, d = handle(g, torch, h, box, tol, ct="double", lr_atom_groups=0)
+    f.assign_atoms(*d)
+    f.calc_sf()
+    f.sum_rmt_sf()
+    f.zero_ef()
+    f.calc_lr_ef()
+    far0 = [t.cpu().numpy() for t in f.get_ef()]
+    f.close()
+    f, d = handle(g, torch, h, box, tol, ct=ct)
+    assert expands(f, d)
+    for _ in range(2):
+        f.assign_atoms(*d)
+        f.calc_sf()
+        f.sum_rmt_sf()
+        f.zero_ef()
+        f.calc_lr_ef()
+        far = [t.cpu().numpy() for t in f.get_ef()]
+        n = crowd + 1  # these atoms alone, then all
+        assert rel_err([a[-n:] for a in far[:3]],
+                       [a[-n:] for a in far0[:3]]) < bar
+        assert rel_err([far[3][-n:]], [far0[3][-n:]]) < bar
+        assert rel_err(far[:3], far0[:3]) < bar
+        assert rel_err(far[3:], far0[3:]) < bar
+    f.close()
