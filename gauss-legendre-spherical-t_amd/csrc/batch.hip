@@ -774,16 +774,19 @@ void glst_batch::harm_step(const HarmSystem &h) {
   uint32_t *out = harm_out[h.slot].as<uint32_t>();
   dev::harm_moments<T>(h.plan, H, atoms, start, g, mom, coef, out, s);
   dev::harm_sf<T>(h.plan, H, atoms, start, k64, g, coef, out, Ss, s);
-  if (mixed() && rmt_wave && dev::rmt_wave_fits(g))
-    dev::rmt_wave(Ss, k64, group, r_in, r_out, d.Kp, g, Rs, s, 0, 0xffffffffu,
-                  true);
-  else if (!(mixed() && dev::rmt_mfma_nodes(g, lds_limit, true) > 0 &&
-             dev::rmt_mfma(Ss, k64, group, r_in, r_out, d.Kp, g, lds_limit, Rs,
-                           s, 0, 0xffffffffu, true)) &&
-           !dev::rmt_lds(mixed(), dev::kRmtMaxNodes, Ss, k64, group, r_in,
+  dev::RmtPath path = dev::rmt_path(mixed(), 4, g, lds_limit, true);
+  if (path == dev::RmtPath::kWave && !rmt_wave) path = dev::RmtPath::kLds;
+  const bool done =
+      path == dev::RmtPath::kWave
+          ? dev::rmt_wave(Ss, k64, group, r_in, r_out, d.Kp, g, Rs, s, 0,
+                          0xffffffffu, true)
+      : path == dev::RmtPath::kMfma
+          ? dev::rmt_mfma(Ss, k64, group, r_in, r_out, d.Kp, g, lds_limit, Rs,
+                          s, 0, 0xffffffffu, true)
+          : dev::rmt_lds(mixed(), dev::kRmtMaxNodes, Ss, k64, group, r_in,
                          r_out, d.Kp, g, lds_limit, Rs, s, 0, 0xffffffffu,
-                         true))
-    throw StateError("shell sums: the cell table does not fit");
+                         true);
+  if (!done) throw StateError("shell sums: the cell table does not fit");
   dev::harm_lr<T>(h.plan, H, g, Rs, coef, mom, s);
   // the atoms' indices count from the batch's first atom
   dev::harm_eval<T>(

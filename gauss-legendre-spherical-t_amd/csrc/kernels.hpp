@@ -263,10 +263,17 @@ inline bool rmt_wave_fits(const GridShape &g) {
 // glst_hip.h) and the layout of its fields: the one place that decides, for
 // the launches, the work field that the global tables need (which a captured
 // step cannot allocate) and the choice of the far field (harmonic_plan.hpp).
+// The default shape (4) takes the matrix cores where the slices of the kernel
+// fill half of their 16 x 16 tile or more; on node-major fields both planes
+// have to, as the z slices' walk is what a thin grid loses (expanded mixed
+// handles at tol 1e-5, LDS tables against matrix cores: 12 x 12 x 3 cells 834
+// and 1,095 us, 12 x 12 x 6 1,061 and 1,134, 9^3 805 and 991, 11^3 1,386 and
+// 1,084; at 1e-4 16 x 16 x 8 338 and 312, 12^3 365 and 261).
 enum class RmtPath { kMfma, kWave, kLds, kGlobal };
 inline RmtPath rmt_path(bool mixed, int shape, const GridShape &g,
                         size_t lds_limit, bool nm) {
-  const bool wide = g.nx * g.ny * 2 >= kRmtMfmaMaxXY * kRmtMfmaMaxXY;
+  const uint32_t plane = g.ny * (nm && g.nz < g.nx ? g.nz : g.nx);
+  const bool wide = plane * 2 >= kRmtMfmaMaxXY * kRmtMfmaMaxXY;
   if (mixed && (shape == 3 || (shape == 4 && wide)) &&
       rmt_mfma_nodes(g, lds_limit, nm) > 0)
     return RmtPath::kMfma;

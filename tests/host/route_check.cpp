@@ -70,6 +70,24 @@ int main() {
   refuses(16, 16, 24, false);
   refuses(15, 15, 15, false);
   refuses(21, 21, 21, false);  // global tables on either layout
+  // thin and small grids, rows of cells and node runs
+  auto path = [&](uint32_t nx, uint32_t ny, uint32_t nz, bool nm, RmtPath want) {
+    const dev::GridShape g{nx, ny, nz, nx * ny * nz, 9.0};
+    if (dev::rmt_path(true, 4, g, kLds, nm) != want) {
+      std::printf("FAIL path of %u x %u x %u, nm %d\n", nx, ny, nz, nm);
+      ++failures;
+    }
+  };
+  path(12, 12, 3, true, RmtPath::kLds);
+  path(12, 12, 3, false, RmtPath::kMfma);
+  path(3, 12, 12, true, RmtPath::kLds);
+  path(12, 12, 6, true, RmtPath::kLds);
+  path(16, 16, 8, true, RmtPath::kMfma);
+  path(15, 15, 15, true, RmtPath::kMfma);
+  path(9, 9, 9, true, RmtPath::kLds);
+  path(6, 6, 6, true, RmtPath::kWave);
+  path(16, 16, 24, true, RmtPath::kLds);
+  path(16, 16, 24, false, RmtPath::kMfma);
   // dilute systems keep the direct sums: (charges, cells, nodes, mixed, taken)
   auto worth = [&](uint32_t n, uint32_t ncell, uint32_t K, bool mixed,
                    bool want) {
