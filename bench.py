@@ -538,7 +538,9 @@ def main():
     # expansion: harm_lr, harm_radial and harm_eval; avg_ms is their sum in one
     # step, HIP events on the handle's stream around them, from the steps run
     # one stage after another).  The bytes it cannot do without: the remote
-    # sums of every (cell, node) once, 8 B (16 B in FP64) each.
+    # sums of every (cell, node) once, 8 B (16 B in FP64) each; `frac` is
+    # against the time these take.  What bounds it is the issue of vector
+    # instructions (harm_eval) and the phases between barriers (harm_lr).
     K = info.num_nodes
     ncell = int(np.prod(info.ncell))
 
@@ -548,7 +550,7 @@ def main():
         return {
             "kernel": "harm_lr, harm_radial and harm_eval (calc_lr_ef through "
                       "the harmonic expansion)",
-            "bound": "hbm",
+            "bound": "issue",
             "achieved": gbs,
             "peak": PEAK_HBM_GBS,
             "unit": "GB/s",

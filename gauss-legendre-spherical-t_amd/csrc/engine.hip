@@ -450,8 +450,7 @@ struct glst_engine {
 
   void sum_rmt_sf() {
     if (!has_lr || Kp == 0) return;
-    if (!sf_done)
-      throw StateError("sum_rmt_sf called before calc_sf");
+    if (!sf_done) throw StateError("sum_rmt_sf called before calc_sf");
     Scope sc(timer, "rmt", stream);
     const bool nm = expanded();
     const double4 *kn = nm ? harm.k64 : k64.as<double4>();
@@ -488,8 +487,7 @@ struct glst_engine {
 
   void calc_lr_ef() {
     if (!has_lr || Kp == 0 || natom == 0) return;
-    if (!rmt_done)
-      throw StateError("calc_lr_ef called before sum_rmt_sf");
+    if (!rmt_done) throw StateError("calc_lr_ef called before sum_rmt_sf");
     lr_partials();
     reduce(false);
   }
@@ -1208,8 +1206,7 @@ glst_status_t glst_get_sf(glst_handle_t h, double *re, double *im) {
   NEED_HANDLE(h);
   return guarded(h, [&] {
     if (!h->has_lr || h->K == 0) return;
-    if (!h->sf_done)
-      throw StateError("glst_get_sf: no structure factors");
+    if (!h->sf_done) throw StateError("glst_get_sf: no structure factors");
     const size_t n = static_cast<size_t>(h->grid.ncell) * h->K;
     std::vector<double> r(n), i(n);
     h->field_to_host(h->S, h->mixed(), 2, true, r.data(), i.data());
@@ -1253,8 +1250,7 @@ glst_status_t glst_get_rmt(glst_handle_t h, double *re, double *im) {
   NEED_HANDLE(h);
   return guarded(h, [&] {
     if (!h->has_lr || h->K == 0) return;
-    if (!h->rmt_done)
-      throw StateError("glst_get_rmt: no remote sums");
+    if (!h->rmt_done) throw StateError("glst_get_rmt: no remote sums");
     const size_t n = static_cast<size_t>(h->grid.ncell) * h->K;
     std::vector<double> r(n), i(n);
     h->field_to_host(h->R, h->mixed(), 2, false, r.data(), i.data());
