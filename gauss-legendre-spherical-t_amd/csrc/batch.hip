@@ -292,10 +292,11 @@ BatchLayout pack_batch(int ct,
     d.ag0 = static_cast<uint32_t>(B.nag);
     d.agtile = 0;
     // expanded far field: the rule of a handle (harm_worth), and no small part
-    // of the batch, whose launches per stage already fill the device (512
-    // mixed systems of 100 to 10,000 waters: 94.2 ms with all that a handle
-    // would expand, 86.4 with those of 8e8 pairs, 92.4 with none; 64 such
-    // systems 13.5, 13.4 and 16.1 ms; 16 systems 2.9, 4.2 and 4.7 ms)
+    // of the batch, whose launches per stage already fill the device.  When
+    // the rule was set (times of the same build): 512 mixed systems of 100 to
+    // 10,000 waters 94.2 ms with all that a handle would expand, 86.4 with
+    // those of 8e8 pairs, 92.4 with none; 64 such systems 13.5, 13.4 and 16.1
+    // ms; 16 systems 2.9, 4.2 and 4.7 ms
     HarmSystem hs{};
     hs.sys = s;
     if (cheb && lr && !cs[s]->direct &&

@@ -128,13 +128,13 @@ struct Plan {
 };
 
 // Systems with an expanded far field (harmonic.hpp) run their passes on this
-// many streams, each with work fields for the largest of its systems (so that a
-// batch needs no more than its systems do alone, one slot each: the sum by
-// which a server admits them): a pass of one
-// system is too short to fill the device.  The rule of a single handle decides
-// which (the launches per stage keep the others): 64 mixed systems of 100 to
-// 10,000 waters take 14.6 ms, 16.0 with direct sums for all; 12 FP64 systems
-// of 100 to 4,000 waters 3.9 against 4.5 ms.
+// many streams, each with work fields for the largest of its systems (so that
+// a batch needs no more than its systems do alone, one slot each: the sum by
+// which a server admits them): a pass of one system is too short to fill the
+// device.  The rule of a single handle decides which, and kHarmShare (the
+// launches per stage keep the others): 64 mixed systems of 100 to 10,000
+// waters take 12.1 ms, 16.2 with direct sums for all; 12 FP64 systems of 100
+// to 4,000 waters 3.9 against 4.5 ms.
 constexpr uint32_t kHarmSlots = 4;
 struct HarmSystem {
   uint32_t sys, slot;

@@ -177,11 +177,14 @@ glst_status_t glst_get_rmt(glst_handle_t h, double *re, double *im);
 
 /* The far field (either CT) runs through an expansion of each cell in
  * spherical harmonics on systems of at least 2e8 (CT = float) or 3e8
- * (CT = double) (atom, node) pairs with the product rule, where the kernels
- * hold its degrees (phases to about 20 and 28 radians) and "sf_cheb" and
- * "lr_atom_groups" are 1 and "rmt_shape" is not 2; otherwise through direct
- * sums over atoms and nodes.  The two agree to the rounding of CT.  With it,
- * "lr_blocks" and "pipeline" have no effect.
+ * (CT = double) (atom, node) pairs and, by the mean, 22 or 24 atoms per cell
+ * (on grids of up to 512 cells any number, or 17) with the product rule, where
+ * the kernels hold its degrees (phases to about 20 and 28 radians), the device
+ * has room for its work fields, it needs no global-memory shell-sum tables
+ * that the direct sums would not, and "sf_cheb" and "lr_atom_groups" are 1 and
+ * "rmt_shape" is not 2; otherwise through direct sums over atoms and nodes.
+ * The two agree to the rounding of CT.  With it, "lr_blocks" and "pipeline"
+ * have no effect, and "rmt_shape" 3 needs z within 16 cells too.
  *
  * Tuning options of a handle:
  *   "overlap_near" (default 1): calc_ener_force runs the near field on a
@@ -195,7 +198,8 @@ glst_status_t glst_get_rmt(glst_handle_t h, double *re, double *im);
  *   CT = float on grids at most 16 cells wide in x and y, separable window
  *   sums on the matrix cores (FP32 direct sums; elsewhere as 0) (3); 3
  *   where nx * ny >= 128 (a z slice fills at least half of the matrix
- *   cores' 16 x 16 tile), else 5 where it applies, else 0 (4); for
+ *   cores' 16 x 16 tile; with the expansion nz * ny >= 128 too), else 5 where
+ *   it applies, else 0 (4); for
  *   CT = float on grids at most 8 cells a side, FP32 window sums along
  *   lines held in registers, one wave per four nodes (elsewhere as 0) (5).
  *   Shapes 0-2 agree to FP64 rounding, shapes 3 and 5 with them to FP32
