@@ -222,3 +222,38 @@ def test_atoms_outside_their_ball(cuda, ct, bar, tol, crowd):
         assert rel_err(far[:3], far0[:3]) < bar
         assert rel_err(far[3:], far0[3:]) < bar
     f.close()
+
+
+@pytest.mark.parametrize("ct", ["double", "float"])
+def test_captured_expanded_steps_replay(cuda, ct):
+    """A handle and a batch (two expanded systems on their own streams beside a
+    small one) captured: every replay gives the eager step's bits, with eager
+    work of the same handle type in between."""
+    import torch
+    import glst_amd as g
+    boxes = [(53.0, 49.0, 62.0), (46.2, 46.2, 46.2), (31.0, 40.0, 36.0)]
+    tol = 2e-5
+    sets = [lattice(b, 2.4, 30 + i) for i, b in enumerate(boxes)]
+    f, d = handle(g, torch, sets[0], boxes[0], tol, ct=ct)
+    assert expands(f, d)
+    eager = step(f, d)
+    e, _ = handle(g, torch, sets[0], boxes[0], tol, ct=ct, graph=1)
+    for _ in range(3):
+        assert same(step(e, d), eager)
+        assert same(step(f, d), eager)
+    e.close()
+    f.close()
+    n = [h[0].size for h in sets]
+    packed = [torch.as_tensor(np.concatenate([h[k] for h in sets]),
+                              dtype=torch.float64, device="cuda")
+              for k in range(4)]
+    out = {}
+    batches = {v: g.GLSTBatch(n, boxes, 9.0, tol, ct=ct) for v in (0, 1)}
+    batches[1].set_option("graph", 1)
+    for _ in range(3):
+        for v, b in batches.items():
+            got = step(b, packed)
+            assert same(got, out.setdefault(v, got))
+    assert same(out[0], out[1])
+    for b in batches.values():
+        b.close()
